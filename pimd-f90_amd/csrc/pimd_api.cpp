@@ -64,6 +64,7 @@ struct pimd_ctx {
   Group self;
   int natoms = 0;
   std::vector<double> kvec, Ak, p4vAk;
+  size_t dcoef_n = 0;            // column weights of the dense dipole matrix
   double polfac[4] = {0, 0, 0, 0};
   double ttm[TTM_NPARAM] = {};  // model parameters (vdW, polarisabilities, Thole, DMS)
   std::vector<int> hkl;
@@ -411,7 +412,18 @@ struct HostTables {
   std::vector<double4> kv;
   std::vector<int4> kh, cols, segs;
   std::vector<int> colk, segk;
+  std::vector<int4> dcol;  // dense dipole matrix: kz-columns by (kx, ky)
+  std::vector<int> dkx;    // first column of each kx plane
+  std::vector<double> dcoef;
 };
+
+// The most site pairs (beads x sites^2) for which the dense dipole matrix is
+// taken by launches.  Its cost grows with the pairs (forming it, then 72 bytes
+// of matrix per pair and iteration), the passes' mostly with the launches.
+// Force call, passes against matrix: TTM3-F 128 x 32 (524k pairs) 789 / 566 us,
+// 512 x 4 (1049k) 682 / 641, 256 x 16 (1049k) 816 / 733, 256 x 32 (2097k)
+// 975 / 1058; TTM2.1-F 128 x 8 (1180k) 835 / 688, 128 x 32 (4719k) 1132 / 1924.
+constexpr long DENSE_MAX_PAIRS = 1200000;
 
 // The k-vector tables, kz-columns and segments and the default launch shapes
 // of a set-up system (no device work).
@@ -438,6 +450,25 @@ void plan_system(pimd_ctx *x, HostTables &t) {
       colk.push_back((int)k);
     }
   }
+  // the same columns in (kx, ky) order for the dense dipole matrix, each with
+  // the summed weights of its +kz and -kz members, padded to fours
+  t.dcol.clear();
+  t.dkx.assign((size_t)c.hmax + 2, 0);
+  t.dcoef.clear();
+  for (size_t i = 0; i < cols.size(); ++i) {
+    const int4 cl = cols[i];
+    const int lm = cl.z + cl.w - 1, cnt = (lm + 4) / 4 * 4;
+    t.dcol.push_back(make_int4(cl.x, cl.y, cnt, (int)t.dcoef.size()));
+    for (int l = 0; l < cnt; ++l) {
+      double e = 0.0;
+      for (int o = 0; o < cl.w; ++o)
+        if (std::abs(cl.z + o) == l) e += x->p4vAk[(size_t)colk[i] + o];
+      t.dcoef.push_back(e);
+    }
+    t.dkx[(size_t)cl.x + 1] = (int)t.dcol.size();
+  }
+  x->dcoef_n = t.dcoef.size();
+  for (int h = 1; h <= c.hmax + 1; ++h) t.dkx[h] = std::max(t.dkx[h], t.dkx[h - 1]);
   // longest columns first: lanes and column groups that run together get
   // similar trip counts
   {
@@ -523,6 +554,19 @@ void plan_system(pimd_ctx *x, HostTables &t) {
   // factors kept (0.312 -> 0.282 ms per step)
   const int dflt_dd = pow2_clamp((c.mixed && !c.dd_cache ? 524288 : 262144) / std::max(mb, 1L), 16,
                                  c.model == 2 ? (c.dd_cache ? 16 : 32) : 64);
+  // Small systems solve for the induced dipoles with a dense matrix (the same
+  // iterates): up to 64 dipole sites one block per bead (the matrix fits its
+  // registers: 32 H2O x 32 beads, Rc 4.9 A, 1065 -> 491 us per force call),
+  // beyond by launches up to DENSE_MAX_PAIRS.
+  // PIMD_SOR_DENSE: 0 never, 1 by size, 2 wherever the tables allow.
+  {
+    const int mode = env_int("PIMD_SOR_DENSE", 1, 0, 2);
+    const long M = (long)c.nd * c.N;
+    const bool can = (c.model == PIMD_TTM21F || c.model == PIMD_TTM3F) && c.lmax <= 15 && M <= 1024;
+    c.dense = !can || mode == 0 ? 0 : M <= 64 ? 1
+              : mode == 2 || c.P * M * M <= DENSE_MAX_PAIRS ? 2 : 0;
+    if (c.dense) c.dd_cache = 0;
+  }
   // structure-factor site chunks: about 8 per bead from 4096 molecule-beads
   // on (with two lane sets per block; 512 H2O x 32 beads: 1.66 -> 1.61 ms per
   // mixed force call, TTM2.1-F 128 x 32: 1.75 -> 1.66 ms FP64), the staged
@@ -587,7 +631,7 @@ void layout_system(pimd_ctx *x, Arena &a, bool full) {
   a.take(&d.dip, P * N * nd * 3);
   a.take(&d.dip_prev, P * N * nd * 3);
   a.take(&d.Efd, P * N * nd * 3);
-  a.take(&d.diff2, P * N * nd);
+  a.take(&d.diff2, P * N * nd * (c.dense == 2 ? 2 : 1));
   a.take(&d.tally, P * N * T_COUNT);
   a.take(&d.hist, P * 4 * N * nd * 3);
   a.take(&d.nbr, P * N * (size_t)c.nbr_cap);
@@ -602,6 +646,12 @@ void layout_system(pimd_ctx *x, Arena &a, bool full) {
     const size_t n = dd_cache_elems(c);
     a.take(&d.ddts, c.mixed ? (n + 1) / 2 : n);
     d.ddtsf = (decltype(d.ddtsf))d.ddts;
+  }
+  if (c.dense) {
+    a.take(&d.dmat, dense_elems(c));
+    a.take(&d.dcol, c.ncol);
+    a.take(&d.dkx, (size_t)c.hmax + 2);
+    a.take(&d.dcoef, x->dcoef_n);
   }
   a.take(&d.Sq, P * nk * 2);
   a.take(&d.Sm, P * nk * 2);
@@ -671,6 +721,11 @@ int upload_system(pimd_ctx *x, const HostTables &t, hipStream_t s) {
   HIPCHK(hipMemcpyAsync(d.colk, t.colk.data(), sizeof(int) * t.colk.size(), hipMemcpyHostToDevice, s));
   HIPCHK(hipMemcpyAsync(d.segs, t.segs.data(), sizeof(int4) * t.segs.size(), hipMemcpyHostToDevice, s));
   HIPCHK(hipMemcpyAsync(d.segk, t.segk.data(), sizeof(int) * t.segk.size(), hipMemcpyHostToDevice, s));
+  if (c.dense) {
+    HIPCHK(hipMemcpyAsync(d.dcol, t.dcol.data(), sizeof(int4) * t.dcol.size(), hipMemcpyHostToDevice, s));
+    HIPCHK(hipMemcpyAsync(d.dkx, t.dkx.data(), sizeof(int) * t.dkx.size(), hipMemcpyHostToDevice, s));
+    HIPCHK(hipMemcpyAsync(d.dcoef, t.dcoef.data(), sizeof(double) * t.dcoef.size(), hipMemcpyHostToDevice, s));
+  }
   d.clk = d.clk_own;
   HIPCHK(hipMemsetAsync(d.clk_own, 0, 2 * sizeof(int), s));
   HIPCHK(hipMemsetAsync(d.flags, 0, sizeof(int), s));
@@ -728,10 +783,14 @@ void timed(pimd_ctx *px, const char *name, F &&f) {
 int run_forces(const Group &g, hipStream_t s, pimd_ctx *px) {
   const int n = g.n();
   bool any_ttm = false, all_fold = true, any_mixed = false;
-  int maxiter = 0;
+  int maxiter = 0, dense_iter = 0;  // of the pass-by-pass and of the dense solves
   for (const SysConst &c : g.hc) {
     if (c.model > 3) continue;
     any_ttm = true;
+    if (c.dense) {
+      dense_iter = std::max(dense_iter, c.maxiter);
+      continue;
+    }
     maxiter = std::max(maxiter, c.maxiter);
     all_fold = all_fold && pair_dd_tests(c);
     any_mixed = any_mixed || c.mixed;
@@ -749,8 +808,8 @@ int run_forces(const Group &g, hipStream_t s, pimd_ctx *px) {
   });
   // the reciprocal-space charge pass (it writes kE / kphi, added by their consumers)
   timed(px, "ewald_tables", [&] { launch_tables(g, s); });
-  timed(px, "sfac_q", [&] { launch_sfac(g, SF_Q, s, false, 1); });
-  timed(px, "sfac_q_reduce", [&] { launch_sfac(g, SF_Q, s, false, 2); });
+  timed(px, "sfac_q", [&] { launch_sfac(g, SF_Q, s, SFAC_ITER, 1); });
+  timed(px, "sfac_q_reduce", [&] { launch_sfac(g, SF_Q, s, SFAC_ITER, 2); });
   timed(px, "field_q", [&] { launch_field(g, FD_Q, 0, s); });
   if (any_ttm) {
     timed(px, "post_qq", [&] { launch_post_qq(g, s); });
@@ -758,12 +817,16 @@ int run_forces(const Group &g, hipStream_t s, pimd_ctx *px) {
     // dipole pair kernel of iteration it, where every replica's dipole
     // kernel can hold it; the last iteration's test stays a launch
     const bool fold = all_fold && !poll;
+    if (dense_iter > 0) {
+      timed(px, "dense_sor", [&] { launch_dense_sor(g, dense_iter, s); });
+      timed(px, "sfac_d", [&] { launch_sfac(g, SF_D, s, SFAC_STALE); });
+    }
     for (int it = 1; it <= maxiter; ++it) {
       // with timing on: the beads this iteration works on, for per-launch work counts
       if (poll && prof) px->count("sor_bead_iterations", it == 1 ? px->c.P : px->h_nactive[it - 1]);
       timed(px, "pair_dd", [&] { launch_pair_dd(g, false, s, fold && it > 1 ? it - 1 : 0, false, it); });
-      timed(px, "sfac_d", [&] { launch_sfac(g, SF_D, s, false, 1); });
-      timed(px, "sfac_d_reduce", [&] { launch_sfac(g, SF_D, s, false, 2); });
+      timed(px, "sfac_d", [&] { launch_sfac(g, SF_D, s, SFAC_ITER, 1); });
+      timed(px, "sfac_d_reduce", [&] { launch_sfac(g, SF_D, s, SFAC_ITER, 2); });
       timed(px, "field_d_sor", [&] { launch_field(g, FD_D, it, s); });
       if (!fold || it == maxiter) timed(px, "converge", [&] { launch_converge(g, it, s); });
       // No host round trip: converged beads are switched off on the device
@@ -784,13 +847,13 @@ int run_forces(const Group &g, hipStream_t s, pimd_ctx *px) {
       timed(px, "refine_dd", [&] {
         launch_refine_prep(g, s);
         launch_pair_dd(g, true, s, 0, true);
-        launch_sfac(g, SF_D, s, true);
+        launch_sfac(g, SF_D, s, SFAC_REFINE);
         launch_field(g, FD_D, -1, s, true);
       });
     }
     timed(px, "pair_final", [&] { launch_pair_final(g, s); });
-    timed(px, "sfac_v", [&] { launch_sfac(g, SF_V, s, false, 1); });
-    timed(px, "sfac_v_reduce", [&] { launch_sfac(g, SF_V, s, false, 2); });
+    timed(px, "sfac_v", [&] { launch_sfac(g, SF_V, s, SFAC_ITER, 1); });
+    timed(px, "sfac_v_reduce", [&] { launch_sfac(g, SF_V, s, SFAC_ITER, 2); });
     timed(px, "field_qd", [&] { launch_field(g, FD_QD, 0, s); });
   }
   timed(px, "virial_k", [&] { launch_virk(g, s); });
@@ -2544,6 +2607,12 @@ extern "C" int pimd_forces_all_beads_noalloc(const pimd_params *params, const do
   x.c.sf_chunks_max = sfac_chunks_used(x.c);
   Arena a;
   layout_system(&x, a, false);
+  if (x.c.dense && a.off > sizeof(scratch)) {
+    // no room for the dense dipole matrix: the pass-by-pass solve
+    x.c.dense = 0;
+    a.off = 0;
+    layout_system(&x, a, false);
+  }
   if (a.off > sizeof(scratch))
     return fail(PIMD_EINVAL, "%d waters x %d beads need %zu bytes of device workspace, more than "
                 "the %zu bytes of pimd_forces_all_beads_noalloc", p.nwaters, p.nbeads, a.off,

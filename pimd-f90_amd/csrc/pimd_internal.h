@@ -72,6 +72,7 @@ struct SysConst {
   int poll;                // 1: read the active-bead count back after every SOR iteration
   int overlap;             // 1: real-space dipole field beside the structure factor (2 streams)
   int dd_cache;            // 1: the SOR dipole pass keeps each pair's screening factors
+  int dense;               // SOR by a dense dipole matrix: 0 no, 1 one block per bead, 2 by launches
   int qq_half;             // once-per-pair charge pass: 0 off, 1 where it fills the device, 2 always
   int fin_half;            // the same for the final dipole pass (with qq_half): 0 off, 1 on
   double box[3], boxi[3], vol;
@@ -139,6 +140,11 @@ struct DevBufs {
   // the others: FP64 (ddts) or, in the mixed form, FP32 (ddtsf, same memory)
   dptr<double2> ddts = nullptr;
   dptr<float2> ddtsf = nullptr;
+  // dense dipole matrix [P][3M][dense_stride] (M dipole sites), its kz-column
+  // weights: kx, ky, count, first weight per column; columns of each kx plane
+  dptr<double> dmat = nullptr, dcoef = nullptr;
+  dptr<int4> dcol = nullptr;
+  dptr<int> dkx = nullptr;
   dptr<double> Sq = nullptr, Sm = nullptr;  // [P][nk][2]
   dptr<double> Sv = nullptr;  // [P][nk][6]
   dptr<double> virk = nullptr;  // [P][nkb][9]
@@ -322,9 +328,19 @@ void launch_monomer(const Group &g, hipStream_t s);
 void launch_neighbors(const Group &g, hipStream_t s);
 void launch_pair_qq(const Group &g, hipStream_t s);
 void launch_tables(const Group &g, hipStream_t s);
-// refine: SF_D in FP64 for the mixed replicas' refinement step.  part: 1 the
-// per-chunk partial sums, 2 their reduction into the structure factor, 3 both.
-void launch_sfac(const Group &g, int mode, hipStream_t s, bool refine = false, int part = 3);
+// sel (SF_D): the SOR iterations, FP64 for the mixed replicas' refinement
+// step, or the last SOR input of the dense systems.  part: 1 the per-chunk
+// partial sums, 2 their reduction into the structure factor, 3 both.
+enum SfacSel { SFAC_ITER = 0, SFAC_REFINE = 1, SFAC_STALE = 2 };
+void launch_sfac(const Group &g, int mode, hipStream_t s, int sel = SFAC_ITER, int part = 3);
+// The whole SOR solve of the systems with a dense dipole matrix.
+void launch_dense_sor(const Group &g, int maxiter, hipStream_t s);
+__host__ __device__ inline size_t dense_stride(const SysConst &c) {
+  return ((size_t)3 * c.nd * c.N + 1) & ~(size_t)1;
+}
+inline size_t dense_elems(const SysConst &c) {
+  return (size_t)c.P * 3 * c.nd * c.N * dense_stride(c);
+}
 int sfac_chunks_used(const SysConst &c);
 void launch_converge(const Group &g, int iter, hipStream_t s);
 // iter: the SOR iteration of FD_D, -1 for the FP64 refinement (maxiter + 1);

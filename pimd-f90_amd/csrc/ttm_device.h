@@ -156,6 +156,46 @@ __device__ __forceinline__ void vadd9(double *t, const double *v) {
   for (int i = 0; i < 9; ++i) t[i] += v[i];
 }
 
+// The SOR convergence test of iteration `iter` for bead b (pot_ttm.f90:306,
+// 380-386), as k_converge forms it: the first 256 threads of the block add
+// the bead's squared dipole changes in the same order.  All blocks of the
+// bead reach the same outcome; block `writer` records it.  Returns whether
+// the bead is still active; every thread of the block must call it.
+__device__ inline bool sor_test(const SysConst &c, const double *__restrict__ diff2, int *active,
+                         int *iters, int *nactive, int b, int iter, bool writer, double *red,
+                         int &act) {
+  const int tid = threadIdx.x;
+  if (tid == 0) act = active[b];  // one read per block: the writer block may change it
+  __syncthreads();
+  if (!act) return false;
+  const int M = c.N * c.nd;
+  if (tid < 256) {
+    double s = 0.0;
+    for (int m = tid; m < M; m += 256) s += diff2[(size_t)b * M + m];
+    red[tid] = s;
+  }
+  __syncthreads();
+  for (int off = 128; off > 0; off >>= 1) {
+    if (tid < off) red[tid] += red[tid + off];
+    __syncthreads();
+  }
+  const double delta = c.stath * sqrt(red[0]);
+  const bool conv = delta < c.peps, last = iter >= c.maxiter;
+  if (writer && tid == 0) {
+    if (conv) {
+      active[b] = 0;
+      iters[b] = iter;
+    } else if (last) {
+      active[b] = 0;
+      iters[b] = -iter;
+    } else {
+      iters[b] = iter;
+      atomicAdd(&nactive[iter], 1);
+    }
+  }
+  return !(conv || last);
+}
+
 // x*x + y*y + z*z rounded exactly as the reference (no fused multiply-add), so
 // cut-off tests (r^2 < Rc^2, r^2 < 25) decide identically.
 __device__ __forceinline__ double norm2_exact(double x, double y, double z) {

@@ -1152,7 +1152,8 @@ __host__ __device__ inline int sfac_sites(const SysConst &c, int mode) {
 // Structure factors with one kz-segment (fixed kx, ky, up to KZ consecutive kz)
 // per lane: the phase of each site is formed once per segment and advanced
 // along kz by e^{i 2 pi z/L}, accumulating every kz of the segment in
-// registers.  A block takes a chunk of
+// registers.  stale (SF_D): of every bead's dip_prev, the input of its last
+// SOR step, in place of its current dipoles (dense systems).  A block takes a chunk of
 // sites of one bead; their phase tables and weights are staged in LDS (rows
 // padded so that lanes reading different rows of one site hit different
 // banks).  Per-chunk partial sums are combined in a fixed order by
@@ -1161,7 +1162,8 @@ __host__ __device__ inline int sfac_sites(const SysConst &c, int mode) {
 // half of the chunk's sites; the second hands its sums to the first through
 // LDS, which adds them and writes (twice the waves for the same partials).
 template <int MODE, int KZ, int SPLIT = 1, class R = double>
-__global__ __launch_bounds__(512) void k_sfac_col(const Rep *__restrict__ reps, BlockMap bm) {
+__global__ __launch_bounds__(512) void k_sfac_col(const Rep *__restrict__ reps, BlockMap bm,
+                                                  int stale) {
   using R2 = typename Vec<R>::v2;
   constexpr int SET = MODE == SF_Q ? SET_CHG : SET_DIP;
   constexpr int NW = MODE == SF_Q ? 1 : 3;
@@ -1175,7 +1177,7 @@ __global__ __launch_bounds__(512) void k_sfac_col(const Rep *__restrict__ reps, 
   const Rep &Rp = reps[bk.r];
   const SysConst &c = Rp.c;
   const Site *__restrict__ site = Rp.b.site;
-  const double *__restrict__ dip = Rp.b.dip;
+  const double *__restrict__ dip = stale ? Rp.b.dip_prev : Rp.b.dip;
   const int4 *__restrict__ cols = Rp.b.segs;
   const int *__restrict__ colk = Rp.b.segk;
   const int *__restrict__ active = Rp.b.active;
@@ -1184,7 +1186,7 @@ __global__ __launch_bounds__(512) void k_sfac_col(const Rep *__restrict__ reps, 
   sfac_chunking(c, MODE, sfac_sites(c, MODE), nch, sc, scp);
   R *lw = reinterpret_cast<R *>(lds_sf + (size_t)c.T * scp);
   const int b = bk.z;
-  if (MODE == SF_D && !active[b]) return;
+  if (MODE == SF_D && !stale && !active[b]) return;
   const int S = 4 * c.N, M = set_size(c, SET);
   const int chunk = bk.y;
   const int m0 = chunk * sc, nt = min(sc, M - m0);
@@ -1307,7 +1309,8 @@ __global__ __launch_bounds__(512) void k_sfac_col(const Rep *__restrict__ reps, 
 //   SF_D: (-sum (k.mu) sin, sum (k.mu) cos)           (ewald.f90:99-110)
 //   SF_V: (sum mu cos, sum mu sin) per component      (ewald.f90:208-213)
 template <int MODE>
-__global__ __launch_bounds__(256) void k_sfac_k(const Rep *__restrict__ reps, BlockMap bm) {
+__global__ __launch_bounds__(256) void k_sfac_k(const Rep *__restrict__ reps, BlockMap bm,
+                                                int stale) {
   constexpr int SET = MODE == SF_Q ? SET_CHG : SET_DIP;
   constexpr int NW = MODE == SF_Q ? 1 : 3;
   constexpr int NV = MODE == SF_V ? 6 : 2;
@@ -1316,7 +1319,7 @@ __global__ __launch_bounds__(256) void k_sfac_k(const Rep *__restrict__ reps, Bl
   const Rep &Rp = reps[bk.r];
   const SysConst &c = Rp.c;
   const Site *__restrict__ site = Rp.b.site;
-  const double *__restrict__ dip = Rp.b.dip;
+  const double *__restrict__ dip = stale ? Rp.b.dip_prev : Rp.b.dip;
   const double4 *__restrict__ kv = Rp.b.kv;
   const int4 *__restrict__ khkl = Rp.b.khkl;
   const int *__restrict__ active = Rp.b.active;
@@ -1325,7 +1328,7 @@ __global__ __launch_bounds__(256) void k_sfac_k(const Rep *__restrict__ reps, Bl
   sfac_chunking(c, MODE, sfac_sites(c, MODE), nch, sc, scp);
   double *lw = reinterpret_cast<double *>(lds_sf + (size_t)c.T * scp);
   const int b = bk.z;
-  if (MODE == SF_D && !active[b]) return;
+  if (MODE == SF_D && !stale && !active[b]) return;
   const int S = 4 * c.N, M = set_size(c, SET);
   const int chunk = bk.y;
   const int m0 = chunk * sc, nt = min(sc, M - m0);
@@ -1388,7 +1391,7 @@ __global__ __launch_bounds__(256) void k_sfac_k(const Rep *__restrict__ reps, Bl
 
 // The per-chunk partial sums of structure factor `mode` added in chunk order.
 __global__ __launch_bounds__(256) void k_sfac_reduce(const Rep *__restrict__ reps, BlockMap bm,
-                                                    int mode) {
+                                                    int mode, int stale) {
   const Blk bk = block_of(bm);
   const Rep &Rp = reps[bk.r];
   const SysConst &c = Rp.c;
@@ -1398,7 +1401,7 @@ __global__ __launch_bounds__(256) void k_sfac_reduce(const Rep *__restrict__ rep
   int nch, sc, scp;
   sfac_chunking(c, mode, sfac_sites(c, mode), nch, sc, scp);
   const int b = bk.y;
-  if (mode == SF_D && !Rp.b.active[b]) return;
+  if (mode == SF_D && !stale && !Rp.b.active[b]) return;
   const int e = bk.x * blockDim.x + threadIdx.x;  // (k, component)
   if (e >= nv * c.nk) return;
   double v = 0.0;
@@ -1821,46 +1824,6 @@ constexpr int dd_block() {
 constexpr int DD_REC = 7;
 // neighbour indices requested ahead by the TTM3-F dipole pass
 constexpr int DD_AHEAD = 4;
-// The SOR convergence test of iteration `iter` for bead b (pot_ttm.f90:306,
-// 380-386), as k_converge forms it: the first 256 threads of the block add
-// the bead's squared dipole changes in the same order.  All blocks of the
-// bead reach the same outcome; block `writer` records it.  Returns whether
-// the bead is still active; every thread of the block must call it.
-__device__ bool sor_test(const SysConst &c, const double *__restrict__ diff2, int *active,
-                         int *iters, int *nactive, int b, int iter, bool writer, double *red,
-                         int &act) {
-  const int tid = threadIdx.x;
-  if (tid == 0) act = active[b];  // one read per block: the writer block may change it
-  __syncthreads();
-  if (!act) return false;
-  const int M = c.N * c.nd;
-  if (tid < 256) {
-    double s = 0.0;
-    for (int m = tid; m < M; m += 256) s += diff2[(size_t)b * M + m];
-    red[tid] = s;
-  }
-  __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if (tid < off) red[tid] += red[tid + off];
-    __syncthreads();
-  }
-  const double delta = c.stath * sqrt(red[0]);
-  const bool conv = delta < c.peps, last = iter >= c.maxiter;
-  if (writer && tid == 0) {
-    if (conv) {
-      active[b] = 0;
-      iters[b] = iter;
-    } else if (last) {
-      active[b] = 0;
-      iters[b] = -iter;
-    } else {
-      iters[b] = iter;
-      atomicAdd(&nactive[iter], 1);
-    }
-  }
-  return !(conv || last);
-}
-
 // (ts1, ts2) of one dipole-site pair in the SOR arithmetic type, and the
 // context's cache of them
 template <typename R>
@@ -2926,37 +2889,39 @@ static const int KZ_BUCKET[6] = {4, 8, 12, 16, 24, 32};
 
 template <int MODE, int KZ, class R>
 static void launch_sfac_col_v(bool split, int threads, dim3 grid, const BlockMap &m, size_t lds,
-                              const Group &g, hipStream_t s) {
-  if (split) hipLaunchKernelGGL((k_sfac_col<MODE, KZ, 2, R>), grid, dim3(2 * threads), lds, s, g.d, m);
-  else hipLaunchKernelGGL((k_sfac_col<MODE, KZ, 1, R>), grid, dim3(threads), lds, s, g.d, m);
+                              int stale, const Group &g, hipStream_t s) {
+  if (split) hipLaunchKernelGGL((k_sfac_col<MODE, KZ, 2, R>), grid, dim3(2 * threads), lds, s, g.d, m, stale);
+  else hipLaunchKernelGGL((k_sfac_col<MODE, KZ, 1, R>), grid, dim3(threads), lds, s, g.d, m, stale);
 }
 
 template <int MODE, class R>
-static void launch_sfac_kz(int v, dim3 grid, const BlockMap &m, size_t lds, const Group &g,
-                           hipStream_t s) {
+static void launch_sfac_kz(int v, dim3 grid, const BlockMap &m, size_t lds, int stale,
+                           const Group &g, hipStream_t s) {
   const bool split = (v & 16) != 0;
   const int threads = ((v >> 5) & 7) * 64;
   switch ((v >> 1) & 7) {
-    case 0: launch_sfac_col_v<MODE, 4, R>(split, threads, grid, m, lds, g, s); break;
-    case 1: launch_sfac_col_v<MODE, 8, R>(split, threads, grid, m, lds, g, s); break;
-    case 2: launch_sfac_col_v<MODE, 12, R>(split, threads, grid, m, lds, g, s); break;
-    case 3: launch_sfac_col_v<MODE, 16, R>(split, threads, grid, m, lds, g, s); break;
-    case 4: launch_sfac_col_v<MODE, 24, R>(split, threads, grid, m, lds, g, s); break;
-    default: launch_sfac_col_v<MODE, 32, R>(split, threads, grid, m, lds, g, s); break;
+    case 0: launch_sfac_col_v<MODE, 4, R>(split, threads, grid, m, lds, stale, g, s); break;
+    case 1: launch_sfac_col_v<MODE, 8, R>(split, threads, grid, m, lds, stale, g, s); break;
+    case 2: launch_sfac_col_v<MODE, 12, R>(split, threads, grid, m, lds, stale, g, s); break;
+    case 3: launch_sfac_col_v<MODE, 16, R>(split, threads, grid, m, lds, stale, g, s); break;
+    case 4: launch_sfac_col_v<MODE, 24, R>(split, threads, grid, m, lds, stale, g, s); break;
+    default: launch_sfac_col_v<MODE, 32, R>(split, threads, grid, m, lds, stale, g, s); break;
   }
 }
 
-// refine: the FP64 dipole structure factor of the mixed form's refinement
-// step (mixed replicas only); otherwise the mixed form's SOR iterations take
-// it in FP32 (variant bit 8).
+// sel (SF_D): SFAC_ITER, the SOR iterations (not the dense systems; the mixed
+// form's in FP32, variant bit 8), SFAC_REFINE the mixed form's FP64
+// refinement step, SFAC_STALE the dense systems' last input.
 // part: 1 the chunk partial sums, 2 their fixed-order reduction, 3 both.
 template <int MODE>
-static void launch_sfac_mode(const Group &g, bool refine, int part, hipStream_t s) {
+static void launch_sfac_mode(const Group &g, int sel, int part, hipStream_t s) {
   constexpr int NV = MODE == SF_V ? 6 : 2;
+  const int stale = MODE == SF_D && sel == SFAC_STALE ? 1 : 0;
   auto plan = [&](const SysConst &c) {
         if (MODE != SF_Q && !is_ttm(c)) return Plan{-1, 0, 0, 0, 0};
-        if (refine && !c.mixed) return Plan{-1, 0, 0, 0, 0};
-        const bool f32 = MODE == SF_D && c.mixed && !refine;
+        if (sel == SFAC_REFINE && !c.mixed) return Plan{-1, 0, 0, 0, 0};
+        if (MODE == SF_D && (c.dense != 0) != (sel == SFAC_STALE)) return Plan{-1, 0, 0, 0, 0};
+        const bool f32 = MODE == SF_D && c.mixed && sel == SFAC_ITER;
         int nch, sc, scp;
         sfac_chunking(c, MODE, sfac_sites(c, MODE), nch, sc, scp);
         const size_t lds = sfac_lds(c, MODE, sc, scp, f32);
@@ -2977,16 +2942,16 @@ static void launch_sfac_mode(const Group &g, bool refine, int part, hipStream_t 
       g, [&](const SysConst &c, const MDConst &) { return plan(c); },
       [&](int v, dim3 grid, const BlockMap &m, size_t lds) {
         if (!(v & 1)) {
-          hipLaunchKernelGGL((k_sfac_k<MODE>), grid, dim3(256), lds, s, g.d, m);
+          hipLaunchKernelGGL((k_sfac_k<MODE>), grid, dim3(256), lds, s, g.d, m, stale);
           return;
         }
         if constexpr (MODE == SF_D) {
           if (v & 256) {
-            launch_sfac_kz<MODE, float>(v, grid, m, lds, g, s);
+            launch_sfac_kz<MODE, float>(v, grid, m, lds, stale, g, s);
             return;
           }
         }
-        launch_sfac_kz<MODE, double>(v, grid, m, lds, g, s);
+        launch_sfac_kz<MODE, double>(v, grid, m, lds, stale, g, s);
       });
   if (part & 2) launch_over(
       g,
@@ -2995,14 +2960,14 @@ static void launch_sfac_mode(const Group &g, bool refine, int part, hipStream_t 
         return Plan{0, idiv((long)NV * c.nk, 256), c.P, 1, 0};
       },
       [&](int, dim3 grid, const BlockMap &m, size_t) {
-        hipLaunchKernelGGL(k_sfac_reduce, grid, dim3(256), 0, s, g.d, m, MODE);
+        hipLaunchKernelGGL(k_sfac_reduce, grid, dim3(256), 0, s, g.d, m, MODE, stale);
       });
 }
 
-void launch_sfac(const Group &g, int mode, hipStream_t s, bool refine, int part) {
-  if (mode == SF_Q) launch_sfac_mode<SF_Q>(g, false, part, s);
-  else if (mode == SF_D) launch_sfac_mode<SF_D>(g, refine, part, s);
-  else launch_sfac_mode<SF_V>(g, false, part, s);
+void launch_sfac(const Group &g, int mode, hipStream_t s, int sel, int part) {
+  if (mode == SF_Q) launch_sfac_mode<SF_Q>(g, SFAC_ITER, part, s);
+  else if (mode == SF_D) launch_sfac_mode<SF_D>(g, sel, part, s);
+  else launch_sfac_mode<SF_V>(g, SFAC_ITER, part, s);
 }
 
 // The FP32 dipole field of the mixed form's SOR iterations (variant bits as
@@ -3031,7 +2996,8 @@ static void launch_field_mode(const Group &g, int iter, bool sel_mixed, hipStrea
   launch_over(
       g,
       [&](const SysConst &c, const MDConst &) {
-        if ((MO != FD_Q && !is_ttm(c)) || (sel_mixed && !c.mixed)) return Plan{-1, 0, 0, 0, 0};
+        if ((MO != FD_Q && !is_ttm(c)) || (sel_mixed && !c.mixed) || (MO == FD_D && c.dense))
+          return Plan{-1, 0, 0, 0, 0};
         const int ML = c.model == 2 ? 2 : 3;
         const int M = MO == FD_D ? c.nd * c.N : (ML == 2 ? 4 * c.N : 3 * c.N);
         // as many column groups as the columns keep busy: more resident waves hide
@@ -3125,7 +3091,7 @@ void launch_pair_dd(const Group &g, bool fp64, hipStream_t s, int test_iter, boo
   launch_over(
       g,
       [&](const SysConst &c, const MDConst &) {
-        if (!is_ttm(c) || (sel_mixed && !c.mixed)) return Plan{-1, 0, 0, 0, 0};
+        if (!is_ttm(c) || (sel_mixed && !c.mixed) || c.dense) return Plan{-1, 0, 0, 0, 0};
         const int v0 = (c.model == 3 ? 1 : 0) | (c.mixed && !fp64 ? 2 : 0);
         if (pair_dd_tests(c)) {
           const int G = c.g_dd == 64 ? 64 : c.g_dd == 32 ? 32 : c.g_dd == 8 ? 8 : 16;
@@ -3157,7 +3123,7 @@ void launch_refine_prep(const Group &g, hipStream_t s) {
       g,
       [](const SysConst &c, const MDConst &) {
         const long n = std::max((long)c.P * c.N * c.nd * 3, (long)c.P);
-        return Plan{is_ttm(c) && c.mixed ? 0 : -1, idiv(n, 256), 1, 1, 0};
+        return Plan{is_ttm(c) && c.mixed && !c.dense ? 0 : -1, idiv(n, 256), 1, 1, 0};
       },
       [&](int, dim3 grid, const BlockMap &m, size_t) {
         hipLaunchKernelGGL(k_refine_prep, grid, dim3(256), 0, s, g.d, m);
@@ -3166,7 +3132,10 @@ void launch_refine_prep(const Group &g, hipStream_t s) {
 
 void launch_converge(const Group &g, int iter, hipStream_t s) {
   launch_over(
-      g, [](const SysConst &c, const MDConst &) { return Plan{is_ttm(c) ? 0 : -1, c.P, 1, 1, 0}; },
+      g,
+      [](const SysConst &c, const MDConst &) {
+        return Plan{is_ttm(c) && !c.dense ? 0 : -1, c.P, 1, 1, 0};
+      },
       [&](int, dim3 grid, const BlockMap &m, size_t) {
         hipLaunchKernelGGL(k_converge, grid, dim3(256), 0, s, g.d, m, iter);
       });
