@@ -20,6 +20,11 @@ namespace pimd {
 
 constexpr double KCAL = 0.00285914375100642899;  // cm-1 -> kcal/mol (nasa.f90:101)
 constexpr int ADJ_BLOCK = 64;
+// Blocks that share 64 molecules, each taking every ADJ_PARTS-th parameter: a
+// parameter is a chain of dual products and a wave reduction, and one wave per
+// 64 molecules leaves the device idle (64 clusters and 64 boxes of 32 H2O, 32
+// waves: 136 -> 28 us).
+constexpr int ADJ_PARTS = 8;
 
 // Exponent table of the PES basis (nasa_mod.f90 idx), this unit's own copy.
 __constant__ int c_idx_adj[PS_NTERM][3];
@@ -40,8 +45,8 @@ static bool set_adjoint_tables() {
   return ok;
 }
 
-// One thread per (bead, molecule); each block sums its molecules' terms for
-// every parameter (wave reduction, fixed order) into partial[block][250].
+// One thread per (bead, molecule); a block sums its molecules' terms of its
+// parameters (wave reduction, fixed order) into partial[block][250].
 __global__ __launch_bounds__(ADJ_BLOCK) void k_pes_adjoint(SysConst c, const double *__restrict__ RR,
                                                           const double *__restrict__ ew,
                                                           const double *__restrict__ gw,
@@ -92,22 +97,21 @@ __global__ __launch_bounds__(ADJ_BLOCK) void k_pes_adjoint(SysConst c, const dou
   const Dual e1 = dexp(-alphaoh * r1), e2 = dexp(-alphaoh * r2);
   const Dual ehh = dexp(-phh2 * dh);
 
-  __shared__ double acc[PES_NPARAM];
-  for (int j = threadIdx.x; j < PES_NPARAM; j += blockDim.x) acc[j] = 0.0;
-  __syncthreads();
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63, part = blockIdx.y;
+  double *out = partial + (size_t)blockIdx.x * PES_NPARAM;
   auto add = [&](int j, Dual g) {
     double v = valid ? KCAL * (ewb * g.v + g.d) : 0.0;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (lane == 0) acc[j] += v;  // one wave per block: a fixed order
+    if (lane == 0) out[j] = v;
   };
   // dEmon/dc5z(1) = 2 (nasa.f90:90); dEmon/dc5z(j) = efac * basis_j (nasa.f90:72-78)
-  add(0, dmk(2.0));
-  for (int j = 1; j < PES_NC; ++j) {
+  if (part == 0) add(0, dmk(2.0));
+  for (int j = 1 + part; j < PES_NC; j += ADJ_PARTS) {
     const int I = c_idx_adj[j][0], J = c_idx_adj[j][1], K = c_idx_adj[j][2];
     add(j, efac * ((f1[I] * f2[J] + f1[J] * f2[I]) * f3[K]));
   }
+  if (part != ADJ_PARTS - 1) return;
   // Va = deoh (e1 (e1 - 2) + e2 (e2 - 2)), e_i = exp(-alphaoh (d_i - roh))
   const Dual two = dmk(2.0);
   add(PES_DEOHA, PS_F5Z * (e1 * (e1 - two) + e2 * (e2 - two)));
@@ -118,9 +122,6 @@ __global__ __launch_bounds__(ADJ_BLOCK) void k_pes_adjoint(SysConst c, const dou
   // Vb = f5z phh1A exp(phh2) exp(-phh2 dHH)
   add(PES_PHH1A, (PS_F5Z * exp(phh2)) * ehh);
   add(PES_PHH2, phh1 * (ehh * (dmk(1.0) - dh)));
-  __syncthreads();
-  for (int j = threadIdx.x; j < PES_NPARAM; j += blockDim.x)
-    partial[(size_t)blockIdx.x * PES_NPARAM + j] = acc[j];
 }
 
 __global__ __launch_bounds__(256) void k_pes_adjoint_sum(const double *__restrict__ partial,
@@ -138,7 +139,7 @@ bool launch_pes_adjoint(const SysConst &c, DevBufs &b, const double *RR, const d
                         const double *gw, double *partial, int nblocks, double *grad,
                         hipStream_t s) {
   if (!set_adjoint_tables()) return false;
-  hipLaunchKernelGGL(k_pes_adjoint, dim3(nblocks), dim3(ADJ_BLOCK), 0, s, c, RR, ew, gw, b.pes,
+  hipLaunchKernelGGL(k_pes_adjoint, dim3(nblocks, ADJ_PARTS), dim3(ADJ_BLOCK), 0, s, c, RR, ew, gw, b.pes,
                      partial);
   hipLaunchKernelGGL(k_pes_adjoint_sum, dim3(1), dim3(256), 0, s, partial, nblocks, grad);
   return true;

@@ -2303,9 +2303,10 @@ static int tangent_start(pimd_ctx *x, const double *RRt, const double *ew, const
   const int nsweep = adj ? 1 : ndir;  // workgroups per configuration
   const size_t P = (size_t)c.P, n = P * x->natoms * 3, nout = P * nsweep * 4;
   const size_t nadj = adj ? P * TTM_ADJ_NPARAM * 2 : 0;
+  const size_t ext = adj ? (adjoint_extra_doubles(c) + 1) & ~(size_t)1 : 0;
   const size_t ws = tangent_ws_duals(c) * P * nsweep * 2, cfg = tangent_cfg_doubles(c) * P;
-  const size_t bytes = sizeof(double) * (ws + cfg + 2 * n + P + nout + nadj);
-  if (bytes > ((size_t)32 << 30))
+  const size_t bytes = sizeof(double) * (ext + ws + cfg + 2 * n + P + nout + nadj);
+  if (bytes - sizeof(double) * ext > ((size_t)32 << 30))
     return fail(PIMD_EINVAL, "parameter derivatives of %zu configurations need %.1f GB of workspace; "
                 "split them into smaller contexts", P, bytes / 1e9);
   if (bytes > d.tan_bytes) {
@@ -2319,8 +2320,11 @@ static int tangent_start(pimd_ctx *x, const double *RRt, const double *ew, const
     d.tan_bytes = bytes;
   }
   TanLaunch L;
-  L.ws = d.tan;  // dual workspace first: 16-byte aligned
-  L.cfg = d.tan + ws;
+  L.extra = d.tan;      // the dual workspaces first: 16-byte aligned
+  L.ws = d.tan + ext;
+  L.cfg = d.tan + ext + ws;
+  L.cols = d.cols;
+  L.colk = d.colk;
   double *dRR = L.cfg + cfg, *dgw = dRR + n, *dew = dgw + n;
   L.out = dew + P;
   L.RR = dRR;

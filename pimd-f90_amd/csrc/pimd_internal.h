@@ -438,8 +438,12 @@ struct TanLaunch {
   int gamma_m;   // 1: the one direction is the M-site fraction gammaM (moves the M sites)
   int adjoint;   // 1: the adjoint of all TTM_ADJ_NPARAM parameters (one sweep along gw)
   double *adj;   // adjoint output [P][TTM_ADJ_NPARAM][2]
+  double *extra; // adjoint: adjoint_extra_doubles(c)
+  const int4 *cols;
+  const int *colk;
   int ndir;
 };
+size_t adjoint_extra_doubles(const SysConst &c);
 size_t tangent_cfg_doubles(const SysConst &c);
 size_t tangent_ws_duals(const SysConst &c);
 void launch_ttm_tangent(const SysConst &c, const TanLaunch &L, hipStream_t s);

@@ -25,6 +25,8 @@
 // what it writes (every site-pair term is evaluated from both ends), so no
 // atomics.  Per configuration a preparatory kernel writes the sites and the
 // per-axis phase tables once for all directions.
+#include <algorithm>
+#include <cstdlib>
 #include <type_traits>
 
 #include "dual.h"
@@ -40,42 +42,6 @@ struct RM<Dual> {
   static __device__ __forceinline__ Dual exp_(Dual x) { return dexp(x); }
   static __device__ __forceinline__ Dual log_(Dual x) { return dlog(x); }
   static __device__ __forceinline__ Dual abs_(Dual x) { return dabs(x); }
-};
-
-// Dual numbers over duals: v is a value with its derivative along the
-// adjoint's position direction, a the derivative of v with respect to one
-// Thole factor, itself with its position derivative.  The adjoint runs the
-// smearing functions on them for d ts / d a along the direction.
-struct HD {
-  Dual v, a;
-  HD() = default;
-  __device__ constexpr HD(double x) : v(x), a(0.0) {}
-  __device__ constexpr HD(Dual x, Dual y) : v(x), a(y) {}
-};
-__device__ __forceinline__ HD operator+(HD x, HD y) { return HD(x.v + y.v, x.a + y.a); }
-__device__ __forceinline__ HD operator-(HD x, HD y) { return HD(x.v - y.v, x.a - y.a); }
-__device__ __forceinline__ HD operator-(HD x) { return HD(-x.v, -x.a); }
-__device__ __forceinline__ HD operator*(HD x, HD y) { return HD(x.v * y.v, x.a * y.v + x.v * y.a); }
-__device__ __forceinline__ HD operator/(HD x, HD y) {
-  const Dual q = x.v / y.v;
-  return HD(q, (x.a - q * y.a) / y.v);
-}
-__device__ __forceinline__ bool operator<(HD x, HD y) { return x.v.v < y.v.v; }
-__device__ __forceinline__ bool operator<=(HD x, HD y) { return x.v.v <= y.v.v; }
-template <>
-struct RM<HD> {
-  static __device__ __forceinline__ HD sqrt_(HD x) {
-    const Dual r = dsqrt(x.v);
-    return HD(r, 0.5 * x.a / r);
-  }
-  static __device__ __forceinline__ HD rcp(HD x) { return HD(1.0) / x; }
-  static __device__ __forceinline__ HD div(HD x, HD y) { return x / y; }
-  static __device__ __forceinline__ HD exp_(HD x) {
-    const Dual e = dexp(x.v);
-    return HD(e, e * x.a);
-  }
-  static __device__ __forceinline__ HD log_(HD x) { return HD(dlog(x.v), x.a / x.v); }
-  static __device__ __forceinline__ HD abs_(HD x) { return x.v.v < 0.0 ? -x : x; }
 };
 
 constexpr int TAN_BLOCK = 256;
@@ -176,7 +142,6 @@ __global__ __launch_bounds__(TAN_BLOCK) void k_tangent_prep(SysConst c, const do
 // Model parameters as duals along one direction.
 struct TanPar {
   Dual vdw[5], polar[4], apCC[4][4], raCC[4][4], apDD[4][4], lrc;
-  double pf[4], dpf[4];  // polfac^(-1/2) per site type and its derivative by polfac
 };
 
 struct TanArgs {
@@ -509,95 +474,9 @@ __device__ __forceinline__ void chain_d(Dual &ts, int n, double ts_next, double 
   ts.d = -0.5 * (2 * n + 1) * ts_next * dd2;
 }
 
-// Sum over the workgroup of a dual.
-__device__ __forceinline__ Dual block_sum(Dual v, double *red) {
-  const double x = block_sum(v.v, red);
-  return Dual(x, block_sum(v.d, red));
-}
-
-// The adjoint's outputs for configuration b: per parameter j of the 16 TTM
-// parameters and the 84 DMS coefficients, adj[b][j] = (dE/dtheta_j,
-// gw . d(dE/dr)/dtheta_j).  Beside the Thole and vdW partials gathered by the
-// pair loops: the polarisabilities (-1/2 |mu|^2 / alpha^2 per dipole site,
-// the alpha^-1 term of the stationary induction energy) and the charge
-// parameters (sum of phi dq/dtheta over the charged sites, phi the potential
-// of charges and dipoles, which is dE/dq).  Each is a dual along the atoms'
-// direction gw, the second part the derivative of the first along it.
-// (gammaM, the last of TTM_ADJ_NPARAM, moves the M sites: its slot is filled
-// by the host from a tangent sweep.)
-__device__ void adjoint_out(const SysConst &c, const TanArgs &a, const TanPar &P, const TanWs &W,
-                            int b, const double vE[5], const double vF[5], Dual accCC, Dual accDD,
-                            const Dual accPF[3], double *red) {
-  const int N = c.N, tid = threadIdx.x, nds = c.nd * N, tdip = c.tdip;
-  double *out = a.adj + (size_t)b * TTM_ADJ_NPARAM * 2;
-  const Dual *phi = W.phi, *q = W.q, *dip = W.dip, *dR = W.dR;
-  const double gM = c.gammaM, tq = 0.5 * gM / (1.0 - gM);
-  // polarisabilities by site type (O, H, M)
-  Dual pol[3] = {0.0, 0.0, 0.0};
-  for (int i = tid; i < nds; i += TAN_BLOCK) {
-    const int t = tdip + i / N, pt = t == 0 ? 0 : t == 3 ? 2 : 1;
-    const double al = P.polar[t].v;
-    const Dual *mu = dip + 3 * i;
-    const Dual m2 = mu[0] * mu[0] + mu[1] * mu[1] + mu[2] * mu[2];
-    if (al > 0.0) pol[pt] -= 0.5 * m2 / (al * al);
-  }
-  const Dual sCC = block_sum(accCC, red), sDD = block_sum(accDD, red);
-  Dual sPF[3], sPol[3];
-  for (int i = 0; i < 3; ++i) {
-    sPF[i] = block_sum(accPF[i], red);
-    sPol[i] = block_sum(pol[i], red);
-  }
-  double sE[5], sF[5];
-  for (int i = 0; i < 5; ++i) {
-    sE[i] = block_sum(vE[i], red);
-    sF[i] = block_sum(vF[i], red);
-  }
-  if (tid == 0) {
-    auto put = [&](int j, Dual v) {
-      out[2 * j] = v.v;
-      out[2 * j + 1] = v.d;
-    };
-    for (int i = 0; i < 5; ++i) put(TP_VDWA + i, Dual(sE[i] + (i < 3 ? a.lrc_coef[i] : 0.0), sF[i]));
-    for (int i = 0; i < 3; ++i) put(TP_POLARO + i, sPol[i]);
-    for (int i = 0; i < 3; ++i) put(TP_POLFACO + i, sPF[i]);
-    put(TP_ADD, sDD);
-    put(TP_ACC, sCC);
-    put(TTM_ADJ_NPARAM - 1, Dual(0.0));
-  }
-  // the charge parameters: dms_param1..3, then the 84 coefficients coefD;
-  // one parameter per lane over the molecules
-  for (int j = tid; j < 3 + DMS_NCOEF; j += TAN_BLOCK) {
-    Dual acc = 0.0;
-    for (int w = 0; w < N; ++w) {
-      const double *rr = a.RR + ((size_t)b * 3 * N + 3 * w) * 3;
-      const double *g = a.gw + ((size_t)b * 3 * N + 3 * w) * 3;
-      double r[3][3], dq3[3], dgq[3][3][3];
-      for (int at = 0; at < 3; ++at)
-        for (int k = 0; k < 3; ++k) r[at][k] = rr[3 * at + k];
-      if (j < 3) dms_tangent(c, r, j, dq3, dgq);
-      else dms_coef_tangent(c, r, j - 3, dq3, dgq);
-      // dq3 in (O, H1, H2), dgq[disp][charge] in (H1, H2, O); along gw
-      const int atom[3] = {1, 2, 0};
-      Dual dqd[3];
-      for (int i = 0; i < 3; ++i) {
-        const int ch = i == 0 ? 2 : i - 1;
-        double v = 0.0;
-        for (int d = 0; d < 3; ++d)
-          for (int k = 0; k < 3; ++k) v += dgq[d][ch][k] * g[3 * atom[d] + k];
-        dqd[i] = Dual(dq3[i] * CHARGECON, v * CHARGECON);
-      }
-      const Dual sH = dqd[1] + dqd[2];
-      acc += phi[N + w] * (dqd[1] + tq * sH) + phi[2 * N + w] * (dqd[2] + tq * sH) +
-             phi[3 * N + w] * dqd[0] * (1.0 / (1.0 - gM));
-    }
-    out[2 * (TP_DMS1 + j)] = acc.v;
-    out[2 * (TP_DMS1 + j) + 1] = acc.d;
-  }
-}
-
 // MODE TAN_PARAMS: one parameter direction per workgroup, plain FP64
-// geometry (GT = double); TAN_GAMMA_M and TAN_ADJOINT: dual site positions
-// and phases (GT = Dual) along dr/dgammaM or along the atoms' direction gw.
+// geometry (GT = double); TAN_GAMMA_M: dual site positions and phases
+// (GT = Dual) along dr/dgammaM.  (The adjoint has kernels of its own.)
 template <int MODE>
 __global__ __launch_bounds__(TAN_BLOCK) void k_ttm_tangent(SysConst c, TanArgs a) {
   constexpr bool GD = MODE != TAN_PARAMS;
@@ -641,11 +520,6 @@ __global__ __launch_bounds__(TAN_BLOCK) void k_ttm_tangent(SysConst c, TanArgs a
                         dpow(par(10), 1.0 / 6.0)};
     Dual pf[4];
     for (int i = 0; i < 4; ++i) pf[i] = Dual(1.0) / (f6[i] * f6[i] * f6[i]);
-    for (int i = 0; i < 4; ++i) {
-      const double pfi = a.theta[TP_POLFACO + (i == 0 ? 0 : i == 3 ? 2 : 1)];
-      P.pf[i] = pf[i].v;
-      P.dpf[i] = -0.5 * pf[i].v / pfi;  // d polfac^(-1/2) / d polfac
-    }
     const Dual aDD = par(11), aCC = par(12);
     for (int i = 0; i < 4; ++i)
       for (int j = 0; j < 4; ++j) {
@@ -663,9 +537,6 @@ __global__ __launch_bounds__(TAN_BLOCK) void k_ttm_tangent(SysConst c, TanArgs a
 
   // ---- real space: vdW and charge-charge terms (pot_ttm.f90:159-228), per site
   Dual uvdw = 0.0;
-  // adjoint: d Uvdw / d(vdwA..E) and gw . d G / d(vdwA..E) of the gradient as
-  // computed (its vdW force, pot_ttm.f90:176, has no vdwA, vdwB terms)
-  double vE[5] = {0, 0, 0, 0, 0}, vF[5] = {0, 0, 0, 0, 0};
   for (int s = tid; s < ns; s += TAN_BLOCK) {
     const int iw = s % N, ti = s / N;
     const double *ROi = Rs + 3 * iw;
@@ -688,21 +559,6 @@ __global__ __launch_bounds__(TAN_BLOCK) void k_ttm_tangent(SysConst c, TanArgs a
                            Dual(c.shiftA * (x * x) + c.shiftB * (x * x * x)));
         for (int k = 0; k < 3; ++k) gv[k] += fsc * Rij[k];
         if (iw < jw) uvdw += uij;
-        if constexpr (MODE == TAN_ADJOINT) {
-          const double Dv = P.vdw[3].v, Ev = P.vdw[4].v, e = exp(-(Ev * dRij));
-          const double *gO = a.gw + ((size_t)b * 3 * N + 3 * iw) * 3;
-          const double gr = gO[0] * Rij[0] + gO[1] * Rij[1] + gO[2] * Rij[2];
-          if (iw < jw) {
-            vE[0] += R6i * R6i;
-            vE[1] += R6i * R4i;
-            vE[2] += R6i;
-            vE[3] += e;
-            vE[4] -= Dv * dRij * e;
-          }
-          vF[2] -= 6.0 * R8i * gr;
-          vF[3] -= e * Ev / dRij * gr;
-          vF[4] -= Dv * e * (1.0 - Ev * dRij) / dRij * gr;
-        }
       }
       GT Ra[3];
       for (int k = 0; k < 3; ++k) Ra[k] = Ri[k] + (Rij[k] - ROi[k] + ROj[k]);
@@ -715,12 +571,6 @@ __global__ __launch_bounds__(TAN_BLOCK) void k_ttm_tangent(SysConst c, TanArgs a
         const GT d2s = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
         Dual ts0, ts1;
         smear01<true, Dual>(c, as_dual(d2s), P.apCC[ti][tj], P.raCC[ti][tj], ts0, ts1);
-        if constexpr (MODE == TAN_ADJOINT) {
-          double u1, u2;
-          smear2<true, double>(c, d2s.v, P.apCC[ti][tj].v, u1, u2);
-          chain_d(ts0, 0, ts1.v, d2s.d);
-          chain_d(ts1, 1, u2, d2s.d);
-        }
         const Dual qj = q[sj];
         pv += ts0 * qj;
         const Dual f = ts1 * qj;
@@ -749,12 +599,6 @@ __global__ __launch_bounds__(TAN_BLOCK) void k_ttm_tangent(SysConst c, TanArgs a
         const GT d2x = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
         GT ts0, ts1;
         self1(c, d2x, ts0, ts1);
-        if constexpr (MODE == TAN_ADJOINT) {
-          double u1, u2;
-          self2(c, d2x.v, u1, u2);
-          chain_d(ts0, 0, ts1.v, d2x.d);
-          chain_d(ts1, 1, u2, d2x.d);
-        }
         phi[si] += ts0 * q[sj];
         phi[sj] += ts0 * q[si];
         for (int k = 0; k < 3; ++k) {
@@ -847,12 +691,6 @@ __global__ __launch_bounds__(TAN_BLOCK) void k_ttm_tangent(SysConst c, TanArgs a
           Dual t1, t2, o[3];
           const GT r2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
           smear2<true, Dual>(c, as_dual(r2), P.apDD[ti][tj], t1, t2);
-          if constexpr (MODE == TAN_ADJOINT) {
-            double u1, u2, u3;
-            smear3<true, double>(c, r2.v, P.apDD[ti][tj].v, u1, u2, u3);
-            chain_d(t1, 1, t2.v, r2.d);
-            chain_d(t2, 2, u3, r2.d);
-          }
           dd3d(r, t1, t2, dip + 3 * j, o);
           for (int k = 0; k < 3; ++k) e[k] += o[k];
         }
@@ -868,12 +706,6 @@ __global__ __launch_bounds__(TAN_BLOCK) void k_ttm_tangent(SysConst c, TanArgs a
         Dual t1, t2, o[3];
         const GT r2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
         smear2<true, Dual>(c, as_dual(r2), P.apDD[ti][tj], t1, t2);
-        if constexpr (MODE == TAN_ADJOINT) {
-          double u1, u2, u3;
-          smear3<true, double>(c, r2.v, P.apDD[ti][tj].v, u1, u2, u3);
-          chain_d(t1, 1, t2.v, r2.d);
-          chain_d(t2, 2, u3, r2.d);
-        }
         dd3d(r, t1, t2, dip + 3 * j, o);
         for (int k = 0; k < 3; ++k) e[k] += o[k];
       }
@@ -933,18 +765,6 @@ __global__ __launch_bounds__(TAN_BLOCK) void k_ttm_tangent(SysConst c, TanArgs a
 
   // ---- Uind (pot_ttm.f90:390) and the final real-space forces (pot_ttm.f90:399-542)
   Dual uind = 0.0;
-  // adjoint: d U / d aCCaCD, aDD, polfacO/H/M at fixed dipoles, through the
-  // Thole factors a = a0 polfac_i^(-1/2) polfac_j^(-1/2) of each site pair
-  Dual accCC = 0.0, accDD = 0.0, accPF[3] = {0.0, 0.0, 0.0};
-  auto ptype = [](int t) { return t == 0 ? 0 : t == 3 ? 2 : 1; };
-  auto thole_acc = [&](Dual w, bool ddt, int ti, int tj) {
-    const double pi = P.pf[ti], pj = P.pf[tj];
-    if (ddt) accDD += w * (pi * pj);
-    else accCC += w * (pi * pj);
-    const Dual wa = w * a.theta[ddt ? TP_ADD : TP_ACC];
-    accPF[ptype(ti)] += wa * (pj * P.dpf[ti]);
-    accPF[ptype(tj)] += wa * (pi * P.dpf[tj]);
-  };
   for (int i = tid; i < nds; i += TAN_BLOCK) {
     const int s = (tdip + i / N) * N + i % N;
     for (int k = 0; k < 3; ++k) uind += dip[3 * i + k] * Efq[3 * s + k];
@@ -1008,52 +828,12 @@ __global__ __launch_bounds__(TAN_BLOCK) void k_ttm_tangent(SysConst c, TanArgs a
           qd = qsq > 1e-9;
           if (qd) smear2<true, Dual>(c, as_dual(d2), P.apCC[ti][tj], ts1, ts2);
         }
-        // the potential of the dipoles (phi, dE/dq) along the direction; the
-        // gradient terms (g) only feed dE/dr, which the adjoint does not use
-        if constexpr (MODE == TAN_ADJOINT) chain_d(ts1, 1, ts2.v, as_dual(d2).d);
         if (qd) {
           Dual o[3];
           dd3d(r, ts1, ts2, qdqd, o);
           for (int k = 0; k < 3; ++k) g[k] += o[k];
         }
         pv += ts1 * (dj[0] * r[0] + dj[1] * r[1] + dj[2] * r[2]);
-        if constexpr (MODE == TAN_ADJOINT) {
-          // The energy is stationary in the converged dipoles, so its
-          // derivative is the explicit one at fixed dipoles: per ordered site
-          // pair 1/2 qi qj dts0/da (Uelec), -qj (di . r) dts1/da (-mu . Efq)
-          // and -1/2 di . dT/da . dj (-1/2 mu T mu); only the Thole terms
-          // (r < 5 A, smear.f90:23,57) depend on a.
-          if (d2.v < 25.0) {
-            const bool cc = !same && qi.v != 0.0 && qj.v != 0.0, cd = !same && adip && qj.v != 0.0;
-            const double av = P.apCC[ti][tj].v, rav = P.raCC[ti][tj].v;
-            const Dual d2d = as_dual(d2);
-            if ((cc || cd) && av > 0.0) {
-              HD t0h, t1h, u1h, u2h, u3h;
-              smear01<true, HD>(c, HD(d2d, Dual(0.0)), HD(Dual(av), Dual(1.0)),
-                                HD(Dual(rav), Dual(rav / (3.0 * av))), t0h, t1h);
-              smear3<true, HD>(c, HD(d2d, Dual(0.0)), HD(Dual(av), Dual(1.0)), u1h, u2h, u3h);
-              Dual da0 = t0h.a, da1 = u1h.a;
-              chain_d(da0, 0, u1h.a.v, d2d.d);
-              chain_d(da1, 1, u2h.a.v, d2d.d);
-              Dual w = 0.0;
-              if (cc) w += 0.5 * qi * qj * da0;
-              if (cd) w -= qj * (di[0] * r[0] + di[1] * r[1] + di[2] * r[2]) * da1;
-              thole_acc(w, false, ti, tj);
-            }
-            if (adip && bdip) {
-              HD u1h, u2h, u3h;
-              smear3<true, HD>(c, HD(d2d, Dual(0.0)), HD(Dual(P.apDD[ti][tj].v), Dual(1.0)), u1h,
-                               u2h, u3h);
-              Dual da1 = u1h.a, da2 = u2h.a;
-              chain_d(da1, 1, u2h.a.v, d2d.d);
-              chain_d(da2, 2, u3h.a.v, d2d.d);
-              const Dual dir_ = di[0] * r[0] + di[1] * r[1] + di[2] * r[2];
-              const Dual djr = dj[0] * r[0] + dj[1] * r[1] + dj[2] * r[2];
-              const Dual dd = di[0] * dj[0] + di[1] * dj[1] + di[2] * dj[2];
-              thole_acc(-0.5 * (3.0 * da2 * dir_ * djr - da1 * dd), true, ti, tj);
-            }
-          }
-        }
       }
     }
     for (int k = 0; k < 3; ++k) dR[3 * s + k] += g[k];
@@ -1137,7 +917,675 @@ __global__ __launch_bounds__(TAN_BLOCK) void k_ttm_tangent(SysConst c, TanArgs a
     o[2] = a.ew[b] * Ed + lg;
     o[3] = (double)iters;
   }
-  if constexpr (MODE == TAN_ADJOINT) adjoint_out(c, a, P, W, b, vE, vF, accCC, accDD, accPF, red);
+}
+
+// ---------------------------------------------------------------------------
+// The adjoint.  A configuration's sweep is cut into kernels, each spread over
+// as many workgroups as its sites, k-vectors or site pairs fill: one workgroup
+// per configuration (64 boxes of 32 H2O: 64 workgroups of a 256-CU device, and
+// 32 of 256 lanes busy in the dipole field) took 8.8 ms.  The dipole solve is
+// the dense one of the force path, on dual numbers: the matrix and its
+// derivative along the positions' direction are formed once (k_adj_build) and
+// an iteration is a product with them (k_adj_solve).  64 five-water clusters
+// and 64 boxes of 32 H2O side by side: 8.8 -> 0.5 ms.
+//
+// Values are evaluated in plain FP64 and their position derivatives follow
+// chain_d; the Thole derivatives d ts / d a come from duals along a.
+// ---------------------------------------------------------------------------
+constexpr int ADJ_G = 16;                       // lanes per site of the pair loops
+constexpr int ADJ_SPB = TAN_BLOCK / ADJ_G;      // sites per workgroup of them
+constexpr int ADJ_NV = 11, ADJ_NA = 10;         // partial sums per workgroup
+constexpr int ADJ_BW = 8;                       // waves of k_adj_build
+constexpr int ADJ_SOLVE = 1024;
+
+struct AdjArgs {
+  TanArgs t;
+  Dual *mat;             // [slice][D][D] dipole matrix, D = 3 nd N
+  int b0;                // first configuration of the slice
+  double *pv, *pa;       // [P][pair workgroups][ADJ_NV], [ADJ_NA]
+  const int4 *cols;      // kz-columns and their first k-vectors
+  const int *colk;
+  double pf[4], dpf[4];  // polfac^(-1/2) per site type and its derivative by polfac
+};
+
+__host__ __device__ inline int adj_pair_blocks(const SysConst &c) {
+  return (4 * c.N + ADJ_SPB - 1) / ADJ_SPB;
+}
+
+// Configuration b's tables and sites.
+struct AdjCfg {
+  const double *Rs, *dS;
+  Phases ph;
+  __device__ AdjCfg(const SysConst &c, const TanArgs &a, int b) {
+    const int ns = 4 * c.N;
+    Rs = a.cfg + (size_t)b * a.cfg_stride;
+    dS = Rs + a.ds_off;
+    ph.ns = ns;
+    ph.kmax = c.kmax;
+    ph.lmax = c.lmax;
+    ph.N = c.N;
+    ph.dS = dS;
+    ph.tx = (const double2 *)(Rs + (size_t)ns * 3);
+    ph.ty = ph.tx + (size_t)(c.hmax + 1) * ns;
+    ph.tz = ph.ty + (size_t)(2 * c.kmax + 1) * ns;
+  }
+  // minimum-image vector from site sj to site si, with its derivative
+  __device__ __forceinline__ void vec(const SysConst &c, int si, int sj, Dual r[3]) const {
+    for (int k = 0; k < 3; ++k)
+      r[k] = Dual(Rs[3 * si + k] - Rs[3 * sj + k], dS[3 * si + k] - dS[3 * sj + k]);
+    minimg(c, r[0], r[1], r[2]);
+  }
+  // whether molecules i and j are within the cut-off, and their O-O vector
+  __device__ __forceinline__ bool within(const SysConst &c, int i, int j, double v[3]) const {
+    for (int k = 0; k < 3; ++k) v[k] = Rs[3 * i + k] - Rs[3 * j + k];
+    minimg(c, v[0], v[1], v[2]);
+    return norm2_exact(v[0], v[1], v[2]) < c.rc2;
+  }
+};
+
+// Sums of n values per lane over the workgroup into out (lane 0 writes).
+template <int n>
+__device__ __forceinline__ void block_sums(double *v, double (*red)[TAN_BLOCK / 64], double *out) {
+  for (int i = 0; i < n; ++i) {
+    v[i] = group_sum<64>(v[i]);
+    if ((threadIdx.x & 63) == 0) red[i][threadIdx.x >> 6] = v[i];
+  }
+  __syncthreads();
+  if (threadIdx.x < n) {
+    double s = 0.0;
+    for (int w = 0; w < TAN_BLOCK / 64; ++w) s += red[threadIdx.x][w];
+    out[threadIdx.x] = s;
+  }
+}
+
+// Real-space charge terms of a site (pot_ttm.f90:159-261): the potential at
+// the charged sites, the field at the dipole sites, the vdW sums at the
+// oxygens; ADJ_G lanes per site over the molecules.
+__global__ __launch_bounds__(TAN_BLOCK) void k_adj_pair_q(SysConst c, AdjArgs x) {
+  __shared__ double red[ADJ_NV][TAN_BLOCK / 64];
+  const TanArgs &a = x.t;
+  const int b = blockIdx.y, N = c.N, ns = 4 * N;
+  const AdjCfg g(c, a, b);
+  const TanWs W(a.ws + (size_t)b * a.ws_stride, c);
+  const int s0 = blockIdx.x * ADJ_SPB + threadIdx.x / ADJ_G, lane = threadIdx.x % ADJ_G;
+  const bool valid = s0 < ns;
+  const int s = valid ? s0 : 0, iw = s % N, ti = s / N;
+  const bool chg = ti > 0, adip = ti >= c.tdip && ti < c.tdip + c.nd;
+  Dual pv = 0.0, ef[3] = {0.0, 0.0, 0.0};
+  double v[ADJ_NV] = {0};  // uvdw, d Uvdw / d(vdwA..E), gw . dG / d(vdwA..E)
+  for (int jw = lane; valid && jw < N; jw += ADJ_G) {
+    const bool same = jw == iw;
+    double Rij[3];
+    if (!same && !g.within(c, iw, jw, Rij)) continue;
+    if (ti == 0 && !same) {
+      const double d2 = norm2_exact(Rij[0], Rij[1], Rij[2]);
+      const double d = sqrt(d2), R2i = 1.0 / d2, R4i = R2i * R2i, R6i = R4i * R2i, R8i = R6i * R2i;
+      const double e = exp(-(c.vdwE * d));
+      const double *gO = a.gw + ((size_t)b * 3 * N + 3 * iw) * 3;
+      const double gr = gO[0] * Rij[0] + gO[1] * Rij[1] + gO[2] * Rij[2];
+      if (iw < jw) {
+        v[0] += R6i * ((c.vdwA * R6i + c.vdwB * R4i) + c.vdwC) + c.vdwD * e;
+        v[1] += R6i * R6i;
+        v[2] += R6i * R4i;
+        v[3] += R6i;
+        v[4] += e;
+        v[5] -= c.vdwD * d * e;
+      }
+      // the gradient as computed: its vdW force (pot_ttm.f90:176) has no
+      // vdwA, vdwB terms
+      v[8] -= 6.0 * R8i * gr;
+      v[9] -= e * c.vdwE / d * gr;
+      v[10] -= c.vdwD * e * (1.0 - c.vdwE * d) / d * gr;
+    }
+    if (!chg && !adip) continue;
+    for (int tj = 0; tj < 4; ++tj) {
+      if ((same && tj == ti) || tj == 0) continue;  // the oxygens carry no charge
+      const int sj = tj * N + jw;
+      Dual r[3];
+      g.vec(c, s, sj, r);
+      const Dual d2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+      double t0, t1, t2 = 0.0, u1;
+      if (same) {
+        self1(c, d2.v, t0, t1);
+        if (adip) self2(c, d2.v, u1, t2);
+      } else {
+        smear01(c, d2.v, c.apolCC[ti][tj], c.raCC[ti][tj], t0, t1);
+        if (adip) smear2(c, d2.v, c.apolCC[ti][tj], u1, t2);
+      }
+      const Dual qj = W.q[sj];
+      Dual ts0 = t0;
+      chain_d(ts0, 0, t1, d2.d);
+      pv += ts0 * qj;
+      if (adip) {
+        Dual ts1 = t1;
+        chain_d(ts1, 1, t2, d2.d);
+        const Dual f = ts1 * qj;
+        for (int k = 0; k < 3; ++k) ef[k] += f * r[k];
+      }
+    }
+  }
+  pv = group_sum(pv, ADJ_G);
+  for (int k = 0; k < 3; ++k) ef[k] = group_sum(ef[k], ADJ_G);
+  if (valid && lane == 0) {
+    W.phi[s] = chg ? pv - c.self_fac * W.q[s] : Dual(0.0);
+    for (int k = 0; k < 3; ++k) W.Efq[3 * s + k] = ef[k];
+  }
+  block_sums<ADJ_NV>(v, red, x.pv + ((size_t)b * gridDim.x + blockIdx.x) * ADJ_NV);
+}
+
+// Structure factor of the charges, or of the dipoles of the last SOR step's
+// input (ewald.f90:1-119): four lanes per k-vector share its sites.
+template <bool DIP>
+__global__ __launch_bounds__(TAN_BLOCK) void k_adj_sfac(SysConst c, AdjArgs x) {
+  const TanArgs &a = x.t;
+  const int b = blockIdx.y, N = c.N;
+  const AdjCfg g(c, a, b);
+  const TanWs W(a.ws + (size_t)b * a.ws_stride, c);
+  const int k = blockIdx.x * (TAN_BLOCK / 4) + threadIdx.x / 4, u = threadIdx.x % 4;
+  if (k >= c.nk) return;  // alike over the four lanes
+  const int4 h = a.khkl[k];
+  const double4 kv = a.kv[k];
+  const int s0 = DIP ? c.tdip * N : N, n = DIP ? c.nd * N : 3 * N;
+  Dual re = 0.0, im = 0.0;
+  for (int i = u; i < n; i += 4) {
+    Dual ck, sk;
+    g.ph.at(s0 + i, h, kv, ck, sk);
+    if (DIP) {
+      const Dual *m = W.old + 3 * i;
+      const Dual dk = m[0] * kv.x + m[1] * kv.y + m[2] * kv.z;
+      re -= dk * sk;
+      im += dk * ck;
+    } else {
+      const Dual q = W.q[s0 + i];
+      re += q * ck;
+      im += q * sk;
+    }
+  }
+  re = group_sum(re, 4);
+  im = group_sum(im, 4);
+  if (u == 0) {
+    Dual *S = DIP ? W.Sm : W.Sq;
+    S[2 * k] = re;
+    S[2 * k + 1] = im;
+  }
+}
+
+// Reciprocal-space potential at the charged sites, field at the dipole sites
+// and starting dipoles (ewald.f90:45-49, pot_ttm.f90:281-297), a wave per
+// site; DIP: the potential of the dipoles (ewald.f90:184-193) onto dR, where
+// k_adj_pair_d left its real-space part.
+template <bool DIP>
+__global__ __launch_bounds__(TAN_BLOCK) void k_adj_field(SysConst c, AdjArgs x) {
+  const TanArgs &a = x.t;
+  const int b = blockIdx.y, N = c.N;
+  const int s = blockIdx.x * (TAN_BLOCK / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (s >= 4 * N) return;
+  const int ti = s / N;
+  const bool chg = ti > 0, adip = !DIP && ti >= c.tdip && ti < c.tdip + c.nd;
+  if (!chg && !adip) return;
+  const AdjCfg g(c, a, b);
+  const TanWs W(a.ws + (size_t)b * a.ws_stride, c);
+  const Dual *S = DIP ? W.Sm : W.Sq;
+  Dual ef[3] = {0.0, 0.0, 0.0}, pv = 0.0;
+  for (int k = lane; k < c.nk; k += 64) {
+    const double4 kv = a.kv[k];
+    Dual ck, sk;
+    g.ph.at(s, a.khkl[k], kv, ck, sk);
+    const Dual re = S[2 * k], im = S[2 * k + 1];
+    pv += kv.w * (ck * re + sk * im);
+    if (adip) {
+      const Dual t = kv.w * (ck * im - sk * re);
+      ef[0] -= t * kv.x;
+      ef[1] -= t * kv.y;
+      ef[2] -= t * kv.z;
+    }
+  }
+  pv = group_sum(pv, 64);
+  if (adip)
+    for (int k = 0; k < 3; ++k) ef[k] = group_sum(ef[k], 64);
+  if (lane != 0) return;
+  if (DIP) {
+    W.dR[s] += pv;
+    return;
+  }
+  if (chg) W.phi[s] += pv;
+  if (adip)
+    for (int k = 0; k < 3; ++k) {
+      const Dual e = W.Efq[3 * s + k] + ef[k];
+      W.Efq[3 * s + k] = e;
+      W.dip[3 * (s - c.tdip * N) + k] = c.polar[ti] * e;
+    }
+}
+
+// The dipole matrix with its derivative along the positions' direction: an
+// 8 x 8 tile of dipole-site pairs (i <= j) per workgroup, a lane per pair, the
+// kz-columns dealt to the waves (sums added in wave order).  With
+// phi = k.(r_i - r_j) the reciprocal part is -sum w k k cos phi and its
+// derivative +sum w k k (k.dr) sin phi: along a column kx and ky are fixed, so
+// the sums over kz of w kz^n cos phi (n <= 2) and w kz^n sin phi (n <= 3) give
+// both.  Bound by FP64 issue: 13 operations per (pair, k); 64 boxes of 32 H2O
+// (3450 k) 108 us, 40 % of the FP64 rate.
+__global__ __launch_bounds__(64 * ADJ_BW) void k_adj_build(SysConst c, AdjArgs x) {
+  __shared__ double part[ADJ_BW][12][64];
+  const TanArgs &a = x.t;
+  const int b = x.b0 + blockIdx.y, N = c.N, M = c.nd * N, sd = c.tdip * N;
+  const AdjCfg g(c, a, b);
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nt = (M + 7) / 8;
+  int ti = 0, t = blockIdx.x;
+  while (t >= nt - ti) {
+    t -= nt - ti;
+    ++ti;
+  }
+  const int i = ti * 8 + lane / 8, j = (ti + t) * 8 + lane % 8;
+  const bool valid = i < M && j < M && i <= j;
+  const int si = sd + (valid ? i : 0), sj = sd + (valid ? j : 0);
+  double dr[3];
+  for (int k = 0; k < 3; ++k) dr[k] = g.dS[3 * si + k] - g.dS[3 * sj + k];
+  auto diff = [&](const double2 *row) {
+    const double2 p = row[si], q = row[sj];
+    return make_double2(p.x * q.x + p.y * q.y, p.y * q.x - p.x * q.y);
+  };
+  auto mul = [](double2 p, double2 q) {
+    return make_double2(p.x * q.x - p.y * q.y, p.y * q.x + p.x * q.y);
+  };
+  const size_t ns = 4 * (size_t)N;
+  const double2 z1 =
+      c.lmax >= 1 ? diff(g.ph.tz + (size_t)(c.lmax + 1) * ns) : make_double2(1.0, 0.0);
+  double K[6] = {0, 0, 0, 0, 0, 0}, L[6] = {0, 0, 0, 0, 0, 0};  // xx, xy, yy, zz, xz, yz
+  for (int n = wv; n < c.ncol; n += ADJ_BW) {
+    const int4 cl = x.cols[n];
+    const int k0 = x.colk[n];
+    double2 e = mul(mul(diff(g.ph.tx + (size_t)cl.x * ns),
+                        diff(g.ph.ty + (size_t)(cl.y + c.kmax) * ns)),
+                    diff(g.ph.tz + (size_t)(cl.z + c.lmax) * ns));
+    const double kx = a.kv[k0].x, ky = a.kv[k0].y;
+    double C0 = 0, C1 = 0, C2 = 0, S0 = 0, S1 = 0, S2 = 0, S3 = 0;
+    for (int m = 0; m < cl.w; ++m) {
+      const double kz = a.kv[k0 + m].z, w = a.kv[k0 + m].w;
+      const double p = w * e.x, q = w * e.y, pz = kz * p, qz = kz * q, qzz = kz * qz;
+      C0 += p;
+      C1 += pz;
+      C2 = fma(kz, pz, C2);
+      S0 += q;
+      S1 += qz;
+      S2 += qzz;
+      S3 = fma(kz, qzz, S3);
+      e = mul(e, z1);
+    }
+    const double D = kx * dr[0] + ky * dr[1];
+    const double T0 = D * S0 + dr[2] * S1, T1 = D * S1 + dr[2] * S2, T2 = D * S2 + dr[2] * S3;
+    K[0] -= kx * kx * C0;
+    K[1] -= kx * ky * C0;
+    K[2] -= ky * ky * C0;
+    K[3] -= C2;
+    K[4] -= kx * C1;
+    K[5] -= ky * C1;
+    L[0] += kx * kx * T0;
+    L[1] += kx * ky * T0;
+    L[2] += ky * ky * T0;
+    L[3] += T2;
+    L[4] += kx * T1;
+    L[5] += ky * T1;
+  }
+  for (int q = 0; q < 6; ++q) {
+    part[wv][q][lane] = K[q];
+    part[wv][6 + q][lane] = L[q];
+  }
+  __syncthreads();
+  if (wv != 0 || !valid) return;
+  Dual E[6];
+  for (int q = 0; q < 6; ++q) {
+    double k = part[0][q][lane], l = part[0][6 + q][lane];
+    for (int w = 1; w < ADJ_BW; ++w) {
+      k += part[w][q][lane];
+      l += part[w][6 + q][lane];
+    }
+    E[q] = Dual(k, l);
+  }
+  const int wi = i % N, wj = j % N, ui = c.tdip + i / N, uj = c.tdip + j / N;
+  double R[3];
+  if (wi == wj ? i != j : g.within(c, wi, wj, R)) {
+    Dual r[3];
+    g.vec(c, si, sj, r);
+    const Dual d2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+    double u1, u2, u3;
+    smear3(c, d2.v, c.apolDD[ui][uj], u1, u2, u3);
+    Dual t1 = u1, t2 = u2;
+    chain_d(t1, 1, u2, d2.d);
+    chain_d(t2, 2, u3, d2.d);
+    const Dual t3 = 3.0 * t2;
+    E[0] += t3 * r[0] * r[0] - t1;
+    E[1] += t3 * r[0] * r[1];
+    E[2] += t3 * r[1] * r[1] - t1;
+    E[3] += t3 * r[2] * r[2] - t1;
+    E[4] += t3 * r[0] * r[2];
+    E[5] += t3 * r[1] * r[2];
+  }
+  const size_t D = 3 * (size_t)M;
+  Dual *m = x.mat + (size_t)blockIdx.y * D * D;
+  const Dual v[3][3] = {{E[0], E[1], E[4]}, {E[1], E[2], E[5]}, {E[4], E[5], E[3]}};
+  for (int p = 0; p < 3; ++p)
+    for (int q = 0; q < 3; ++q) {
+      m[(3 * i + p) * D + 3 * j + q] = v[p][q];
+      if (i != j) m[(3 * j + p) * D + 3 * i + q] = v[p][q];
+    }
+}
+
+// The SOR iterations (pot_ttm.f90:306-392) on duals, one workgroup per
+// configuration: 16 lanes per matrix row, the matrix streamed from L2 (147 KB
+// for 32 H2O, about 3 us per iteration: 64 B per clock into one CU), the
+// dipoles in LDS or, beyond 2048 components, in global memory.  Leaves the final dipoles in dip and the last step's input in old.
+template <bool LDS>
+__global__ __launch_bounds__(ADJ_SOLVE) void k_adj_solve(SysConst c, AdjArgs x) {
+  extern __shared__ Dual lds_mu[];  // [2][D]
+  __shared__ double red[2][ADJ_SOLVE / 64];
+  const TanArgs &a = x.t;
+  const int b = x.b0 + blockIdx.x, N = c.N, D = 3 * c.nd * N, sd = c.tdip * N;
+  const TanWs W(a.ws + (size_t)b * a.ws_stride, c);
+  const Dual *m = x.mat + (size_t)blockIdx.x * D * D;
+  const int g = threadIdx.x >> 4, u = threadIdx.x & 15;
+  Dual *buf[2] = {W.dip, W.old};
+  if constexpr (LDS) {
+    buf[0] = lds_mu;
+    buf[1] = lds_mu + D;
+    for (int e = threadIdx.x; e < D; e += ADJ_SOLVE) lds_mu[e] = W.dip[e];
+    __syncthreads();
+  }
+  const double om = c.sor;
+  int cur = 0;
+  for (int it = 1;; ++it) {
+    const Dual *mu = LDS ? lds_mu + (size_t)cur * D : buf[cur];
+    Dual *nu = LDS ? lds_mu + (size_t)(cur ^ 1) * D : buf[cur ^ 1];
+    double ss = 0.0;
+    for (int row = g; row < D; row += ADJ_SOLVE / 16) {
+      const Dual *A = m + (size_t)row * D;
+      Dual f = 0.0;
+#pragma unroll 4
+      for (int col = u; col < D; col += 16) f += A[col] * mu[col];
+      f = group_sum(f, 16);
+      if (u == 0) {
+        const Dual mr = mu[row], ek = f + W.Efq[3 * sd + row] + c.fac_dd * mr;
+        const Dual nr = (1.0 - om) * mr + (om * c.polar[c.tdip + row / (3 * N)]) * ek;
+        const double df = nr.v - (it == 1 ? 0.0 : mr.v);
+        ss += df * df;
+        nu[row] = nr;
+      }
+    }
+    ss = pimd::group_sum<64>(ss);
+    if ((threadIdx.x & 63) == 0) red[it & 1][threadIdx.x >> 6] = ss;
+    __syncthreads();
+    double sum = 0.0;
+    for (int w = 0; w < ADJ_SOLVE / 64; ++w) sum += red[it & 1][w];
+    cur ^= 1;
+    if (c.stath * sqrt(sum) < c.peps || it >= c.maxiter) break;
+  }
+  if constexpr (LDS) {
+    for (int e = threadIdx.x; e < D; e += ADJ_SOLVE) {
+      W.dip[e] = lds_mu[(size_t)cur * D + e];
+      W.old[e] = lds_mu[(size_t)(cur ^ 1) * D + e];
+    }
+  } else if (cur == 1) {  // the final dipoles are in old: exchange the buffers
+    for (int e = threadIdx.x; e < D; e += ADJ_SOLVE) {
+      const Dual t = W.dip[e];
+      W.dip[e] = W.old[e];
+      W.old[e] = t;
+    }
+  }
+}
+
+// The dipoles' potential at the charged sites (into dR) and d U / d (aCCaCD,
+// aDD, polfacO/H/M) at fixed dipoles, through the Thole factors
+// a = a0 polfac_i^(-1/2) polfac_j^(-1/2) of each ordered site pair.  The energy
+// is stationary in the converged dipoles, so its derivative is the explicit
+// one: 1/2 qi qj dts0/da (Uelec), -qj (di . r) dts1/da (-mu . Efq) and
+// -1/2 di . dT/da . dj (-1/2 mu T mu); only the Thole terms (r < 5 A,
+// smear.f90:23,57) depend on a.
+__global__ __launch_bounds__(TAN_BLOCK) void k_adj_pair_d(SysConst c, AdjArgs x) {
+  __shared__ double red[ADJ_NA][TAN_BLOCK / 64];
+  const TanArgs &a = x.t;
+  const int b = blockIdx.y, N = c.N, ns = 4 * N, tend = c.tdip + c.nd;
+  const AdjCfg g(c, a, b);
+  const TanWs W(a.ws + (size_t)b * a.ws_stride, c);
+  const int s0 = blockIdx.x * ADJ_SPB + threadIdx.x / ADJ_G, lane = threadIdx.x % ADJ_G;
+  const bool valid = s0 < ns;
+  const int s = valid ? s0 : 0, iw = s % N, ti = s / N;
+  const bool chg = ti > 0, adip = ti >= c.tdip && ti < tend;
+  Dual accCC = 0.0, accDD = 0.0, accPF[3] = {0.0, 0.0, 0.0}, pv = 0.0;
+  auto ptype = [](int t) { return t == 0 ? 0 : t == 3 ? 2 : 1; };
+  auto thole_acc = [&](Dual w, bool ddt, int tj) {
+    const double pi = x.pf[ti], pj = x.pf[tj];
+    if (ddt) accDD += w * (pi * pj);
+    else accCC += w * (pi * pj);
+    const Dual wa = w * a.theta[ddt ? TP_ADD : TP_ACC];
+    const Dual wi = wa * (pj * x.dpf[ti]), wj = wa * (pi * x.dpf[tj]);
+    // constant indices: the accumulators stay in registers
+    for (int q = 0; q < 3; ++q) {
+      if (ptype(ti) == q) accPF[q] += wi;
+      if (ptype(tj) == q) accPF[q] += wj;
+    }
+  };
+  const Dual qi = W.q[s];
+  Dual di[3] = {0.0, 0.0, 0.0};
+  if (adip)
+    for (int k = 0; k < 3; ++k) di[k] = W.dip[3 * (s - c.tdip * N) + k];
+  for (int jw = lane; valid && (chg || adip) && jw < N; jw += ADJ_G) {
+    const bool same = jw == iw;
+    double Rij[3];
+    if (!same && !g.within(c, iw, jw, Rij)) continue;
+    for (int tj = 0; tj < 4; ++tj) {
+      if (same && tj == ti) continue;
+      const bool bdip = tj >= c.tdip && tj < tend, bchg = tj > 0;
+      if (!bdip && !bchg) continue;
+      const int sj = tj * N + jw;
+      Dual r[3];
+      g.vec(c, s, sj, r);
+      const Dual d2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+      const Dual qj = W.q[sj];
+      Dual dj[3] = {0.0, 0.0, 0.0};
+      if (bdip)
+        for (int k = 0; k < 3; ++k) dj[k] = W.dip[3 * (sj - c.tdip * N) + k];
+      if (bdip && chg) {
+        double qsq = 0.0, t1, t2;
+        for (int k = 0; k < 3; ++k) {
+          const double qd = qj.v * di[k].v - qi.v * dj[k].v;
+          qsq += qd * qd;
+        }
+        if (same || qsq > 1e-9) {
+          if (same) self2(c, d2.v, t1, t2);
+          else smear2(c, d2.v, c.apolCC[ti][tj], t1, t2);
+          Dual ts1 = t1;
+          chain_d(ts1, 1, t2, d2.d);
+          pv += ts1 * (dj[0] * r[0] + dj[1] * r[1] + dj[2] * r[2]);
+        }
+      }
+      if (!(d2.v < 25.0)) continue;
+      const bool cc = !same && qi.v != 0.0 && qj.v != 0.0, cd = !same && adip && qj.v != 0.0;
+      const double av = c.apolCC[ti][tj], rav = c.raCC[ti][tj];
+      Dual t0, t1, u1, u2, u3;
+      if ((cc || cd) && av > 0.0) {
+        // duals along a; their position derivatives by the chain
+        smear3<true, Dual>(c, Dual(d2.v), Dual(av, 1.0), u1, u2, u3);
+        Dual w = 0.0;
+        if (cc) {
+          smear01<true, Dual>(c, Dual(d2.v), Dual(av, 1.0), Dual(rav, rav / (3.0 * av)), t0, t1);
+          Dual da0 = t0.d;
+          chain_d(da0, 0, u1.d, d2.d);
+          w += 0.5 * qi * qj * da0;
+        }
+        if (cd) {
+          Dual da1 = u1.d;
+          chain_d(da1, 1, u2.d, d2.d);
+          w -= qj * (di[0] * r[0] + di[1] * r[1] + di[2] * r[2]) * da1;
+        }
+        thole_acc(w, false, tj);
+      }
+      if (adip && bdip) {
+        smear3<true, Dual>(c, Dual(d2.v), Dual(c.apolDD[ti][tj], 1.0), u1, u2, u3);
+        Dual da1 = u1.d, da2 = u2.d;
+        chain_d(da1, 1, u2.d, d2.d);
+        chain_d(da2, 2, u3.d, d2.d);
+        const Dual dir_ = di[0] * r[0] + di[1] * r[1] + di[2] * r[2];
+        const Dual djr = dj[0] * r[0] + dj[1] * r[1] + dj[2] * r[2];
+        const Dual dd = di[0] * dj[0] + di[1] * dj[1] + di[2] * dj[2];
+        thole_acc(-0.5 * (3.0 * da2 * dir_ * djr - da1 * dd), true, tj);
+      }
+    }
+  }
+  pv = group_sum(pv, ADJ_G);
+  if (valid && lane == 0) W.dR[s] = pv;
+  double v[ADJ_NA] = {accCC.v, accCC.d, accDD.v, accDD.d, accPF[0].v, accPF[0].d,
+                      accPF[1].v, accPF[1].d, accPF[2].v, accPF[2].d};
+  block_sums<ADJ_NA>(v, red, x.pa + ((size_t)b * gridDim.x + blockIdx.x) * ADJ_NA);
+}
+
+// The adjoint's outputs for configuration b: per parameter j of the 16 TTM
+// parameters and the 84 DMS coefficients, adj[b][j] = (dE/dtheta_j,
+// gw . d(dE/dr)/dtheta_j), and the energy.  Beside the Thole and vdW partials
+// of the pair kernels: the polarisabilities (-1/2 |mu|^2 / alpha^2 per dipole
+// site, the alpha^-1 term of the stationary induction energy) in workgroup 0,
+// and the charge parameters (sum of phi dq/dtheta over the charged sites, phi
+// the potential of charges and dipoles, which is dE/dq) in the others, eight
+// lanes per parameter over the molecules.  (gammaM, the last of
+// TTM_ADJ_NPARAM, moves the M sites: its slot is filled by the host from a
+// tangent sweep.)
+constexpr int ADJ_PPB = TAN_BLOCK / 8;  // charge parameters per workgroup
+__global__ __launch_bounds__(TAN_BLOCK) void k_adj_out(SysConst c, AdjArgs x) {
+  __shared__ double red[TAN_BLOCK];
+  const TanArgs &a = x.t;
+  const int b = blockIdx.y, N = c.N, tid = threadIdx.x;
+  const TanWs W(a.ws + (size_t)b * a.ws_stride, c);
+  double *out = a.adj + (size_t)b * TTM_ADJ_NPARAM * 2;
+  if (blockIdx.x == 0) {
+    const int nds = c.nd * N, nb = adj_pair_blocks(c);
+    Dual pol[3] = {0.0, 0.0, 0.0};  // by site type (O, H, M)
+    double ue = 0.0, ui = 0.0;
+    for (int i = tid; i < nds; i += TAN_BLOCK) {
+      const int t = c.tdip + i / N, pt = t == 0 ? 0 : t == 3 ? 2 : 1;
+      const double al = c.polar[t];
+      const Dual *mu = W.dip + 3 * i, *e = W.Efq + 3 * (c.tdip * N + i);
+      const Dual m2 = mu[0] * mu[0] + mu[1] * mu[1] + mu[2] * mu[2];
+      for (int q = 0; q < 3; ++q)
+        if (q == pt && al > 0.0) pol[q] -= 0.5 * m2 / (al * al);
+      for (int k = 0; k < 3; ++k) ui += mu[k].v * e[k].v;
+    }
+    for (int s = N + tid; s < 4 * N; s += TAN_BLOCK) ue += W.q[s].v * W.phi[s].v;
+    Dual sPol[3];
+    for (int i = 0; i < 3; ++i)
+      sPol[i] = Dual(block_sum(pol[i].v, red), block_sum(pol[i].d, red));
+    ue = block_sum(ue, red);
+    ui = block_sum(ui, red);
+    if (tid != 0) return;
+    double sv[ADJ_NV] = {0}, sa[ADJ_NA] = {0};
+    for (int q = 0; q < nb; ++q) {
+      for (int i = 0; i < ADJ_NV; ++i) sv[i] += x.pv[((size_t)b * nb + q) * ADJ_NV + i];
+      for (int i = 0; i < ADJ_NA; ++i) sa[i] += x.pa[((size_t)b * nb + q) * ADJ_NA + i];
+    }
+    auto put = [&](int j, double v, double d) {
+      out[2 * j] = v;
+      out[2 * j + 1] = d;
+    };
+    for (int i = 0; i < 5; ++i)
+      put(TP_VDWA + i, sv[1 + i] + (i < 3 ? a.lrc_coef[i] : 0.0), sv[6 + i]);
+    for (int i = 0; i < 3; ++i) put(TP_POLARO + i, sPol[i].v, sPol[i].d);
+    for (int i = 0; i < 3; ++i) put(TP_POLFACO + i, sa[4 + 2 * i], sa[5 + 2 * i]);
+    put(TP_ADD, sa[2], sa[3]);
+    put(TP_ACC, sa[0], sa[1]);
+    put(TTM_ADJ_NPARAM - 1, 0.0, 0.0);
+    double *o = a.out + (size_t)b * 4;
+    o[0] = W.umon->v + sv[0] + 0.5 * ue - 0.5 * ui + c.Uvdw_lrc;
+    o[1] = o[2] = o[3] = 0.0;
+    return;
+  }
+  // dms_param1..3, then the 84 coefficients coefD
+  const int j = (blockIdx.x - 1) * ADJ_PPB + tid / 8;
+  const double gM = c.gammaM, tq = 0.5 * gM / (1.0 - gM);
+  Dual acc = 0.0;
+  for (int w = tid % 8; j < 3 + DMS_NCOEF && w < N; w += 8) {
+    const double *rr = a.RR + ((size_t)b * 3 * N + 3 * w) * 3;
+    const double *gw = a.gw + ((size_t)b * 3 * N + 3 * w) * 3;
+    double r[3][3], dq3[3], dgq[3][3][3];
+    for (int at = 0; at < 3; ++at)
+      for (int k = 0; k < 3; ++k) r[at][k] = rr[3 * at + k];
+    if (j < 3) dms_tangent(c, r, j, dq3, dgq);
+    else dms_coef_tangent(c, r, j - 3, dq3, dgq);
+    // dq3 in (O, H1, H2), dgq[disp][charge] in (H1, H2, O); along gw
+    const int atom[3] = {1, 2, 0};
+    Dual dqd[3];
+    for (int i = 0; i < 3; ++i) {
+      const int ch = i == 0 ? 2 : i - 1;
+      double v = 0.0;
+      for (int d = 0; d < 3; ++d)
+        for (int k = 0; k < 3; ++k) v += dgq[d][ch][k] * gw[3 * atom[d] + k];
+      dqd[i] = Dual(dq3[i] * CHARGECON, v * CHARGECON);
+    }
+    const Dual sH = dqd[1] + dqd[2];
+    const Dual p1 = W.phi[N + w] + W.dR[N + w], p2 = W.phi[2 * N + w] + W.dR[2 * N + w],
+               pm = W.phi[3 * N + w] + W.dR[3 * N + w];
+    acc += p1 * (dqd[1] + tq * sH) + p2 * (dqd[2] + tq * sH) + pm * dqd[0] * (1.0 / (1.0 - gM));
+  }
+  acc = group_sum(acc, 8);
+  if (tid % 8 == 0 && j < 3 + DMS_NCOEF) {
+    out[2 * (TP_DMS1 + j)] = acc.v;
+    out[2 * (TP_DMS1 + j) + 1] = acc.d;
+  }
+}
+
+// Configurations whose dipole matrices are held at a time (PIMD_ADJ_MAT_MB of
+// them, default 1024, at least one), and the adjoint's workspace beyond the
+// duals of tangent_ws_duals: the matrices and the pair kernels' partial sums.
+static size_t adj_mat_duals(const SysConst &c) {
+  const size_t D = 3 * (size_t)c.nd * c.N;
+  return D * D;
+}
+static size_t adj_slice(const SysConst &c) {
+  const char *e = std::getenv("PIMD_ADJ_MAT_MB");
+  const long mb = e ? std::strtol(e, nullptr, 10) : 0;
+  const size_t n = ((size_t)(mb > 0 ? mb : 1024) << 20) / (sizeof(Dual) * adj_mat_duals(c));
+  return std::min((size_t)c.P, std::max<size_t>(n, 1));
+}
+size_t adjoint_extra_doubles(const SysConst &c) {
+  return 2 * adj_slice(c) * adj_mat_duals(c) +
+         (size_t)c.P * adj_pair_blocks(c) * (ADJ_NV + ADJ_NA);
+}
+
+static void launch_adjoint(const SysConst &c, const TanLaunch &L, const TanArgs &a, hipStream_t s) {
+  AdjArgs x;
+  x.t = a;
+  x.mat = (Dual *)L.extra;
+  x.pv = L.extra + 2 * adj_slice(c) * adj_mat_duals(c);
+  x.pa = x.pv + (size_t)c.P * adj_pair_blocks(c) * ADJ_NV;
+  x.cols = L.cols;
+  x.colk = L.colk;
+  x.b0 = 0;
+  for (int i = 0; i < 4; ++i) {
+    // polfac^(-1/2) as (polfac^(1/6))^-3 (potential.f90:157-160)
+    const double p = L.theta[TP_POLFACO + (i == 0 ? 0 : i == 3 ? 2 : 1)], f6 = std::pow(p, 1.0 / 6.0);
+    x.pf[i] = 1.0 / (f6 * f6 * f6);
+    x.dpf[i] = -0.5 * x.pf[i] / p;
+  }
+  const int P = c.P, ns = 4 * c.N, M = c.nd * c.N, D = 3 * M, nt = (M + 7) / 8;
+  const dim3 B(TAN_BLOCK), gp(adj_pair_blocks(c), P), gs((c.nk + TAN_BLOCK / 4 - 1) / (TAN_BLOCK / 4), P),
+      gf((ns + TAN_BLOCK / 64 - 1) / (TAN_BLOCK / 64), P);
+  hipLaunchKernelGGL(k_tangent_monomer<TAN_ADJOINT>, dim3(P, 1), B, 0, s, c, a);
+  hipLaunchKernelGGL(k_adj_pair_q, gp, B, 0, s, c, x);
+  hipLaunchKernelGGL(k_adj_sfac<false>, gs, B, 0, s, c, x);
+  hipLaunchKernelGGL(k_adj_field<false>, gf, B, 0, s, c, x);
+  const int slice = (int)adj_slice(c);
+  for (int b0 = 0; b0 < P; b0 += slice) {
+    const int n = std::min(slice, P - b0);
+    x.b0 = b0;
+    hipLaunchKernelGGL(k_adj_build, dim3(nt * (nt + 1) / 2, n), dim3(64 * ADJ_BW), 0, s, c, x);
+    if (D <= 2048)
+      hipLaunchKernelGGL(k_adj_solve<true>, dim3(n), dim3(ADJ_SOLVE), 2 * sizeof(Dual) * D, s, c, x);
+    else
+      hipLaunchKernelGGL(k_adj_solve<false>, dim3(n), dim3(ADJ_SOLVE), 0, s, c, x);
+  }
+  hipLaunchKernelGGL(k_adj_sfac<true>, gs, B, 0, s, c, x);
+  hipLaunchKernelGGL(k_adj_pair_d, gp, B, 0, s, c, x);
+  hipLaunchKernelGGL(k_adj_field<true>, gf, B, 0, s, c, x);
+  hipLaunchKernelGGL(k_adj_out, dim3(1 + (3 + DMS_NCOEF + ADJ_PPB - 1) / ADJ_PPB, P), B, 0, s, c, x);
 }
 
 void launch_ttm_tangent(const SysConst &c, const TanLaunch &L, hipStream_t s) {
@@ -1165,8 +1613,7 @@ void launch_ttm_tangent(const SysConst &c, const TanLaunch &L, hipStream_t s) {
   a.ds_off = ds_off;
   a.adj = L.adj;
   if (mode == TAN_ADJOINT) {
-    hipLaunchKernelGGL(k_tangent_monomer<TAN_ADJOINT>, dim3(c.P, 1), dim3(TAN_BLOCK), 0, s, c, a);
-    hipLaunchKernelGGL(k_ttm_tangent<TAN_ADJOINT>, dim3(c.P, 1), dim3(TAN_BLOCK), 0, s, c, a);
+    launch_adjoint(c, L, a, s);
   } else if (mode == TAN_GAMMA_M) {
     hipLaunchKernelGGL(k_tangent_monomer<TAN_GAMMA_M>, dim3(c.P, 1), dim3(TAN_BLOCK), 0, s, c, a);
     hipLaunchKernelGGL(k_ttm_tangent<TAN_GAMMA_M>, dim3(c.P, 1), dim3(TAN_BLOCK), 0, s, c, a);
