@@ -20,20 +20,14 @@ __device__ __forceinline__ void flag_nonfinite(int *flags, const double (&r)[3][
 }
 
 
-// Exponent tables of the PES and DMS bases, built at compile time into the
-// constant memory of each unit that uses them (the PES and DMS coefficients
-// are per context, in its parameter array).
+// Exponent table of the DMS basis, built at compile time into the constant
+// memory of each unit that uses it (the PES and DMS coefficients are per
+// context, in its parameter array).
 struct PsTables {
-  int idx[PS_NTERM][3];
   int idxd[PS_NDMS][3];
 };
 constexpr PsTables make_ps_tables() {
   PsTables t{};
-  for (int j = 0; j < PS_NTERM; ++j) {
-    t.idx[j][0] = PS_IDX1[j];
-    t.idx[j][1] = PS_IDX2[j];
-    t.idx[j][2] = PS_IDX3[j];
-  }
   for (int j = 0; j < PS_NDMS; ++j) {
     t.idxd[j][0] = PS_IDXD1[j];
     t.idxd[j][1] = PS_IDXD2[j];
@@ -42,6 +36,45 @@ constexpr PsTables make_ps_tables() {
   return t;
 }
 static __constant__ PsTables c_ps = make_ps_tables();
+
+// The order of the PES terms: by the sum deg = I + J of the stretch exponents
+// (2..10, I >= J), then I, then the bend's exponent K = 1..17 - deg.  Number of
+// the pair (I, deg - I) and its first term.
+constexpr int ps_group(int deg, int I) {
+  int g = 0;
+  for (int d = 2; d < deg; ++d) g += d / 2;
+  return g + I - (deg + 1) / 2;
+}
+constexpr int ps_first(int deg, int I) {
+  int j = 0;
+  for (int d = 2; d < deg; ++d) j += (d / 2) * (17 - d);
+  return j + (I - (deg + 1) / 2) * (17 - deg);
+}
+// The order of the DMS terms: by total degree of (i, k, m) (exponents from 0),
+// then i, then k.
+constexpr int DMS_DEG = 6;
+constexpr int dms_term(int i, int k, int m) {
+  const int d = i + k + m;
+  int j = d * (d + 1) * (d + 2) / 6 + k;
+  for (int a = 0; a < i; ++a) j += d + 1 - a;
+  return j;
+}
+constexpr bool ps_order_ok() {
+  for (int deg = 2; deg <= 10; ++deg)
+    for (int I = (deg + 1) / 2; I < deg; ++I)
+      for (int k = 0; k < 17 - deg; ++k) {
+        const int j = ps_first(deg, I) + k;
+        if (PS_IDX1[j] != I || PS_IDX2[j] != deg - I || PS_IDX3[j] != k + 1) return false;
+      }
+  for (int i = 0; i <= DMS_DEG; ++i)
+    for (int k = 0; i + k <= DMS_DEG; ++k)
+      for (int m = 0; i + k + m <= DMS_DEG; ++m) {
+        const int j = dms_term(i, k, m);
+        if (PS_IDXD1[j] != i + 1 || PS_IDXD2[j] != k + 1 || PS_IDXD3[j] != m + 1) return false;
+      }
+  return ps_first(10, 9) + 7 == PS_NTERM && dms_term(DMS_DEG, 0, 0) + 1 == PS_NDMS;
+}
+static_assert(ps_order_ok(), "the term loops of ps_monomer follow the tables' order");
 
 // Nearest integer for the minimum image.  The reference's anint rounds halves
 // away from zero; rint rounds them to even.  The two differ only when r/box is
@@ -76,11 +109,36 @@ struct WaveSplit {
   }
 };
 
-// Sum over the G lanes of a lane group (G a power of two, groups aligned).
+// Sum over the G lanes of a lane group (G a power of two, groups aligned),
+// the same on every lane of it.  Within a row of 16 lanes by DPP moves (lanes
+// 1 and 2 apart, then the mirrored half row and row, whose quads hold equal
+// sums), across rows by the row and half-wave swaps: register moves, where a
+// shuffle is an LDS instruction with its latency, twice per double and step.
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+  return v + __hiloint2double(hi, lo);
+}
 template <int G>
 __device__ __forceinline__ double group_sum(double v) {
-#pragma unroll
-  for (int off = G / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, G);
+  static_assert(G == 1 || G == 2 || G == 4 || G == 8 || G == 16 || G == 32 || G == 64, "lanes");
+  if constexpr (G >= 2) v = dpp_add<0xB1>(v);    // quad_perm [1, 0, 3, 2]
+  if constexpr (G >= 4) v = dpp_add<0x4E>(v);    // quad_perm [2, 3, 0, 1]
+  if constexpr (G >= 8) v = dpp_add<0x141>(v);   // row_half_mirror
+  if constexpr (G >= 16) v = dpp_add<0x140>(v);  // row_mirror
+  if constexpr (G >= 32) {
+    const unsigned l = __double2loint(v), h = __double2hiint(v);
+    const auto a = __builtin_amdgcn_permlane16_swap(l, l, false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap(h, h, false, false);
+    v = __hiloint2double(b[0], a[0]) + __hiloint2double(b[1], a[1]);
+  }
+  if constexpr (G >= 64) {
+    const unsigned l = __double2loint(v), h = __double2hiint(v);
+    const auto a = __builtin_amdgcn_permlane32_swap(l, l, false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(h, h, false, false);
+    v = __hiloint2double(b[0], a[0]) + __hiloint2double(b[1], a[1]);
+  }
   return v;
 }
 
@@ -426,15 +484,14 @@ __device__ inline void ps_monomer(const SysConst &c, const double r[3][3], doubl
   double costh = (R1[0] * R2[0] + R1[1] * R2[1] + R1[2] * R2[2]) / (d1 * d2);
   const double costhe = -.24780227221366464506;
   double x1 = (d1 - PS_REOH) / PS_REOH, x2 = (d2 - PS_REOH) / PS_REOH, x3 = costh - costhe;
-  // powers x^(n-1) for n = 0..15 with x^(-1) := 0 (fmat of nasa.f90:61-67)
-  double f1[16], f2[16], f3[16];
-  f1[0] = f2[0] = f3[0] = 0.0;
-  f1[1] = f2[1] = f3[1] = 1.0;
+  // powers x^(n-1) for n = 0..9 with x^(-1) := 0 (fmat of nasa.f90:61-67)
+  double f1[10], f2[10];
+  f1[0] = f2[0] = 0.0;
+  f1[1] = f2[1] = 1.0;
 #pragma unroll
-  for (int j = 2; j < 16; ++j) {
+  for (int j = 2; j < 10; ++j) {
     f1[j] = f1[j - 1] * x1;
     f2[j] = f2[j - 1] * x2;
-    f3[j] = f3[j - 1] * x3;
   }
   // ---- potential energy surface
   double deoh = PS_F5Z * deohA;
@@ -449,18 +506,33 @@ __device__ inline void ps_monomer(const SysConst &c, const double r[3][3], doubl
   double dVb = -phh2 * Vb / dh;
   double efac = exp(-PS_B1 * ((d1 - PS_REOH) * (d1 - PS_REOH) + (d2 - PS_REOH) * (d2 - PS_REOH)));
   double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-  // the loop is unrolled, so the table indices are constants; a part skips
-  // the other parts' terms with a branch that is uniform across the wave
+  // Terms of one pair of stretch exponents are consecutive with the bend's
+  // exponent running from 0 (ps_order_ok): a polynomial in x3, evaluated with
+  // its derivative by Horner's rule (two FMAs per term instead of fourteen
+  // operations: k_monomer 30 -> 18 us at 512 H2O x 32 beads, the fast forces of
+  // contracted MD 12.5 -> 6.4 us; bound by the
+  // latency of one chain per wave and the coefficients' scalar loads).  The
+  // loops are unrolled, so exponents and coefficient offsets are constants; a
+  // part skips the other parts' pairs with a branch that is uniform across
+  // the wave.
 #pragma unroll
-  for (int j = 1; j < PS_NTERM; ++j) {
-    if (L > 1 && (j - 1) % L != part) continue;
-    int I = c_ps.idx[j][0], J = c_ps.idx[j][1], K = c_ps.idx[j][2];
-    double cz = pes[j];
-    double fI1 = f1[I], fJ2 = f2[J], fJ1 = f1[J], fI2 = f2[I], fK3 = f3[K];
-    s0 = s0 + cz * (fI1 * fJ2 + fJ1 * fI2) * fK3;
-    s1 = s1 + cz * ((double)(I - 1) * f1[I - 1] * fJ2 + (double)(J - 1) * f1[J - 1] * fI2) * fK3;
-    s2 = s2 + cz * ((double)(J - 1) * fI1 * f2[J - 1] + (double)(I - 1) * fJ1 * f2[I - 1]) * fK3;
-    s3 = s3 + cz * (fI1 * fJ2 + fJ1 * fI2) * (double)(K - 1) * f3[K - 1];
+  for (int deg = 2; deg <= 10; ++deg) {
+#pragma unroll
+    for (int I = (deg + 1) / 2; I < deg; ++I) {
+      if (L > 1 && ps_group(deg, I) % L != part) continue;
+      const int J = deg - I, n = 17 - deg, j0 = ps_first(deg, I);
+      double q = 0.0, dq = 0.0;  // sum c x3^k and its derivative
+#pragma unroll
+      for (int k = n - 1; k >= 0; --k) {
+        dq = fma(dq, x3, q);
+        q = fma(q, x3, j0 + k == 0 ? 0.0 : pes[j0 + k]);  // the constant is apart
+      }
+      const double f = f1[I] * f2[J] + f1[J] * f2[I];
+      s0 = fma(f, q, s0);
+      s3 = fma(f, dq, s3);
+      s1 = fma((double)(I - 1) * f1[I - 1] * f2[J] + (double)(J - 1) * f1[J - 1] * f2[I], q, s1);
+      s2 = fma((double)(J - 1) * f1[I] * f2[J - 1] + (double)(I - 1) * f1[J] * f2[I - 1], q, s2);
+    }
   }
   if (L > 1) {
     double v[4] = {s0, s1, s2, s3};
@@ -494,19 +566,30 @@ __device__ inline void ps_monomer(const SysConst &c, const double r[3][3], doubl
   double efd = exp(-DMS_B1D * ((d1 - PS_REOH) * (d1 - PS_REOH) + (d2 - PS_REOH) * (d2 - PS_REOH)));
   double P1 = 0, P2 = 0, PL1 = costh, PL2 = 0.5 * (3.0 * PL1 * PL1 - 1.0);
   double p1r1 = 0, p1r2 = 0, p1c = 0, p2r1 = 0, p2r2 = 0, p2c = 0;
+  // as above; the terms run by total degree, and for each pair of stretch
+  // exponents the bend's by one per degree (dms_term)
 #pragma unroll
-  for (int j = 1; j < PS_NDMS; ++j) {
-    if (L > 1 && (j - 1) % L != part) continue;
-    int I = c_ps.idxd[j][0], J = c_ps.idxd[j][1], K = c_ps.idxd[j][2];
-    double cj = pes[PES_DMSC + j];
-    P1 = P1 + cj * f1[I] * f2[J] * f3[K];
-    P2 = P2 + cj * f1[J] * f2[I] * f3[K];
-    p1r1 = p1r1 + cj * ((double)(I - 1) * f1[I - 1] * f2[J] * f3[K]);
-    p1r2 = p1r2 + cj * ((double)(J - 1) * f1[I] * f2[J - 1] * f3[K]);
-    p1c = p1c + cj * ((double)(K - 1) * f1[I] * f2[J] * f3[K - 1]);
-    p2r1 = p2r1 + cj * ((double)(J - 1) * f1[J - 1] * f2[I] * f3[K]);
-    p2r2 = p2r2 + cj * ((double)(I - 1) * f1[J] * f2[I - 1] * f3[K]);
-    p2c = p2c + cj * ((double)(K - 1) * f1[J] * f2[I] * f3[K - 1]);
+  for (int i = 0; i <= DMS_DEG; ++i) {
+#pragma unroll
+    for (int k = 0; k <= DMS_DEG - i; ++k) {
+      if (L > 1 && (i * (2 * DMS_DEG + 3 - i) / 2 + k) % L != part) continue;
+      double q = 0.0, dq = 0.0;
+#pragma unroll
+      for (int m = DMS_DEG - i - k; m >= 0; --m) {
+        const int j = dms_term(i, k, m);
+        dq = fma(dq, x3, q);
+        q = fma(q, x3, j == 0 ? 0.0 : pes[PES_DMSC + j]);
+      }
+      const double a = f1[i + 1] * f2[k + 1], b = f1[k + 1] * f2[i + 1];
+      P1 = fma(a, q, P1);
+      P2 = fma(b, q, P2);
+      p1c = fma(a, dq, p1c);
+      p2c = fma(b, dq, p2c);
+      p1r1 = fma((double)i * f1[i] * f2[k + 1], q, p1r1);
+      p1r2 = fma((double)k * f1[i + 1] * f2[k], q, p1r2);
+      p2r1 = fma((double)k * f1[k] * f2[i + 1], q, p2r1);
+      p2r2 = fma((double)i * f1[k + 1] * f2[i], q, p2r2);
+    }
   }
   if (L > 1) {
     double v[8] = {P1, P2, p1r1, p1r2, p1c, p2r1, p2r2, p2c};
