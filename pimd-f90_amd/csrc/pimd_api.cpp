@@ -257,9 +257,11 @@ void apply_ttm_params(pimd_ctx *x) {
   for (int i = 0; i < 4; ++i) x->polfac[i] = pf[i];
   for (int i = 0; i < 4; ++i)
     for (int j = 0; j < 4; ++j) {
-      c.apolCC[i][j] = aCC * pf[i] * pf[j];
+      // the same bits from either site of a pair
+      const double lo = pf[std::min(i, j)], hi = pf[std::max(i, j)];
+      c.apolCC[i][j] = aCC * lo * hi;
       c.raCC[i][j] = std::pow(c.apolCC[i][j], 1.0 / 3.0);
-      c.apolDD[i][j] = aDD * pf[i] * pf[j];
+      c.apolDD[i][j] = aDD * lo * hi;
       c.apol3DD[i][j] = c.apolDD[i][j];
     }
   c.same_a = std::fabs(aCC - aDD) < 1e-12;

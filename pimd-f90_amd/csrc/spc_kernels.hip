@@ -221,7 +221,7 @@ __global__ __launch_bounds__(256) void k_spc_pair(const Rep *__restrict__ reps, 
   double ph[4] = {0, 0, 0, 0}, ef[4][3] = {{0}}, dro[3] = {0, 0, 0};
   // the energy and virial terms of a pair are the same from either
   // molecule: every lane adds them for all its pairs, halved at the end
-  double uvdw = 0.0, vt[9] = {0};
+  double uvdw = 0.0, vt[6] = {0};
   const int nf = valid ? nbrc[grp] : 0, nn = valid ? nbrn[grp] : 0;
   const int *list = nbr + (size_t)grp * c.nbr_cap;
   auto visit = [&](const int j) {
@@ -238,8 +238,7 @@ __global__ __launch_bounds__(256) void k_spc_pair(const Rep *__restrict__ reps, 
                          (double)(fsc * (R)r[2])};
     for (int k = 0; k < 3; ++k) dro[k] += d[k];
     uvdw += (double)uij;
-    for (int col = 0; col < 3; ++col)
-      for (int row = 0; row < 3; ++row) vt[col * 3 + row] += d[col] * r[row];
+    sym_add(vt, d, r);
 #pragma unroll
     for (int sa = 1; sa < 4; ++sa) {
 #pragma unroll
@@ -248,7 +247,7 @@ __global__ __launch_bounds__(256) void k_spc_pair(const Rep *__restrict__ reps, 
         minimg(c, v[0], v[1], v[2]);
         const double d2 = norm2_exact(v[0], v[1], v[2]);
         const R vr[3] = {(R)v[0], (R)v[1], (R)v[2]};
-        const Smear<R> sm = smear_base<R>(c, (R)d2);
+        const Smear<R> sm = smear_base<false, R>(c, (R)d2);
         const R ts0 = sm.er * sm.dri;
         const R ts1 = (ts0 + (R)c.cts1 * sm.expon) * sm.drsqi;
         const R qb = (R)B[sb].q;
@@ -258,8 +257,7 @@ __global__ __launch_bounds__(256) void k_spc_pair(const Rep *__restrict__ reps, 
           const R qa = (R)A[sa].q;
           double dd[3];
           for (int k = 0; k < 3; ++k) dd[k] = (double)(-(ts1 * qa * qb * vr[k]));
-          for (int col = 0; col < 3; ++col)
-            for (int row = 0; row < 3; ++row) vt[col * 3 + row] += dd[col] * v[row];
+          sym_add(vt, dd, v);
         }
       }
     }
@@ -272,7 +270,7 @@ __global__ __launch_bounds__(256) void k_spc_pair(const Rep *__restrict__ reps, 
     for (int k = 0; k < 3; ++k) ef[t][k] = group_sum<G>(ef[t][k]);
   for (int k = 0; k < 3; ++k) dro[k] = group_sum<G>(dro[k]);
   uvdw = group_sum<G>(uvdw);
-  for (int i = 0; i < 9; ++i) vt[i] = group_sum<G>(vt[i]);
+  for (int i = 0; i < 6; ++i) vt[i] = group_sum<G>(vt[i]);
   if (valid && lane == 0) {
     const size_t base = ((size_t)bb * N + a) * 4;
     for (int t = 1; t < 4; ++t) {
@@ -280,10 +278,10 @@ __global__ __launch_bounds__(256) void k_spc_pair(const Rep *__restrict__ reps, 
       for (int k = 0; k < 3; ++k) Efq[(base + t) * 3 + k] += ef[t][k];
     }
     for (int k = 0; k < 3; ++k) dR[base * 3 + k] += dro[k];
-    for (int i = 0; i < 9; ++i) vt[i] *= 0.5;
+    for (int i = 0; i < 6; ++i) vt[i] *= 0.5;
     double *tl = tally + ((size_t)bb * N + a) * T_COUNT;
     tl[T_UVDW] += 0.5 * uvdw;
-    vadd9(tl + T_VIRT, vt);
+    vadd_sym(tl + T_VIRT, vt);
   }
 }
 

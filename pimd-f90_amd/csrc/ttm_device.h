@@ -254,23 +254,85 @@ __device__ inline bool sor_test(const SysConst &c, const double *__restrict__ di
   return !(conv || last);
 }
 
+// The outer product of parallel vectors, a symmetric matrix: xx, xy, xz, yy,
+// yz, zz; and such a sum onto a 3 x 3 one.
+__device__ __forceinline__ void sym_add(double (&t)[6], const double a[3], const double b[3]) {
+  t[0] += a[0] * b[0];
+  t[1] += a[0] * b[1];
+  t[2] += a[0] * b[2];
+  t[3] += a[1] * b[1];
+  t[4] += a[1] * b[2];
+  t[5] += a[2] * b[2];
+}
+__device__ __forceinline__ void vadd_sym(double *t, const double (&v)[6]) {
+  t[0] += v[0];
+  t[1] += v[1];
+  t[2] += v[2];
+  t[3] += v[1];
+  t[4] += v[3];
+  t[5] += v[4];
+  t[6] += v[2];
+  t[7] += v[4];
+  t[8] += v[5];
+}
+
 // x*x + y*y + z*z rounded exactly as the reference (no fused multiply-add), so
 // cut-off tests (r^2 < Rc^2, r^2 < 25) decide identically.
 __device__ __forceinline__ double norm2_exact(double x, double y, double z) {
   return __dadd_rn(__dadd_rn(__dmul_rn(x, x), __dmul_rn(y, y)), __dmul_rn(z, z));
 }
 
+// Elementary functions of the pair terms in FP64, without the range checks and
+// correctly rounded divisions of the library's: about 1 ulp over the arguments
+// of the pair terms (distances, and exponents between -700 and 0).
+// 1/sqrt(x), x > 0: the hardware estimate y (relative error e/2 with
+// e = 1 - x y^2, below 2^-20) corrected to third order.
+__device__ __forceinline__ double rsqrt_fast(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+// sqrt(x) from y = 1/sqrt(x), rounded correctly but for rare ties: exponents
+// such as E r and a r^3 multiply its error.
+__device__ __forceinline__ double sqrt_from(double x, double y) {
+  const double d = x * y;
+  return fma(fma(-d, d, x), 0.5 * y, d);
+}
+__device__ __forceinline__ double rcp_fast(double x) {
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  return fma(y, fma(e, e, e), y);
+}
+// e^x = 2^n e^r, |r| <= ln 2 / 2; e^r by its interpolation polynomial of
+// degree 11 at the Chebyshev nodes of that interval (relative error 1.7e-17).
+__device__ __forceinline__ double exp_fast(double x) {
+  const double n = __builtin_rint(x * 1.44269504088896340736);
+  const double r = fma(-n, 2.3190468138462996e-17, fma(-n, 0.69314718055994528623, x));
+  double p = fma(r, 2.5110049204818658e-08, 2.763265472252779e-07);
+  p = fma(r, p, 2.755724088722987e-06);
+  p = fma(r, p, 2.4801485441561313e-05);
+  p = fma(r, p, 0.00019841269890076403);
+  p = fma(r, p, 0.0013888888952352863);
+  p = fma(r, p, 0.008333333333319589);
+  p = fma(r, p, 0.04166666666648795);
+  p = fma(r, p, 0.1666666666666668);
+  p = fma(r, p, 0.5000000000000019);
+  p = fma(r, p, 1.0);
+  p = fma(r, p, 1.0);
+  return __builtin_amdgcn_ldexp(p, (int)n);
+}
+
 // Elementary functions of the compute type R.  FP64 is the reference's
-// arithmetic; FP32 (the mixed-precision pair terms) uses the hardware
-// square root, reciprocal and the ocml exp / log.
+// arithmetic to about 1 ulp; FP32 (the mixed-precision pair terms) uses the
+// hardware square root, reciprocal and the ocml exp / log.
 template <typename R>
 struct RM;
 template <>
 struct RM<double> {
-  static __device__ __forceinline__ double sqrt_(double x) { return sqrt(x); }
-  static __device__ __forceinline__ double rcp(double x) { return 1.0 / x; }
-  static __device__ __forceinline__ double div(double a, double b) { return a / b; }
-  static __device__ __forceinline__ double exp_(double x) { return exp(x); }
+  static __device__ __forceinline__ double sqrt_(double x) { return sqrt_from(x, rsqrt_fast(x)); }
+  static __device__ __forceinline__ double rcp(double x) { return rcp_fast(x); }
+  static __device__ __forceinline__ double div(double a, double b) { return a * rcp_fast(b); }
+  static __device__ __forceinline__ double exp_(double x) { return exp_fast(x); }
   static __device__ __forceinline__ double log_(double x) { return log(x); }
   static __device__ __forceinline__ double abs_(double x) { return fabs(x); }
 };
@@ -304,9 +366,11 @@ __device__ __forceinline__ R erfc_as(R x, R expmx2) {
 
 // Regularised upper incomplete gamma Q(2/3, x) with the reference's series /
 // continued-fraction split, tolerance and iteration caps (math.f90:188-285).
+// pre = x^(2/3) e^-x / Gamma(2/3), which the caller has from factors it forms
+// anyway.
 template <typename R>
-__device__ inline R gammq23(R x) {
-  const R a = (R)(2.0 / 3.0), gln = (R)0.303150275147547, EPS = (R)3e-7, FPMIN = (R)1e-30;
+__device__ inline R gammq23(R x, R pre) {
+  const R a = (R)(2.0 / 3.0), EPS = (R)3e-7, FPMIN = (R)1e-30;
   if (x < a + (R)1.0) {
     if (x <= (R)0.0) return (R)1.0;
     R ap = a, sum = RM<R>::rcp(a), del = sum;
@@ -316,7 +380,7 @@ __device__ inline R gammq23(R x) {
       sum = sum + del;
       if (RM<R>::abs_(del) < RM<R>::abs_(sum) * EPS) break;
     }
-    return (R)1.0 - sum * RM<R>::exp_(-x + a * RM<R>::log_(x) - gln);
+    return (R)1.0 - sum * pre;
   }
   R b = x + (R)1.0 - a, cc = RM<R>::rcp(FPMIN), d = RM<R>::rcp(b), h = d;
   for (int i = 1; i <= 100; ++i) {
@@ -331,7 +395,45 @@ __device__ inline R gammq23(R x) {
     h = h * del;
     if (RM<R>::abs_(del - (R)1.0) < EPS) break;
   }
-  return RM<R>::exp_(-x + a * RM<R>::log_(x) - gln) * h;
+  return pre * h;
+}
+// The same sums in FP64 without divisions in the loops.  Series: the terms'
+// denominators 2/3 + n are constants.  Continued fraction: its n-th convergent
+// as a quotient N_n / D_n of the three-term recurrences; the step test
+// |del - 1| < EPS is |N_n D_(n-1) - N_(n-1) D_n| < EPS N_(n-1) D_n, whose left
+// side is the product of i (i - 2/3) up to n.  Stops at the same term.  (N, D
+// and that product stay below 1e60 for the at most 30 terms x >= 5/3 takes.)
+template <>
+__device__ inline double gammq23<double>(double x, double pre) {
+  const double a = 2.0 / 3.0, EPS = 3e-7;
+  if (x < a + 1.0) {
+    if (x <= 0.0) return 1.0;
+    double sum = 1.5, del = 1.5;
+#pragma unroll
+    for (int n = 1; n <= 24; ++n) {
+      del *= x * (3.0 / (3.0 * n + 2.0));
+      sum += del;
+      if (del < sum * EPS) break;
+    }
+    return fma(-sum, pre, 1.0);
+  }
+  double b = x + (1.0 - a), Np = 0.0, Dp = 1.0, N = 1.0, D = b, prod = 1.0;
+  double c = 1.0 - a, dc = 3.0 - a;  // i (i - a) and its next difference
+#pragma unroll 4
+  for (int i = 1; i <= 100; ++i) {
+    b += 2.0;
+    const double Nn = fma(b, N, -c * Np), Dn = fma(b, D, -c * Dp);
+    prod *= c;
+    const bool done = prod < EPS * (N * Dn);
+    Np = N;
+    N = Nn;
+    Dp = D;
+    D = Dn;
+    if (done) break;
+    c += dc;
+    dc += 2.0;
+  }
+  return pre * (N * rcp_fast(D));
 }
 
 // Screened Coulomb derivatives shared by PBCsmear01/2/3 (smear.f90:2-107):
@@ -342,11 +444,16 @@ struct Smear {
   R dd, dri, drsqi, expon, er;
 };
 
-template <typename R>
+template <bool THOLE, typename R>
 __device__ __forceinline__ Smear<R> smear_base(const SysConst &c, R drsq) {
   Smear<R> s;
-  s.dd = RM<R>::sqrt_(drsq);
-  s.dri = RM<R>::rcp(s.dd);
+  if constexpr (std::is_same_v<R, double>) {
+    s.dri = rsqrt_fast(drsq);
+    s.dd = THOLE ? sqrt_from(drsq, s.dri) : drsq * s.dri;
+  } else {
+    s.dd = RM<R>::sqrt_(drsq);
+    s.dri = RM<R>::rcp(s.dd);
+  }
   s.drsqi = s.dri * s.dri;
   s.expon = RM<R>::exp_(-((R)c.a2 * drsq));
   s.er = erfc_as<R>((R)c.aewald * s.dd, s.expon);
@@ -358,7 +465,7 @@ __device__ __forceinline__ Smear<R> smear_base(const SysConst &c, R drsq) {
 // the r^2 < 25 branch cannot be taken.
 template <bool THOLE = true, typename R>
 __device__ __forceinline__ void smear01(const SysConst &c, R drsq, R apol, R ra, R &ts0, R &ts1) {
-  Smear<R> s = smear_base<R>(c, drsq);
+  Smear<R> s = smear_base<THOLE, R>(c, drsq);
   R t0 = s.er * s.dri;
   R t1 = (t0 + (R)c.cts1 * s.expon) * s.drsqi;
   if (THOLE && drsq < (R)25.0) {
@@ -367,7 +474,15 @@ __device__ __forceinline__ void smear01(const SysConst &c, R drsq, R apol, R ra,
     R ch1 = (R)-1.0 * s.dri * s.drsqi;
     R sr1 = ((R)1.0 - exp1) * s.dri * s.drsqi;
     t1 = t1 + ch1 + sr1;
-    t0 = t0 - exp1 * s.dri + ra * (R)1.3541179394264 * gammq23<R>(rA3);
+    // x^(2/3) e^-x / Gamma(2/3) at x = rA3 (gln = 0.303150275147547,
+    // math.f90:188-285): from e^-x and ra = apol^(1/3); in FP32 by its
+    // logarithm, whose rounding is the smaller
+    R pre;
+    if constexpr (std::is_same_v<R, float>)
+      pre = RM<R>::exp_(-rA3 + (R)(2.0 / 3.0) * RM<R>::log_(rA3) - (R)0.303150275147547);
+    else
+      pre = exp1 * (drsq * (ra * ra)) * (R)0.738488111621631;
+    t0 = t0 - exp1 * s.dri + ra * (R)1.3541179394264 * gammq23<R>(rA3, pre);
   }
   ts0 = t0;
   ts1 = t1;
@@ -377,7 +492,7 @@ __device__ __forceinline__ void smear01(const SysConst &c, R drsq, R apol, R ra,
 // dipole-dipole field tensors.
 template <bool THOLE = true, typename R>
 __device__ __forceinline__ void smear2(const SysConst &c, R drsq, R apol, R &ts1, R &ts2) {
-  Smear<R> s = smear_base<R>(c, drsq);
+  Smear<R> s = smear_base<THOLE, R>(c, drsq);
   R t1 = (s.er * s.dri + (R)c.cts1 * s.expon) * s.drsqi;
   R t2 = (t1 + (R)c.cts2 * s.expon) * s.drsqi;
   if (THOLE && drsq < (R)25.0) {
@@ -396,7 +511,7 @@ __device__ __forceinline__ void smear2(const SysConst &c, R drsq, R apol, R &ts1
 // PBCsmear3 (smear.f90:71-107): ts1, ts2, ts3 for the dipole-dipole forces.
 template <bool THOLE = true, typename R>
 __device__ __forceinline__ void smear3(const SysConst &c, R drsq, R apol, R &ts1, R &ts2, R &ts3) {
-  Smear<R> s = smear_base<R>(c, drsq);
+  Smear<R> s = smear_base<THOLE, R>(c, drsq);
   R t1 = (s.er * s.dri + (R)c.cts1 * s.expon) * s.drsqi;
   R t2 = (t1 + (R)c.cts2 * s.expon) * s.drsqi;
   R t3 = (t2 + (R)c.cts3 * s.expon) * s.drsqi;

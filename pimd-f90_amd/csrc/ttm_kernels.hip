@@ -602,6 +602,7 @@ __global__ __launch_bounds__(256) void k_neighbors_cells(const Rep *__restrict__
 template <int MODEL, int G, typename R, bool LDS = false>
 __global__ __launch_bounds__(256) void k_pair_qq(const Rep *__restrict__ reps, BlockMap bm) {
   constexpr int SA0 = MODEL == 2 ? 0 : 1;  // TTM3-F: O carries neither charge nor dipole
+  constexpr bool SITE_ARM = sizeof(R) == 8;
   // sites of j: unrolled in the FP32 form (more independent work per lane
   // at the same occupancy), one at a time in the FP64 form (fewer live
   // registers: two waves per SIMD instead of one)
@@ -644,12 +645,11 @@ __global__ __launch_bounds__(256) void k_pair_qq(const Rep *__restrict__ reps, B
   // halved at the end (no branch on which molecule is the lower one).  The
   // centroid virial's Rc(a, site) . F part is formed once per site at the end
   // from the site's field: its pair forces are -q(a, site) times the field terms.
-  double uvdw = 0.0, vc = 0.0, vt[9] = {0};
+  double uvdw = 0.0, vc = 0.0, vt[6] = {0};
   const int nf = valid ? nbrc[grp] : 0, nn = valid ? nbrn[grp] : 0;
   const int *list = nbr + (size_t)grp * c.nbr_cap;
   auto visit = [&](const int j, auto thole_tag) {
     constexpr bool THOLE = decltype(thole_tag)::value;
-    const bool lo = a < j;
     const Site B0 = bead_sites[j * 4];
     // vdW between oxygens
     double r[3] = {A[0].x - B0.x, A[0].y - B0.y, A[0].z - B0.z};
@@ -673,8 +673,7 @@ __global__ __launch_bounds__(256) void k_pair_qq(const Rep *__restrict__ reps, B
       minimg(c, cx, cy, cz);
       vc += cx * d[0] + cy * d[1] + cz * d[2];
     }
-    for (int col = 0; col < 3; ++col)
-      for (int row = 0; row < 3; ++row) vt[col * 3 + row] += d[col] * r[row];
+    sym_add(vt, d, r);
     // O-O image shift of the reference's charge loop, Rij - R(iO) + R(jO)
     // (pot_ttm.f90:193); it enters the centroid virial of the lower molecule.
     const double s0[3] = {r[0] - A[0].x + B0.x, r[1] - A[0].y + B0.y, r[2] - A[0].z + B0.z};
@@ -685,9 +684,11 @@ __global__ __launch_bounds__(256) void k_pair_qq(const Rep *__restrict__ reps, B
     for (int sb = 1; sb < 4; ++sb) {
       const Site Bs = bead_sites[j * 4 + sb];
       const R qb = (R)Bs.q;
-      // the pair-side part of the centroid virial's lever arm
-      const double w[3] = {s0[0] - Rcs[(j * 4 + sb) * 3 + 0], s0[1] - Rcs[(j * 4 + sb) * 3 + 1],
-                           s0[2] - Rcs[(j * 4 + sb) * 3 + 2]};
+      // the pair-side part of the centroid virial's lever arm; in FP64 only
+      // the image shift, the rest at the end
+      double w[3] = {s0[0], s0[1], s0[2]};
+      if constexpr (!SITE_ARM)
+        for (int k = 0; k < 3; ++k) w[k] -= Rcs[(j * 4 + sb) * 3 + k];
 #pragma unroll
       for (int sa = SA0; sa < 4; ++sa) {
         // site-site minimum image, oriented from a to b (pot_ttm.f90:206-207)
@@ -696,8 +697,8 @@ __global__ __launch_bounds__(256) void k_pair_qq(const Rep *__restrict__ reps, B
         const double d2 = norm2_exact(v[0], v[1], v[2]);
         const R vr[3] = {(R)v[0], (R)v[1], (R)v[2]};
         R ts0, ts1;
-        smear01<THOLE>(c, (R)d2, (R)(lo ? c.apolCC[sa][sb] : c.apolCC[sb][sa]),
-                       (R)(lo ? c.raCC[sa][sb] : c.raCC[sb][sa]), ts0, ts1);
+        smear01<THOLE>(c, (R)d2, (R)c.apolCC[sa][sb],
+                       (R)c.raCC[sa][sb], ts0, ts1);
         if (sa > 0) ph[sa] += (double)(ts0 * qb);
         for (int k = 0; k < 3; ++k) ef[sa][k] += (double)(ts1 * qb * vr[k]);
         if (sa > 0) {
@@ -705,8 +706,7 @@ __global__ __launch_bounds__(256) void k_pair_qq(const Rep *__restrict__ reps, B
           double dd[3];
           for (int k = 0; k < 3; ++k) dd[k] = (double)(-(ts1 * qa * qb * vr[k]));
           vc += w[0] * dd[0] + w[1] * dd[1] + w[2] * dd[2];
-          for (int col = 0; col < 3; ++col)
-            for (int row = 0; row < 3; ++row) vt[col * 3 + row] += dd[col] * v[row];
+          sym_add(vt, dd, v);
         }
       }
     }
@@ -719,7 +719,7 @@ __global__ __launch_bounds__(256) void k_pair_qq(const Rep *__restrict__ reps, B
   for (int k = 0; k < 3; ++k) dro[k] = group_sum<G>(dro[k]);
   uvdw = group_sum<G>(uvdw);
   vc = group_sum<G>(vc);
-  for (int i = 0; i < 9; ++i) vt[i] = group_sum<G>(vt[i]);
+  for (int i = 0; i < 6; ++i) vt[i] = group_sum<G>(vt[i]);
   if (valid && lane == 0) {
     const size_t base = ((size_t)b * N + a) * 4;
     for (int t = 1; t < 4; ++t) phi[base + t] += ph[t];
@@ -730,13 +730,13 @@ __global__ __launch_bounds__(256) void k_pair_qq(const Rep *__restrict__ reps, B
     // -q(a, site) times its field terms
     for (int t = 1; t < 4; ++t) {
       const double *rc = Rcs + (a * 4 + t) * 3;
-      vc -= A[t].q * (rc[0] * ef[t][0] + rc[1] * ef[t][1] + rc[2] * ef[t][2]);
+      vc -= (SITE_ARM ? 2.0 : 1.0) * A[t].q * (rc[0] * ef[t][0] + rc[1] * ef[t][1] + rc[2] * ef[t][2]);
     }
-    for (int i = 0; i < 9; ++i) vt[i] *= 0.5;
+    for (int i = 0; i < 6; ++i) vt[i] *= 0.5;
     double *tl = tally + ((size_t)b * N + a) * T_COUNT;
     tl[T_UVDW] += 0.5 * uvdw;
     tl[T_VIRC] += 0.5 * vc;
-    vadd9(tl + T_VIRT, vt);
+    vadd_sym(tl + T_VIRT, vt);
   }
 }
 
@@ -752,15 +752,19 @@ __global__ __launch_bounds__(256) void k_pair_qq(const Rep *__restrict__ reps, B
 // feeding both sides (TTM2.1-F adds the pairs with the partner's oxygen,
 // which k_pair_qq takes from the partner's side).  Energies and virials per
 // pair are those k_pair_qq halves from its two sides, taken once.
-// FP64 form: a value v goes in as h = rint(v 2^32) (range +-2^31) and the
-// remainder v - h 2^-32, exact in FP64, as rint(. 2^64): each addition is
+// FP64 form: a value v goes in as h = rint(v 2^20) (range +-2^31) and the
+// remainder v - h 2^-20, exact in FP64, as rint(. 2^64): each addition is
 // exact to 2^-65, finer than FP64 rounding of the sums, so the result
 // matches an FP64 sum and stays smooth in the model parameters.  FP32 form:
 // one word, rint(v 2^40) (range +-2^23): its pair terms already round at
 // 1e-7 relative, far above that quantum, and one LDS atomic per value in
 // place of two.  Integer addition wraps modulo 2^64 and is associative: only
-// totals must fit.
-constexpr double QQ_HI = 4294967296.0;            // 2^32
+// totals must fit.  Bound by FP64 issue: about 80 instructions per site pair
+// beyond the 5 A radius and some 300 more inside it (the gamma function's
+// loop), 6 per partner value; 512 H2O x 32 beads 212 -> 117 us FP64 against
+// library exp, sqrt and division, divisions in the gamma function's loops and
+// f64-to-i64 conversions of the partner values; 110 -> 101 us FP32.
+constexpr double QQ_HI = 1048576.0;               // 2^20
 constexpr double QQ_LO = 18446744073709551616.0;  // 2^64
 constexpr double QQ_ONE = 1099511627776.0;        // 2^40
 template <typename R>
@@ -773,15 +777,26 @@ template <typename R>
 struct QqUnroll {
   static constexpr int v = 1;
 };
+// The integers come from FP64 addition: v + 3 2^(51-q) has rint(v 2^q) in its
+// low mantissa bits, so that its bits less the constant's are that integer.
+constexpr double qq_magic(int q) {
+  double m = 3.0;
+  for (int i = 0; i < 51 - q; ++i) m *= 2.0;
+  for (int i = 0; i < q - 51; ++i) m *= 0.5;
+  return m;
+}
+constexpr double QQ_M20 = qq_magic(20), QQ_M40 = qq_magic(40), QQ_M64 = qq_magic(64);
 template <int NW>
 __device__ __forceinline__ void qq_fix_add(unsigned long long *acc, double v) {
+  const double t = v + QQ_M20, h = t - QQ_M20, rem = v - h;
+  const long long a = __double_as_longlong(t) - __double_as_longlong(QQ_M20);
   if constexpr (NW == 2) {
-    const double h = rint(fmin(fmax(v * QQ_HI, -9.2e18), 9.2e18));
-    const double rem = fmin(fmax(v - h * (1.0 / QQ_HI), -1.0 / QQ_HI), 1.0 / QQ_HI);
-    atomicAdd(acc, (unsigned long long)(long long)h);
-    atomicAdd(acc + 1, (unsigned long long)__double2ll_rn(rem * QQ_LO));
+    const long long b = __double_as_longlong(rem + QQ_M64) - __double_as_longlong(QQ_M64);
+    atomicAdd(acc, (unsigned long long)a);
+    atomicAdd(acc + 1, (unsigned long long)b);
   } else {
-    atomicAdd(acc, (unsigned long long)__double2ll_rn(fmin(fmax(v * QQ_ONE, -9.2e18), 9.2e18)));
+    const long long b = __double_as_longlong(rem + QQ_M40) - __double_as_longlong(QQ_M40);
+    atomicAdd(acc, ((unsigned long long)a << 20) + (unsigned long long)b);
   }
 }
 template <int NW>
@@ -796,6 +811,7 @@ template <int MODEL, int G, typename R>
 __global__ __launch_bounds__(QQ_HALF_BLOCK) void k_pair_qq_half(const Rep *__restrict__ reps,
                                                                 BlockMap bm) {
   constexpr int SA0 = MODEL == 2 ? 0 : 1;  // first dipole-carrying (field-target) site type
+  constexpr bool SITE_ARM = sizeof(R) == 8;
   constexpr int OWN = QQ_HALF_BLOCK / G;  // owners per block
   constexpr int NW = QqWords<R>::n;       // words per partner value
   extern __shared__ Site lds_site[];  // [W][4] sites, then [W][QQ_NV][NW] partner sums
@@ -827,13 +843,12 @@ __global__ __launch_bounds__(QQ_HALF_BLOCK) void k_pair_qq_half(const Rep *__res
   for (int t = 0; t < 4; ++t) A[t] = lds_site[(a - i0) * 4 + t];
   const double RcO[3] = {Rcs[a * 12 + 0], Rcs[a * 12 + 1], Rcs[a * 12 + 2]};
   double ph[4] = {0, 0, 0, 0}, ef[4][3] = {{0}}, dro[3] = {0, 0, 0};
-  double uvdw = 0.0, vc = 0.0, vt[9] = {0};
+  double uvdw = 0.0, vc = 0.0, vt[6] = {0};
   const int *list = nbr + (size_t)grp * c.nbr_cap;
   // partner-side sums of molecule j: ph[1..3], then ef of sites SA0..3, then dro
   auto jslot = [&](int rj, int k) { return jacc + ((size_t)rj * QQ_NV + k) * NW; };
   auto visit = [&](const int j, auto thole_tag) {
     constexpr bool THOLE = decltype(thole_tag)::value;
-    const bool lo = a < j;
     const int rj = row(j);
     const Site B0 = lds_site[rj * 4];
     double r[3] = {A[0].x - B0.x, A[0].y - B0.y, A[0].z - B0.z};
@@ -860,14 +875,12 @@ __global__ __launch_bounds__(QQ_HALF_BLOCK) void k_pair_qq_half(const Rep *__res
       minimg(c, cx, cy, cz);
       vc += cx * d[0] + cy * d[1] + cz * d[2];
     }
-    for (int col = 0; col < 3; ++col)
-      for (int row = 0; row < 3; ++row) vt[col * 3 + row] += d[col] * r[row];
+    sym_add(vt, d, r);
     const double s0[3] = {r[0] - A[0].x + B0.x, r[1] - A[0].y + B0.y, r[2] - A[0].z + B0.z};
 #pragma unroll QqUnroll<R>::v
     for (int sb = SA0; sb < 4; ++sb) {
       const Site Bs = lds_site[rj * 4 + sb];
       const R qb = (R)Bs.q;
-      const double *rcb = Rcs + (j * 4 + sb) * 3;
       double jp = 0.0, je[3] = {0.0, 0.0, 0.0};  // the partner's site sb
 #pragma unroll
       for (int sa = SA0; sa < 4; ++sa) {
@@ -877,8 +890,8 @@ __global__ __launch_bounds__(QQ_HALF_BLOCK) void k_pair_qq_half(const Rep *__res
         const double d2 = norm2_exact(v[0], v[1], v[2]);
         const R vr[3] = {(R)v[0], (R)v[1], (R)v[2]};
         R ts0, ts1;
-        smear01<THOLE>(c, (R)d2, (R)(lo ? c.apolCC[sa][sb] : c.apolCC[sb][sa]),
-                       (R)(lo ? c.raCC[sa][sb] : c.raCC[sb][sa]), ts0, ts1);
+        smear01<THOLE>(c, (R)d2, (R)c.apolCC[sa][sb],
+                       (R)c.raCC[sa][sb], ts0, ts1);
         const R qa = (R)A[sa].q;
         // this molecule's site sa from the partner's charge, and the
         // partner's site sb from this one's (the field along -v)
@@ -892,13 +905,17 @@ __global__ __launch_bounds__(QQ_HALF_BLOCK) void k_pair_qq_half(const Rep *__res
           double dd[3];
           for (int k = 0; k < 3; ++k) dd[k] = (double)(-(ts1 * qa * qb * vr[k]));
           // the mean of the two sides' lever arms (s0 - Rc(j, sb) from this
-          // side, -s0 - Rc(a, sa) with the force reversed from the partner's)
-          const double *rca = Rcs + (a * 4 + sa) * 3;
-          double w[3];
-          for (int k = 0; k < 3; ++k) w[k] = s0[k] + 0.5 * (rca[k] - rcb[k]);
+          // side, -s0 - Rc(a, sa) with the force reversed from the partner's);
+          // in FP64 only the image shift, the sites' whole Rc . F following
+          // from their fields at the end (the FP32 form rounds the two sides'
+          // fields of a pair apart, so keeps their difference here)
+          double w[3] = {s0[0], s0[1], s0[2]};
+          if constexpr (!SITE_ARM) {
+            const double *rca = Rcs + (a * 4 + sa) * 3, *rcb = Rcs + (j * 4 + sb) * 3;
+            for (int k = 0; k < 3; ++k) w[k] += 0.5 * (rca[k] - rcb[k]);
+          }
           vc += w[0] * dd[0] + w[1] * dd[1] + w[2] * dd[2];
-          for (int col = 0; col < 3; ++col)
-            for (int row = 0; row < 3; ++row) vt[col * 3 + row] += dd[col] * v[row];
+          sym_add(vt, dd, v);
         }
       }
       if (sb > 0) qq_fix_add<NW>(jslot(rj, sb - 1), jp);
@@ -925,23 +942,23 @@ __global__ __launch_bounds__(QQ_HALF_BLOCK) void k_pair_qq_half(const Rep *__res
   for (int k = 0; k < 3; ++k) dro[k] = group_sum<G>(dro[k]);
   uvdw = group_sum<G>(uvdw);
   vc = group_sum<G>(vc);
-  for (int i = 0; i < 9; ++i) vt[i] = group_sum<G>(vt[i]);
+  for (int i = 0; i < 6; ++i) vt[i] = group_sum<G>(vt[i]);
   if (valid && lane == 0) {
     const size_t base = ((size_t)b * N + a) * 4;
     for (int t = 1; t < 4; ++t) phi[base + t] += ph[t];
     for (int t = SA0; t < 4; ++t)
       for (int k = 0; k < 3; ++k) Efq[(base + t) * 3 + k] += ef[t][k];
     for (int k = 0; k < 3; ++k) dR[base * 3 + k] += dro[k];
-    // half of Rc(a, site) . (the site's pair forces) from this side's field;
-    // the partner side's half follows in k_pair_qq_partner
+    // Rc(a, site) . (the site's pair forces) from this side's field (half of
+    // it in FP32); the partner side's follows in k_pair_qq_partner
     for (int t = 1; t < 4; ++t) {
       const double *rc = Rcs + (a * 4 + t) * 3;
-      vc -= 0.5 * A[t].q * (rc[0] * ef[t][0] + rc[1] * ef[t][1] + rc[2] * ef[t][2]);
+      vc -= (SITE_ARM ? 1.0 : 0.5) * A[t].q * (rc[0] * ef[t][0] + rc[1] * ef[t][1] + rc[2] * ef[t][2]);
     }
     double *tl = tally + ((size_t)b * N + a) * T_COUNT;
     tl[T_UVDW] += uvdw;
     tl[T_VIRC] += vc;
-    vadd9(tl + T_VIRT, vt);
+    vadd_sym(tl + T_VIRT, vt);
   }
   __syncthreads();
   // the block's exact row sums, rounded once
@@ -953,7 +970,7 @@ __global__ __launch_bounds__(QQ_HALF_BLOCK) void k_pair_qq_half(const Rep *__res
 // The partner-side sums of k_pair_qq_half: 32 lanes per molecule, lane k
 // adding value k over the blocks whose window holds the molecule, in block
 // order, onto its potential, field or oxygen gradient; the lanes then sum the
-// other half of Rc . F of the centroid virial.
+// partner side's Rc . F of the centroid virial (half of it in the mixed form).
 template <int MODEL>
 __global__ __launch_bounds__(256) void k_pair_qq_partner(const Rep *__restrict__ reps, BlockMap bm) {
   constexpr int SA0 = MODEL == 2 ? 0 : 1;
@@ -983,7 +1000,7 @@ __global__ __launch_bounds__(256) void k_pair_qq_partner(const Rep *__restrict__
     } else if (k < 3 + 3 * (4 - SA0)) {
       const int t = SA0 + (k - 3) / 3, x = (k - 3) % 3;
       Rp.b.Efq[(base + t) * 3 + x] += v;
-      if (t > 0) vc = -0.5 * Rp.b.site[base + t].q * Rp.b.Rcs[(a * 4 + t) * 3 + x] * v;
+      if (t > 0) vc = -(c.mixed ? 0.5 : 1.0) * Rp.b.site[base + t].q * Rp.b.Rcs[(a * 4 + t) * 3 + x] * v;
     } else {
       Rp.b.dR[base * 3 + (k - 3 - 3 * (4 - SA0))] += v;
     }
@@ -1755,7 +1772,6 @@ __global__ __launch_bounds__(256) void k_pair_dd(const Rep *__restrict__ reps, B
   const int *list = nbr + (size_t)grp * c.nbr_cap;
   auto visit = [&](const int j, auto thole_tag) {
     constexpr bool THOLE = decltype(thole_tag)::value;
-    const bool lo = a < j;
     const Site *Bs = site + ((size_t)b * N + j) * 4;
     double mub[ND][3];
     for (int u = 0; u < ND; ++u)
@@ -1770,7 +1786,7 @@ __global__ __launch_bounds__(256) void k_pair_dd(const Rep *__restrict__ reps, B
         minimg(c, v[0], v[1], v[2]);
         const double d2 = norm2_exact(v[0], v[1], v[2]);
         R ts1, ts2;
-        smear2<THOLE>(c, (R)d2, (R)(lo ? c.apolDD[sa][sb] : c.apolDD[sb][sa]), ts1, ts2);
+        smear2<THOLE>(c, (R)d2, (R)c.apolDD[sa][sb], ts1, ts2);
         const R vr[3] = {(R)v[0], (R)v[1], (R)v[2]};
         const R mr[3] = {(R)mub[ub][0], (R)mub[ub][1], (R)mub[ub][2]};
         R o[3];
@@ -1941,7 +1957,6 @@ __global__ __launch_bounds__(dd_block<MODEL>()) void k_pair_dd_lds(const Rep *__
   } else {
     auto visit = [&](const int j, const int at, auto thole_tag) {
       constexpr bool THOLE = decltype(thole_tag)::value;
-      const bool lo = a < j;
 #pragma unroll
       for (int ua = 0; ua < ND; ++ua) {
 #pragma unroll
@@ -1952,7 +1967,7 @@ __global__ __launch_bounds__(dd_block<MODEL>()) void k_pair_dd_lds(const Rep *__
           minimg(c, v[0], v[1], v[2]);
           const double d2 = norm2_exact(v[0], v[1], v[2]);
           R ts1, ts2;
-          smear2<THOLE>(c, (R)d2, (R)(lo ? c.apolDD[sa][sb] : c.apolDD[sb][sa]), ts1, ts2);
+          smear2<THOLE>(c, (R)d2, (R)c.apolDD[sa][sb], ts1, ts2);
           opaque(ts1);
           opaque(ts2);
           if (store) tsrow[(size_t)at * NP + ua * ND + ub] = R2{ts1, ts2};
@@ -2121,12 +2136,11 @@ __global__ __launch_bounds__(256) void k_pair_final(const Rep *__restrict__ reps
     for (int k = 0; k < 3; ++k)
       mua[t][k] = is_dip<MODEL>(t) ? bead_dip[((size_t)a * ND + (t - T0)) * 3 + k] : 0.0;
   }
-  double ph[4] = {0, 0, 0, 0}, fr[4][3] = {{0}}, vc = 0.0, vt[9] = {0};
+  double ph[4] = {0, 0, 0, 0}, fr[4][3] = {{0}}, vt[9] = {0};
   const int nf = valid ? nbrc[grp] : 0, nn = valid ? nbrn[grp] : 0;
   const int *list = nbr + (size_t)grp * c.nbr_cap;
   auto visit = [&](const int j, auto thole_tag) {
     constexpr bool THOLE = decltype(thole_tag)::value;
-    const bool lo = a < j;
     // one site of j at a time (read in the loop) against every site of a:
     // each accumulator of a site of a still takes its terms in the order
     // (j, site of j).  Unrolled except in the FP64 form of TTM2.1-F, where one
@@ -2166,7 +2180,7 @@ __global__ __launch_bounds__(256) void k_pair_final(const Rep *__restrict__ reps
         bool have_ts1 = false;
         if (da && db) {
           R t1d, t2d, t3d;
-          smear3<THOLE>(c, (R)d2, (R)(lo ? c.apol3DD[sa][sb] : c.apol3DD[sb][sa]), t1d, t2d, t3d);
+          smear3<THOLE>(c, (R)d2, (R)c.apol3DD[sa][sb], t1d, t2d, t3d);
           // di . T3(r) . dj with T3_abc = 15 r_a r_b r_c ts3 - 3 ts2 (r_a d_bc + r_b d_ac + r_c d_ab)
           const R rdi = r[0] * di[0] + r[1] * di[1] + r[2] * di[2];
           const R rdj = r[0] * dj[0] + r[1] * dj[1] + r[2] * dj[2];
@@ -2179,7 +2193,7 @@ __global__ __launch_bounds__(256) void k_pair_final(const Rep *__restrict__ reps
               ts1 = t1d;
               ts2 = t2d;
             } else {
-              smear2<THOLE>(c, (R)d2, (R)(lo ? c.apolCC[sa][sb] : c.apolCC[sb][sa]), ts1, ts2);
+              smear2<THOLE>(c, (R)d2, (R)c.apolCC[sa][sb], ts1, ts2);
             }
             have_ts1 = true;
             R o[3];
@@ -2187,7 +2201,7 @@ __global__ __launch_bounds__(256) void k_pair_final(const Rep *__restrict__ reps
             for (int k = 0; k < 3; ++k) dijr[k] += o[k];
           }
         } else if (qsq > (R)1e-9) {
-          smear2<THOLE>(c, (R)d2, (R)(lo ? c.apolCC[sa][sb] : c.apolCC[sb][sa]), ts1, ts2);
+          smear2<THOLE>(c, (R)d2, (R)c.apolCC[sa][sb], ts1, ts2);
           have_ts1 = true;
           R o[3];
           dd3_apply(r, ts1, ts2, qd, o);
@@ -2196,14 +2210,9 @@ __global__ __launch_bounds__(256) void k_pair_final(const Rep *__restrict__ reps
         if (have_ts1 && db) ph[sa] += (double)(ts1 * (r[0] * dj[0] + r[1] * dj[1] + r[2] * dj[2]));
         const double dij[3] = {(double)dijr[0], (double)dijr[1], (double)dijr[2]};
         for (int k = 0; k < 3; ++k) fr[sa][k] += dij[k];
-        if (lo) {
-          double rcv[3];
-          // Rij0 of the dipole loop is wrapped to ~0 (pot_ttm.f90:406-407,468)
-          for (int k = 0; k < 3; ++k) rcv[k] = Rcs[(a * 4 + sa) * 3 + k] - Rcs[(j * 4 + sb) * 3 + k];
-          vc += rcv[0] * dij[0] + rcv[1] * dij[1] + rcv[2] * dij[2];
-          for (int col = 0; col < 3; ++col)
-            for (int row = 0; row < 3; ++row) vt[col * 3 + row] += dij[row] * v[col];
-        }
+        // the same from either molecule: halved at the end
+        for (int col = 0; col < 3; ++col)
+          for (int row = 0; row < 3; ++row) vt[col * 3 + row] += dij[row] * v[col];
       }
     }
   };
@@ -2213,7 +2222,6 @@ __global__ __launch_bounds__(256) void k_pair_final(const Rep *__restrict__ reps
     ph[t] = group_sum<G>(ph[t]);
     for (int k = 0; k < 3; ++k) fr[t][k] = group_sum<G>(fr[t][k]);
   }
-  vc = group_sum<G>(vc);
   for (int i = 0; i < 9; ++i) vt[i] = group_sum<G>(vt[i]);
   if (valid && lane == 0) {
     const size_t base = ((size_t)b * N + a) * 4;
@@ -2221,6 +2229,12 @@ __global__ __launch_bounds__(256) void k_pair_final(const Rep *__restrict__ reps
       phi[base + t] += ph[t];
       for (int k = 0; k < 3; ++k) dR[(base + t) * 3 + k] += fr[t][k];
     }
+    // Rij0 of the dipole loop is wrapped to ~0 (pot_ttm.f90:406-407,468): the
+    // centroid virial is Rc . F summed over the sites
+    double vc = 0.0;
+    for (int t = 0; t < 4; ++t)
+      for (int k = 0; k < 3; ++k) vc += Rcs[(a * 4 + t) * 3 + k] * fr[t][k];
+    for (int i = 0; i < 9; ++i) vt[i] *= 0.5;
     double *tl = tally + ((size_t)b * N + a) * T_COUNT;
     tl[T_VIRC] += vc;
     vadd9(tl + T_VIRT, vt);
@@ -2288,12 +2302,11 @@ __global__ __launch_bounds__(QQ_HALF_BLOCK) void k_pair_final_half(const Rep *__
     for (int k = 0; k < 3; ++k)
       mua[t][k] = is_dip<MODEL>(t) ? lds_dip[((a - i0) * ND + (t - T0)) * 3 + k] : 0.0;
   }
-  double ph[4] = {0, 0, 0, 0}, fr[4][3] = {{0}}, vc = 0.0, vt[9] = {0};
+  double ph[4] = {0, 0, 0, 0}, fr[4][3] = {{0}}, vt[9] = {0};
   const int *list = nbr + (size_t)grp * c.nbr_cap;
   auto jslot = [&](int rj, int k) { return jacc + ((size_t)rj * FIN_NV + k) * NW; };
   auto visit = [&](const int j, auto thole_tag) {
     constexpr bool THOLE = decltype(thole_tag)::value;
-    const bool lo = a < j;
     const int rj = row(j);
 #pragma unroll 1
     for (int sb = SB0; sb < 4; ++sb) {
@@ -2325,7 +2338,7 @@ __global__ __launch_bounds__(QQ_HALF_BLOCK) void k_pair_final_half(const Rep *__
         bool have_ts1 = false;
         if (da && db) {
           R t1d, t2d, t3d;
-          smear3<THOLE>(c, (R)d2, (R)(lo ? c.apol3DD[sa][sb] : c.apol3DD[sb][sa]), t1d, t2d, t3d);
+          smear3<THOLE>(c, (R)d2, (R)c.apol3DD[sa][sb], t1d, t2d, t3d);
           const R rdi = r[0] * di[0] + r[1] * di[1] + r[2] * di[2];
           const R rdj = r[0] * dj[0] + r[1] * dj[1] + r[2] * dj[2];
           const R didj = di[0] * dj[0] + di[1] * dj[1] + di[2] * dj[2];
@@ -2337,7 +2350,7 @@ __global__ __launch_bounds__(QQ_HALF_BLOCK) void k_pair_final_half(const Rep *__
               ts1 = t1d;
               ts2 = t2d;
             } else {
-              smear2<THOLE>(c, (R)d2, (R)(lo ? c.apolCC[sa][sb] : c.apolCC[sb][sa]), ts1, ts2);
+              smear2<THOLE>(c, (R)d2, (R)c.apolCC[sa][sb], ts1, ts2);
             }
             have_ts1 = true;
             R o[3];
@@ -2345,7 +2358,7 @@ __global__ __launch_bounds__(QQ_HALF_BLOCK) void k_pair_final_half(const Rep *__
             for (int k = 0; k < 3; ++k) dijr[k] += o[k];
           }
         } else if (qsq > (R)1e-9) {
-          smear2<THOLE>(c, (R)d2, (R)(lo ? c.apolCC[sa][sb] : c.apolCC[sb][sa]), ts1, ts2);
+          smear2<THOLE>(c, (R)d2, (R)c.apolCC[sa][sb], ts1, ts2);
           have_ts1 = true;
           R o[3];
           dd3_apply(r, ts1, ts2, qd, o);
@@ -2360,10 +2373,6 @@ __global__ __launch_bounds__(QQ_HALF_BLOCK) void k_pair_final_half(const Rep *__
           fr[sa][k] += dij[k];
           jf[k] -= dij[k];
         }
-        // Rij0 of the dipole loop is wrapped to ~0 (pot_ttm.f90:406-407,468)
-        double rcv[3];
-        for (int k = 0; k < 3; ++k) rcv[k] = Rcs[(a * 4 + sa) * 3 + k] - Rcs[(j * 4 + sb) * 3 + k];
-        vc += rcv[0] * dij[0] + rcv[1] * dij[1] + rcv[2] * dij[2];
         for (int col = 0; col < 3; ++col)
           for (int rw = 0; rw < 3; ++rw) vt[col * 3 + rw] += dij[rw] * rd[col];
       }
@@ -2385,7 +2394,6 @@ __global__ __launch_bounds__(QQ_HALF_BLOCK) void k_pair_final_half(const Rep *__
     ph[t] = group_sum<G>(ph[t]);
     for (int k = 0; k < 3; ++k) fr[t][k] = group_sum<G>(fr[t][k]);
   }
-  vc = group_sum<G>(vc);
   for (int i = 0; i < 9; ++i) vt[i] = group_sum<G>(vt[i]);
   if (valid && lane == 0) {
     const size_t base = ((size_t)b * N + a) * 4;
@@ -2393,6 +2401,12 @@ __global__ __launch_bounds__(QQ_HALF_BLOCK) void k_pair_final_half(const Rep *__
       phi[base + t] += ph[t];
       for (int k = 0; k < 3; ++k) dR[(base + t) * 3 + k] += fr[t][k];
     }
+    // Rij0 of the dipole loop is wrapped to ~0 (pot_ttm.f90:406-407,468): the
+    // centroid virial is Rc . F summed over the sites, the partner side's in
+    // k_pair_final_partner
+    double vc = 0.0;
+    for (int t = SB0; t < 4; ++t)
+      for (int k = 0; k < 3; ++k) vc += Rcs[(a * 4 + t) * 3 + k] * fr[t][k];
     double *tl = tally + ((size_t)b * N + a) * T_COUNT;
     tl[T_VIRC] += vc;
     vadd9(tl + T_VIRT, vt);
@@ -2407,7 +2421,8 @@ __global__ __launch_bounds__(QQ_HALF_BLOCK) void k_pair_final_half(const Rep *__
 }
 
 // The partner-side sums of k_pair_final_half (as k_pair_qq_partner): lane k
-// of a molecule's 32 adds value k over the blocks, in block order.
+// of a molecule's 32 adds value k over the blocks, in block order; the lanes then
+// sum the partner side's Rc . F of the centroid virial.
 template <int MODEL>
 __global__ __launch_bounds__(256) void k_pair_final_partner(const Rep *__restrict__ reps,
                                                             BlockMap bm) {
@@ -2417,22 +2432,31 @@ __global__ __launch_bounds__(256) void k_pair_final_partner(const Rep *__restric
   const int N = c.N;
   const long m = ((long)bk.x * blockDim.x + threadIdx.x) / 32;
   const int k = threadIdx.x % 32;
+  const bool valid = m < (long)c.P * N;  // alike over the 32 lanes of a molecule
   // TTM3-F: no values for the oxygen (slots 0 and 4-6)
-  const bool used = k < FIN_NV && !(MODEL == 3 && (k == 0 || (k >= 4 && k < 7)));
-  if (m >= (long)c.P * N || !used) return;
-  const int b = (int)(m / N), a = (int)(m % N);
+  const bool used = valid && k < FIN_NV && !(MODEL == 3 && (k == 0 || (k >= 4 && k < 7)));
+  const int b = valid ? (int)(m / N) : 0, a = valid ? (int)(m % N) : 0;
   const int G = half_lanes(c.g_fin), own = QQ_HALF_BLOCK / G;
   const int nblk = qq_half_blocks(N, G), W = qq_half_rows(N, G);
-  const double *slab = Rp.b.qqslab + (size_t)b * nblk * W * QQ_NV + k;
-  double v = 0.0;
-  for (int q = 0; q < nblk; ++q) {
-    int r = a - q * own;
-    r += r < 0 ? N : 0;
-    if (r < W) v += slab[((size_t)q * W + r) * QQ_NV];
+  double vc = 0.0;
+  if (used) {
+    const double *slab = Rp.b.qqslab + (size_t)b * nblk * W * QQ_NV + k;
+    double v = 0.0;
+    for (int q = 0; q < nblk; ++q) {
+      int r = a - q * own;
+      r += r < 0 ? N : 0;
+      if (r < W) v += slab[((size_t)q * W + r) * QQ_NV];
+    }
+    const size_t base = ((size_t)b * N + a) * 4;
+    if (k < 4) {
+      Rp.b.phi[base + k] += v;
+    } else {
+      Rp.b.dR[(base + (k - 4) / 3) * 3 + (k - 4) % 3] += v;
+      vc = Rp.b.Rcs[a * 12 + (k - 4)] * v;
+    }
   }
-  const size_t base = ((size_t)b * N + a) * 4;
-  if (k < 4) Rp.b.phi[base + k] += v;
-  else Rp.b.dR[(base + (k - 4) / 3) * 3 + (k - 4) % 3] += v;
+  vc = group_sum<32>(vc);
+  if (valid && k == 0) Rp.b.tally[((size_t)b * N + a) * T_COUNT + T_VIRC] += vc;
 }
 
 // Reciprocal-space virial (ewald.f90:194-224), partial sums per block of k:
