@@ -162,6 +162,9 @@ __global__ __launch_bounds__(64 * DB_W) void k_dense_build(const Rep *__restrict
   const size_t DS = dense_stride(c);
   dptr<double> m = Rp.b.dmat + (size_t)b * 3 * M * DS;
   const double v[3][3] = {{K[0], K[1], K[4]}, {K[1], K[2], K[5]}, {K[4], K[5], K[3]}};
+  // the rows' padding, read with the last column (times a zero)
+  if (j == M - 1 && DS != (size_t)3 * M)
+    for (int a = 0; a < 3; ++a) m[(size_t)(3 * i + a) * DS + 3 * M] = 0.0;
 #pragma unroll
   for (int a = 0; a < 3; ++a)
 #pragma unroll
