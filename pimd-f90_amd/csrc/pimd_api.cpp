@@ -412,8 +412,9 @@ int env_int(const char *name, int dflt, int lo, int hi) {
 // Host-side tables of a system: k-vectors, kz-columns and their segments.
 struct HostTables {
   std::vector<double4> kv;
-  std::vector<int4> kh, cols, segs;
-  std::vector<int> colk, segk;
+  std::vector<int4> kh, cols;
+  std::vector<int> colk, sftask;
+  std::vector<ColRec> colrec;
   std::vector<int4> dcol;  // dense dipole matrix: kz-columns by (kx, ky)
   std::vector<int> dkx;    // first column of each kx plane
   std::vector<double> dcoef;
@@ -471,13 +472,14 @@ void plan_system(pimd_ctx *x, HostTables &t) {
   }
   x->dcoef_n = t.dcoef.size();
   for (int h = 1; h <= c.hmax + 1; ++h) t.dkx[h] = std::max(t.dkx[h], t.dkx[h - 1]);
-  // longest columns first: lanes and column groups that run together get
-  // similar trip counts
+  // the columns that reach farthest along kz first: the 16 columns of a
+  // matrix tile get similar reaches
   {
+    auto reach = [](int4 cl) { return std::max(std::abs(cl.z), std::abs(cl.z + cl.w - 1)); };
     std::vector<int> order(cols.size());
     for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
     std::stable_sort(order.begin(), order.end(),
-                     [&](int a, int b2) { return cols[a].w > cols[b2].w; });
+                     [&](int a, int b2) { return reach(cols[a]) > reach(cols[b2]); });
     std::vector<int4> cs(cols.size());
     std::vector<int> ck(colk.size());
     for (size_t i = 0; i < order.size(); ++i) {
@@ -488,42 +490,10 @@ void plan_system(pimd_ctx *x, HostTables &t) {
     colk.swap(ck);
   }
   c.ncol = (int)cols.size();
-  c.kzmax = 0;
-  for (auto &cl : cols) c.kzmax = std::max(c.kzmax, cl.w);
-  // segments for the structure-factor kernel: the columns cut into pieces of
-  // at most segmax consecutive kz, longest first
-  std::vector<int4> &segs = t.segs;
-  std::vector<int> &segk = t.segk;
-  segs.clear();
-  segk.clear();
-  {
-    // 4 kz per segment: twice the lanes of 8 for the same sites (512 H2O x 32
-    // beads: 1.273 -> 1.251 ms per mixed step, 1.592 -> 1.586 FP64; the
-    // 32-water, 32-bead Rc 4.9 A system gains more)
-    const int seg = env_int("PIMD_SFAC_SEG", 4, 1, 32);
-    for (size_t i = 0; i < cols.size(); ++i)
-      for (int o = 0; o < cols[i].w; o += seg) {
-        segs.push_back(make_int4(cols[i].x, cols[i].y, cols[i].z + o, std::min(seg, cols[i].w - o)));
-        segk.push_back(colk[i] + o);
-      }
-    std::vector<int> order(segs.size());
-    for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
-    std::stable_sort(order.begin(), order.end(),
-                     [&](int a, int b2) { return segs[a].w > segs[b2].w; });
-    std::vector<int4> ss(segs.size());
-    std::vector<int> sk(segk.size());
-    for (size_t i = 0; i < order.size(); ++i) {
-      ss[i] = segs[order[i]];
-      sk[i] = segk[order[i]];
-    }
-    segs.swap(ss);
-    segk.swap(sk);
-  }
-  c.nseg = (int)segs.size();
-  c.segmax = 0;
-  for (auto &sg : segs) c.segmax = std::max(c.segmax, sg.w);
-  // site chunks of at most 64 sites keep the staged tables within LDS
-  c.sf_chunks_max = std::max(32, (3 * c.N + 63) / 64);
+  t.colrec = column_records(c, cols);
+  t.sftask = sfac_tasks(cols);
+  c.sf_ntask = (int)t.sftask.size();
+  c.sf_chunks_max = sfac_chunks_max(c);
   // launch-shape tuning (results do not depend on them)
   // default launch shapes by size: a system of few molecule-beads (a
   // contracted run's one-bead centroid, small replicas) gives each molecule
@@ -569,23 +539,13 @@ void plan_system(pimd_ctx *x, HostTables &t) {
               : mode == 2 || c.P * M * M <= DENSE_MAX_PAIRS ? 2 : 0;
     if (c.dense) c.dd_cache = 0;
   }
-  // structure-factor site chunks: about 8 per bead from 4096 molecule-beads
-  // on (with two lane sets per block; 512 H2O x 32 beads: 1.66 -> 1.61 ms per
-  // mixed force call, TTM2.1-F 128 x 32: 1.75 -> 1.66 ms FP64), the staged
-  // tables of a chunk within 60 KB; 8 sites below, to spread small systems
-  int dflt_sites = 8;
-  if (mb >= 4096) {
-    const int lds_cap = std::max(8, 60 * 1024 / (16 * c.T) - 17);
-    dflt_sites = std::max(8, std::min({(c.nd * c.N + 7) / 8, 128, lds_cap}));
-  }
+  // structure-factor site chunks: as many as give every CU one block of the
+  // dipole pass, at least 8 sites each (512 H2O x 32 beads, FP64 MD step: 16,
+  // 32, 48, 64, 96 and 128 sites 1.44, 1.31, 1.34, 1.26, 1.31 and 1.34 ms)
+  const int dflt_chunks = (256 + c.P - 1) / c.P;
+  const int dflt_sites = std::max(8, std::min((c.nd * c.N + dflt_chunks - 1) / dflt_chunks, 128));
   c.sf_sites = env_int("PIMD_SFAC_SITES", dflt_sites, 1, 128);
   c.fd_cg = env_int("PIMD_FIELD_CG", 0, 0, 16);
-  c.sf_kind = env_int("PIMD_SFAC_KIND", 1, 0, 1);
-  c.sfv_col = env_int("PIMD_SFV_COL", 1, 0, 1);
-  c.sf_split = env_int("PIMD_SFAC_SPLIT", 1, 0, 1);
-  c.fd_klds = env_int("PIMD_FIELD_KLDS", 1, 0, 1);
-  // phase tables of 64 sites, or the 16-group reduction if larger (in double2)
-  c.fd_tab_d2 = std::max(c.T * 64, 16 * 4 * 64 / 2);
   c.g_dd = env_int("PIMD_G_DD", dflt_dd, 0, 64);
   c.g_qq = env_int("PIMD_G_QQ", dflt_qq, 0, 32);
   c.g_fin = env_int("PIMD_G_FIN", dflt_qq, 0, 32);
@@ -659,7 +619,8 @@ void layout_system(pimd_ctx *x, Arena &a, bool full) {
   a.take(&d.Sm, P * nk * 2);
   a.take(&d.Sv, P * nk * 6);
   a.take(&d.virk, P * ((nk + 255) / 256) * 18);
-  a.take(&d.part, P * (size_t)c.sf_chunks_max * nk * 6);
+  a.take(&d.part, full ? P * (size_t)c.sf_chunks_max * nk * 6 : sfac_part_elems(c));
+  a.take(&d.wk, field_operand_elems(c));
   a.take(&d.active, P);
   a.take(&d.iters, P);
   a.take(&d.nactive, (size_t)c.maxiter + 1);
@@ -668,8 +629,8 @@ void layout_system(pimd_ctx *x, Arena &a, bool full) {
   a.take(&d.red, nk);  // A_k
   a.take(&d.cols, c.ncol);
   a.take(&d.colk, c.ncol);
-  a.take(&d.segs, c.nseg);
-  a.take(&d.segk, c.nseg);
+  a.take(&d.colrec, ((size_t)c.ncol + 15) / 16 * 16);
+  a.take(&d.sftask, c.sf_ntask);
   a.take(&d.Upot, P);
   a.take(&d.virt, P * 9);
   a.take(&d.virialc, P);
@@ -721,8 +682,8 @@ int upload_system(pimd_ctx *x, const HostTables &t, hipStream_t s) {
   HIPCHK(hipMemcpyAsync(d.red, x->Ak.data(), sizeof(double) * nk, hipMemcpyHostToDevice, s));
   HIPCHK(hipMemcpyAsync(d.cols, t.cols.data(), sizeof(int4) * t.cols.size(), hipMemcpyHostToDevice, s));
   HIPCHK(hipMemcpyAsync(d.colk, t.colk.data(), sizeof(int) * t.colk.size(), hipMemcpyHostToDevice, s));
-  HIPCHK(hipMemcpyAsync(d.segs, t.segs.data(), sizeof(int4) * t.segs.size(), hipMemcpyHostToDevice, s));
-  HIPCHK(hipMemcpyAsync(d.segk, t.segk.data(), sizeof(int) * t.segk.size(), hipMemcpyHostToDevice, s));
+  HIPCHK(hipMemcpyAsync(d.colrec, t.colrec.data(), sizeof(ColRec) * t.colrec.size(), hipMemcpyHostToDevice, s));
+  HIPCHK(hipMemcpyAsync(d.sftask, t.sftask.data(), sizeof(int) * t.sftask.size(), hipMemcpyHostToDevice, s));
   if (c.dense) {
     HIPCHK(hipMemcpyAsync(d.dcol, t.dcol.data(), sizeof(int4) * t.dcol.size(), hipMemcpyHostToDevice, s));
     HIPCHK(hipMemcpyAsync(d.dkx, t.dkx.data(), sizeof(int) * t.dkx.size(), hipMemcpyHostToDevice, s));
@@ -2608,9 +2569,6 @@ extern "C" int pimd_forces_all_beads_noalloc(const pimd_params *params, const do
   x.c.poll = 0;
   x.c.overlap = 0;
   x.c.dd_cache = 0;
-  // partial sums for the chunks the structure factors use (the same
-  // chunking as a context's, so the results are the same bits)
-  x.c.sf_chunks_max = sfac_chunks_used(x.c);
   Arena a;
   layout_system(&x, a, false);
   if (x.c.dense && a.off > sizeof(scratch)) {

@@ -44,6 +44,13 @@ struct __align__(32) Site {
   double x, y, z, q;
 };
 
+// One kz-column: its kx, ky, the phase-table rows of both, the sign bit where
+// ky < 0 (the row is |ky|'s) and its largest |kz|.
+struct __align__(16) ColRec {
+  double kx, ky;
+  int rx, ry, sgn, reach;
+};
+
 // Everything the kernels need about the model and the box, passed by value.
 struct SysConst {
   int N, P, model;        // waters, beads, pot_model (2, 3 TTM; 4, 5 fixed-charge SPC)
@@ -56,16 +63,10 @@ struct SysConst {
   int nbr_cap;
   int cells;               // 1: neighbour search through a cell list
   int ncell[3];            // cells per axis (>= 3 each when cells = 1), width >= Rc
-  int kzmax;               // longest kz-column
-  int nseg, segmax;        // kz-columns cut into segments of at most segmax k
-  int sf_chunks_max;       // site chunks of the column structure-factor kernel
+  int sf_ntask;            // structure-factor tasks (16 kz-columns x 8 |kz|)
+  int sf_chunks_max;       // most site chunks of a structure factor
   int sf_sites;            // fewest sites per structure-factor chunk
-  int fd_cg;               // column groups per field block (0: by occupancy)
-  int fd_klds;             // 1: field kernels stage the bead's k data in LDS
-  int fd_tab_d2;           // double2 slots of the field kernel's table / reduction area
-  int sf_kind;             // structure-factor kernel: 0 one k per lane, 1 kz-columns
-  int sfv_col;             // 1: the 6-component SF_V by kz-columns too
-  int sf_split;            // 1: column structure factors with two lane sets per block
+  int fd_cg;               // waves (column groups) per field block (0: by columns)
   int g_dd;                // lanes per molecule of the LDS-staged dipole kernel (0: gather kernel)
   int g_qq, g_fin;         // the same for the charge and final pair kernels
   int g_nolds;             // lanes per molecule of the pair kernels that do not stage in LDS
@@ -148,15 +149,16 @@ struct DevBufs {
   dptr<double> Sq = nullptr, Sm = nullptr;  // [P][nk][2]
   dptr<double> Sv = nullptr;  // [P][nk][6]
   dptr<double> virk = nullptr;  // [P][nkb][9]
-  dptr<double> part = nullptr;  // [P][sf_chunks_max][nk][2]
+  dptr<double> part = nullptr;  // [P][chunks][nk][2 or 6] structure-factor chunk sums
+  dptr<double> wk = nullptr;  // field operands of the structure factors (recip.hip)
   dptr<int> active = nullptr, iters = nullptr;  // [P]
   dptr<int> nactive = nullptr;  // [1]
   dptr<double4> kv = nullptr;  // [nk] kx, ky, kz, Ak
   dptr<int4> khkl = nullptr;  // [nk] h, k, l, 0
   dptr<int4> cols = nullptr;  // [ncol] h, k, l_first, count
   dptr<int> colk = nullptr;  // [ncol] first k index
-  dptr<int4> segs = nullptr;  // [nseg] h, k, l_first, count
-  dptr<int> segk = nullptr;  // [nseg] first k index
+  dptr<ColRec> colrec = nullptr;  // [ncol up to a multiple of 16]
+  dptr<int> sftask = nullptr;  // [sf_ntask] column tile | |kz| tile << 16
   // outputs of the last force call
   dptr<double> Upot = nullptr, virt = nullptr, virialc = nullptr, terms = nullptr;  // [P],[P][9],[P],[P][5]
   dptr<double> dRR = nullptr, dipI = nullptr, dipE = nullptr, chg = nullptr;
@@ -341,7 +343,11 @@ __host__ __device__ inline size_t dense_stride(const SysConst &c) {
 inline size_t dense_elems(const SysConst &c) {
   return (size_t)c.P * 3 * c.nd * c.N * dense_stride(c);
 }
-int sfac_chunks_used(const SysConst &c);
+int sfac_chunks_max(const SysConst &c);
+size_t sfac_part_elems(const SysConst &c);
+size_t field_operand_elems(const SysConst &c);
+std::vector<ColRec> column_records(const SysConst &c, const std::vector<int4> &cols);
+std::vector<int> sfac_tasks(const std::vector<int4> &cols);
 void launch_converge(const Group &g, int iter, hipStream_t s);
 // iter: the SOR iteration of FD_D, -1 for the FP64 refinement (maxiter + 1);
 // sel_mixed: only the replicas of the mixed form

@@ -1013,671 +1013,6 @@ __global__ __launch_bounds__(256) void k_pair_qq_partner(const Rep *__restrict__
 static size_t bead_sites_lds(const SysConst &c) { return sizeof(Site) * 4 * c.N; }
 constexpr size_t PAIR_LDS_MAX = 150 * 1024;
 
-
-
-
-
-// ---------------------------------------------------------------------------
-// Ewald reciprocal space (ewald.f90:1-226, 403-437).
-// ---------------------------------------------------------------------------
-
-// Per-site phase tables, the reference's ssincos recurrence (ewald.f90:403-437).
-__global__ __launch_bounds__(256) void k_tables(const Rep *__restrict__ reps, BlockMap bm) {
-  const Blk bk = block_of(bm);
-  const Rep &Rp = reps[bk.r];
-  const SysConst &c = Rp.c;
-  const Site *__restrict__ site = Rp.b.site;
-  double2 *tab = Rp.b.tab;
-  const int S = 4 * c.N;
-  const int s = bk.x * blockDim.x + threadIdx.x;
-  const int b = bk.y;
-  if (s >= S) return;
-  const Site p = site[(size_t)b * S + s];
-  const double xyz[3] = {p.x, p.y, p.z};
-  const int hm[3] = {c.hmax, c.kmax, c.lmax};
-  int row = 0;
-  double2 *tb = tab + (size_t)b * c.T * S + s;
-  // the dipole sites' rows again, contiguous in dipole-site order (mol * nd +
-  // j), for the passes over dipole sites only; FP32 too in the mixed form
-  const int type = s & 3, MD = c.nd * c.N;
-  const bool dsite = type >= c.tdip && type < c.tdip + c.nd;
-  const size_t dm = (size_t)b * c.T * MD + (size_t)(s >> 2) * c.nd + (type - c.tdip);
-  double2 *td = Rp.b.tabd + dm;
-  float2 *tf = c.mixed ? Rp.b.tabdf + dm : nullptr;
-  auto put = [&](int r, double2 v) {
-    tb[(size_t)r * S] = v;
-    if (dsite) {
-      td[(size_t)r * MD] = v;
-      if (tf) tf[(size_t)r * MD] = make_float2((float)v.x, (float)v.y);
-    }
-  };
-  for (int ax = 0; ax < 3; ++ax) {
-    const double arg = TWOPI * c.boxi[ax] * xyz[ax];
-    const double c1 = cos(arg), s1 = sin(arg);
-    double cc = 1.0, ss = 0.0;
-    put(row++, make_double2(1.0, 0.0));
-    for (int h = 1; h <= hm[ax]; ++h) {
-      double nc, ns;
-      if (h == 1) {
-        nc = c1;
-        ns = s1;
-      } else {
-        nc = cc * c1 - ss * s1;
-        ns = cc * s1 + ss * c1;
-      }
-      cc = nc;
-      ss = ns;
-      put(row++, make_double2(cc, ss));
-    }
-  }
-}
-
-
-// Site index of the m-th member of a site set.  SET_CHG: H1, H2, M of every
-// molecule; SET_DIP: the dipole sites; SET_ALL: all four.
-// SET_CHG_T / SET_ALL_T: the same sites as SET_CHG / SET_ALL, type-major
-// (all H1, then all H2, ...), so that a wave of the final reciprocal pass holds
-// one site type and its dipole-site branch is wave-uniform.
-enum SiteSet { SET_CHG = 0, SET_DIP = 1, SET_ALL = 2, SET_CHG_T = 3, SET_ALL_T = 4 };
-
-__device__ __forceinline__ int set_size(const SysConst &c, int set) {
-  return set == SET_CHG || set == SET_CHG_T ? 3 * c.N : set == SET_DIP ? c.nd * c.N : 4 * c.N;
-}
-__device__ __forceinline__ int set_site(const SysConst &c, int set, int m) {
-  if (set == SET_CHG) return (m / 3) * 4 + 1 + m % 3;
-  if (set == SET_DIP) return (m / c.nd) * 4 + c.tdip + m % c.nd;
-  if (set == SET_CHG_T) return (m % c.N) * 4 + 1 + m / c.N;
-  if (set == SET_ALL_T) return (m % c.N) * 4 + m / c.N;
-  return m;
-}
-
-// Phase e^{i k.r} of one site from its table rows, in the reference's
-// product order (ewald.f90:30-39).
-template <class V, class R>
-__device__ __forceinline__ void phase_from(V x, V y, V z, R &ck, R &sk) {
-  const R cxy = x.x * y.x - x.y * y.y;
-  const R sxy = x.y * y.x + x.x * y.y;
-  ck = cxy * z.x - sxy * z.y;
-  sk = sxy * z.x + cxy * z.y;
-}
-
-// Two- and four-component vectors of an arithmetic type.
-template <class R> struct Vec;
-template <> struct Vec<double> {
-  using v2 = double2;
-  using v4 = double4;
-  static __device__ __forceinline__ double2 two(double a, double b) { return make_double2(a, b); }
-  static __device__ __forceinline__ double4 four(double a, double b, double c, double d) {
-    return make_double4(a, b, c, d);
-  }
-};
-template <> struct Vec<float> {
-  using v2 = float2;
-  using v4 = float4;
-  static __device__ __forceinline__ float2 two(double a, double b) {
-    return make_float2((float)a, (float)b);
-  }
-  static __device__ __forceinline__ float4 four(double a, double b, double c, double d) {
-    return make_float4((float)a, (float)b, (float)c, (float)d);
-  }
-};
-
-// Phase-table rows of the m-th member of a site set: the dipole sites from
-// their contiguous table (FP32 in the mixed form's SOR iterations), the
-// other sets from the all-site table.
-template <class R, int SET>
-__device__ __forceinline__ const typename Vec<R>::v2 *set_rows(const Rep &Rp, int b, int &stride) {
-  const SysConst &c = Rp.c;
-  if constexpr (SET == SET_DIP) {
-    stride = c.nd * c.N;
-    const size_t off = (size_t)b * c.T * stride;
-    if constexpr (sizeof(R) == 4) return Rp.b.tabdf + off;
-    else return Rp.b.tabd + off;
-  } else {
-    static_assert(sizeof(R) == 8, "the all-site table is FP64");
-    stride = 4 * c.N;
-    return Rp.b.tab + (size_t)b * c.T * stride;
-  }
-}
-template <int SET>
-__device__ __forceinline__ int row_index(const SysConst &c, int m) {
-  return SET == SET_DIP ? m : set_site(c, SET, m);
-}
-
-// Site chunk of the column structure-factor kernel and its padded LDS row
-// (a multiple of 16 plus one double2, so rows start 4 banks apart).
-__host__ __device__ inline void sfac_chunking(const SysConst &c, int mode, int M, int &nch,
-                                              int &sc, int &scp) {
-  // the dipole structure factor takes c.sf_sites per chunk; the charge and
-  // virial ones at most 32, which keeps their blocks spread over the device
-  const int sites = mode == SF_D ? c.sf_sites : (c.sf_sites < 32 ? c.sf_sites : 32);
-  const int want = (M + sites - 1) / sites;
-  nch = want < c.sf_chunks_max ? want : c.sf_chunks_max;
-  if (nch < 1) nch = 1;
-  sc = (M + nch - 1) / nch;
-  if (sc < 1) sc = 1;  // an empty site set (no dipole sites): one empty chunk
-  nch = (M + sc - 1) / sc;
-  if (nch < 1) nch = 1;
-  scp = ((sc + 15) / 16) * 16 + 1;
-}
-
-// Sites of a structure factor's site set.
-__host__ __device__ inline int sfac_sites(const SysConst &c, int mode) {
-  return mode == SF_Q ? 3 * c.N : c.nd * c.N;
-}
-
-// Structure factors with one kz-segment (fixed kx, ky, up to KZ consecutive kz)
-// per lane: the phase of each site is formed once per segment and advanced
-// along kz by e^{i 2 pi z/L}, accumulating every kz of the segment in
-// registers.  stale (SF_D): of every bead's dip_prev, the input of its last
-// SOR step, in place of its current dipoles (dense systems).  A block takes a chunk of
-// sites of one bead; their phase tables and weights are staged in LDS (rows
-// padded so that lanes reading different rows of one site hit different
-// banks).  Per-chunk partial sums are combined in a fixed order by
-// k_sfac_reduce.  SF_Q and SF_D as above.
-// SPLIT = 2: the block holds two lane sets for the same segments, each over
-// half of the chunk's sites; the second hands its sums to the first through
-// LDS, which adds them and writes (twice the waves for the same partials).
-template <int MODE, int KZ, int SPLIT = 1, class R = double>
-__global__ __launch_bounds__(512) void k_sfac_col(const Rep *__restrict__ reps, BlockMap bm,
-                                                  int stale) {
-  using R2 = typename Vec<R>::v2;
-  constexpr int SET = MODE == SF_Q ? SET_CHG : SET_DIP;
-  constexpr int NW = MODE == SF_Q ? 1 : 3;
-  constexpr int NV = MODE == SF_V ? 6 : 2;  // values per k
-  // sites per unrolled step: the grid, not the registers, limits the waves
-  // per SIMD, so more independent phase chains per wave hide FP64 latency
-  constexpr int SITE_UNROLL = MODE == SF_V ? 2 : 4;
-  extern __shared__ double2 lds_raw[];
-  R2 *lds_sf = reinterpret_cast<R2 *>(lds_raw);  // [T][scp] tables, then [sc][NW] weights
-  const Blk bk = block_of(bm);
-  const Rep &Rp = reps[bk.r];
-  const SysConst &c = Rp.c;
-  const Site *__restrict__ site = Rp.b.site;
-  const double *__restrict__ dip = stale ? Rp.b.dip_prev : Rp.b.dip;
-  const int4 *__restrict__ cols = Rp.b.segs;
-  const int *__restrict__ colk = Rp.b.segk;
-  const int *__restrict__ active = Rp.b.active;
-  double *__restrict__ part = Rp.b.part;
-  int nch, sc, scp;
-  sfac_chunking(c, MODE, sfac_sites(c, MODE), nch, sc, scp);
-  R *lw = reinterpret_cast<R *>(lds_sf + (size_t)c.T * scp);
-  const int b = bk.z;
-  if (MODE == SF_D && !stale && !active[b]) return;
-  const int S = 4 * c.N, M = set_size(c, SET);
-  const int chunk = bk.y;
-  const int m0 = chunk * sc, nt = min(sc, M - m0);
-  int RS;
-  const R2 *__restrict__ tb = set_rows<R, SET>(Rp, b, RS);
-  for (int e = threadIdx.x; e < c.T * sc; e += blockDim.x) {
-    const int row = e / sc, l = e % sc;
-    if (l < nt) lds_sf[row * scp + l] = tb[(size_t)row * RS + row_index<SET>(c, m0 + l)];
-  }
-  for (int l = threadIdx.x; l < nt; l += blockDim.x) {
-    const int sidx = set_site(c, SET, m0 + l);
-    if (MODE == SF_Q) {
-      lw[l] = site[(size_t)b * S + sidx].q;
-    } else {
-      const double *mu = dip + ((size_t)b * c.N * c.nd + m0 + l) * 3;
-      lw[l * 3 + 0] = (R)mu[0];
-      lw[l * 3 + 1] = (R)mu[1];
-      lw[l * 3 + 2] = (R)mu[2];
-    }
-  }
-  __syncthreads();
-  const int nl = blockDim.x / SPLIT, half_id = threadIdx.x / nl;
-  const int col = bk.x * nl + threadIdx.x % nl;
-  const bool live = col < c.nseg;
-  const int hn = (nt + SPLIT - 1) / SPLIT;
-  const int e0 = half_id * hn, e1 = min(nt, e0 + hn);
-  const int4 cl = cols[live ? col : 0];
-  const int n = cl.w;
-  const int k0 = colk[live ? col : 0];
-  const int rowx = cl.x, rowy = c.hmax + 1 + abs(cl.y), rowz = c.hmax + c.kmax + 2 + abs(cl.z);
-  const int rowz1 = c.hmax + c.kmax + 3;
-  const R sgy = cl.y < 0 ? -1.0 : 1.0, sgz = cl.z < 0 ? -1.0 : 1.0;
-  const R kvx = TWOPI * c.boxi[0] * (double)cl.x, kvy = TWOPI * c.boxi[1] * (double)cl.y;
-  const double tpz = TWOPI * c.boxi[2];
-  // kz of each k of the segment
-  R kzs[KZ];
-#pragma unroll
-  for (int i = 0; i < KZ; ++i) kzs[i] = (R)(tpz * (double)(cl.z + i));
-  // SF_Q, SF_D: (re, im) per k; SF_V: (sum mu cos, sum mu sin) per component
-  R acc[NV][KZ];
-#pragma unroll
-  for (int v = 0; v < NV; ++v)
-#pragma unroll
-    for (int i = 0; i < KZ; ++i) acc[v][i] = 0.0;
-  #pragma unroll SITE_UNROLL
-  for (int e = live ? e0 : e1; e < e1; ++e) {
-    const R2 x = lds_sf[rowx * scp + e];
-    R2 y = lds_sf[rowy * scp + e];
-    R2 z = lds_sf[rowz * scp + e];
-    const R2 z1 = c.lmax >= 1 ? lds_sf[rowz1 * scp + e] : Vec<R>::two(1.0, 0.0);
-    y.y *= sgy;
-    z.y *= sgz;
-    R ck, sk;
-    phase_from(x, y, z, ck, sk);
-    R w = 0.0, wxy = 0.0, mz = 0.0;
-    if (MODE == SF_Q) {
-      w = lw[e];
-    } else if (MODE == SF_D) {
-      wxy = kvx * lw[e * 3 + 0] + kvy * lw[e * 3 + 1];
-      mz = lw[e * 3 + 2];
-    }
-#pragma unroll
-    for (int i = 0; i < KZ; ++i) {
-      if (i < n) {
-        if (i > 0) {
-          const R nc = ck * z1.x - sk * z1.y;
-          sk = sk * z1.x + ck * z1.y;
-          ck = nc;
-        }
-        if (MODE == SF_Q) {
-          acc[0][i] += w * ck;
-          acc[1][i] += w * sk;
-        } else if (MODE == SF_D) {
-          const R dk = wxy + kzs[i] * mz;
-          acc[0][i] -= dk * sk;
-          acc[1][i] += dk * ck;
-        } else {
-#pragma unroll
-          for (int cc = 0; cc < 3; ++cc) {
-            acc[cc][i] += lw[e * 3 + cc] * ck;
-            acc[3 + cc][i] += lw[e * 3 + cc] * sk;
-          }
-        }
-      }
-    }
-  }
-  if (SPLIT == 2) {
-    // after the weights, 16-byte aligned: [NV][KZ][nl] sums of the second set
-    constexpr int AL = 16 / sizeof(R);
-    R *red = lw + ((sc * NW + AL - 1) & ~(AL - 1));
-    if (half_id == 1 && live)
-#pragma unroll
-      for (int v = 0; v < NV; ++v)
-#pragma unroll
-        for (int i = 0; i < KZ; ++i) red[(v * KZ + i) * nl + threadIdx.x % nl] = acc[v][i];
-    __syncthreads();
-    if (half_id == 0)
-#pragma unroll
-      for (int v = 0; v < NV; ++v)
-#pragma unroll
-        for (int i = 0; i < KZ; ++i) acc[v][i] += red[(v * KZ + i) * nl + threadIdx.x];
-  }
-  if (!live || half_id != 0) return;
-  double *o = part + (((size_t)b * nch + chunk) * c.nk + k0) * NV;
-#pragma unroll
-  for (int i = 0; i < KZ; ++i)
-    if (i < n)
-#pragma unroll
-      for (int v = 0; v < NV; ++v) o[NV * i + v] = (double)acc[v][i];
-}
-
-// Structure factors with one k-vector per lane.  A block holds 256 k of one
-// bead and a chunk of its sites; the sites' phase tables and weights are
-// staged in LDS (rows padded so that lanes reading different rows of one site
-// hit different banks; lanes on the same row read the same address).  Each
-// lane forms e^{i k.r} = X(kx) Y(ky) Z(kz) of every site from the tables and
-// accumulates its weighted sum; per-chunk partial sums are combined in a fixed
-// order by k_sfac_reduce.
-//   SF_Q: (sum q cos, sum q sin)                      (ewald.f90:41-44)
-//   SF_D: (-sum (k.mu) sin, sum (k.mu) cos)           (ewald.f90:99-110)
-//   SF_V: (sum mu cos, sum mu sin) per component      (ewald.f90:208-213)
-template <int MODE>
-__global__ __launch_bounds__(256) void k_sfac_k(const Rep *__restrict__ reps, BlockMap bm,
-                                                int stale) {
-  constexpr int SET = MODE == SF_Q ? SET_CHG : SET_DIP;
-  constexpr int NW = MODE == SF_Q ? 1 : 3;
-  constexpr int NV = MODE == SF_V ? 6 : 2;
-  extern __shared__ double2 lds_sf[];  // [T][scp] tables, then [sc][NW] weights
-  const Blk bk = block_of(bm);
-  const Rep &Rp = reps[bk.r];
-  const SysConst &c = Rp.c;
-  const Site *__restrict__ site = Rp.b.site;
-  const double *__restrict__ dip = stale ? Rp.b.dip_prev : Rp.b.dip;
-  const double4 *__restrict__ kv = Rp.b.kv;
-  const int4 *__restrict__ khkl = Rp.b.khkl;
-  const int *__restrict__ active = Rp.b.active;
-  double *__restrict__ part = Rp.b.part;
-  int nch, sc, scp;
-  sfac_chunking(c, MODE, sfac_sites(c, MODE), nch, sc, scp);
-  double *lw = reinterpret_cast<double *>(lds_sf + (size_t)c.T * scp);
-  const int b = bk.z;
-  if (MODE == SF_D && !stale && !active[b]) return;
-  const int S = 4 * c.N, M = set_size(c, SET);
-  const int chunk = bk.y;
-  const int m0 = chunk * sc, nt = min(sc, M - m0);
-  int RS;
-  const double2 *__restrict__ tb = set_rows<double, SET>(Rp, b, RS);
-  for (int e = threadIdx.x; e < c.T * sc; e += blockDim.x) {
-    const int row = e / sc, l = e % sc;
-    if (l < nt) lds_sf[row * scp + l] = tb[(size_t)row * RS + row_index<SET>(c, m0 + l)];
-  }
-  for (int l = threadIdx.x; l < nt; l += blockDim.x) {
-    if (MODE == SF_Q) {
-      lw[l] = site[(size_t)b * S + set_site(c, SET, m0 + l)].q;
-    } else {
-      const double *mu = dip + ((size_t)b * c.N * c.nd + m0 + l) * 3;
-      lw[l * 3 + 0] = mu[0];
-      lw[l * 3 + 1] = mu[1];
-      lw[l * 3 + 2] = mu[2];
-    }
-  }
-  __syncthreads();
-  const int k = bk.x * blockDim.x + threadIdx.x;
-  if (k >= c.nk) return;
-  const int4 h = khkl[k];
-  const double4 kvec = kv[k];
-  const int rowx = h.x * scp, rowy = (c.hmax + 1 + abs(h.y)) * scp;
-  const int rowz = (c.hmax + c.kmax + 2 + abs(h.z)) * scp;
-  const double sy = h.y < 0 ? -1.0 : 1.0, sz = h.z < 0 ? -1.0 : 1.0;
-  double acc[NV];
-#pragma unroll
-  for (int v = 0; v < NV; ++v) acc[v] = 0.0;
-#pragma unroll 2
-  for (int e = 0; e < nt; ++e) {
-    const double2 x = lds_sf[rowx + e];
-    double2 y = lds_sf[rowy + e];
-    double2 z = lds_sf[rowz + e];
-    y.y *= sy;
-    z.y *= sz;
-    double ck, sk;
-    phase_from(x, y, z, ck, sk);
-    if (MODE == SF_Q) {
-      const double q = lw[e];
-      acc[0] += q * ck;
-      acc[1] += q * sk;
-    } else if (MODE == SF_D) {
-      const double dk = (kvec.x * lw[e * 3] + kvec.y * lw[e * 3 + 1]) + kvec.z * lw[e * 3 + 2];
-      acc[0] -= dk * sk;
-      acc[1] += dk * ck;
-    } else {
-#pragma unroll
-      for (int cc = 0; cc < 3; ++cc) {
-        acc[cc] += lw[e * 3 + cc] * ck;
-        acc[3 + cc] += lw[e * 3 + cc] * sk;
-      }
-    }
-  }
-  double *o = part + (((size_t)b * nch + chunk) * c.nk + k) * NV;
-#pragma unroll
-  for (int v = 0; v < NV; ++v) o[v] = acc[v];
-}
-
-// The per-chunk partial sums of structure factor `mode` added in chunk order.
-__global__ __launch_bounds__(256) void k_sfac_reduce(const Rep *__restrict__ reps, BlockMap bm,
-                                                    int mode, int stale) {
-  const Blk bk = block_of(bm);
-  const Rep &Rp = reps[bk.r];
-  const SysConst &c = Rp.c;
-  const double *__restrict__ part = Rp.b.part;
-  double *__restrict__ out = mode == SF_Q ? Rp.b.Sq : mode == SF_D ? Rp.b.Sm : Rp.b.Sv;
-  const int nv = mode == SF_V ? 6 : 2;
-  int nch, sc, scp;
-  sfac_chunking(c, mode, sfac_sites(c, mode), nch, sc, scp);
-  const int b = bk.y;
-  if (mode == SF_D && !stale && !Rp.b.active[b]) return;
-  const int e = bk.x * blockDim.x + threadIdx.x;  // (k, component)
-  if (e >= nv * c.nk) return;
-  double v = 0.0;
-  const double *pp = part + (size_t)b * nch * c.nk * nv + e;
-#pragma unroll 8
-  for (int q = 0; q < nch; ++q) v += pp[(size_t)q * c.nk * nv];
-  out[(size_t)b * c.nk * nv + e] = v;
-}
-
-static size_t sfac_lds(const SysConst &c, int mode, int sc, int scp, bool f32 = false) {
-  const size_t r = f32 ? sizeof(float) : sizeof(double);
-  return 2 * r * c.T * scp + r * sc * (mode == SF_Q ? 1 : 3);
-}
-
-// The most site chunks any structure factor of a force call uses (the
-// partial sums hold P x this many chunks of nk k-vectors).
-int sfac_chunks_used(const SysConst &c) {
-  int most = 1;
-  for (int mode : {SF_Q, SF_D, SF_V}) {
-    int nch, sc, scp;
-    sfac_chunking(c, mode, sfac_sites(c, mode), nch, sc, scp);
-    most = std::max(most, nch);
-  }
-  return most;
-}
-
-
-
-
-
-
-// Reciprocal-space fields at each site.  A block holds 64 sites of one bead,
-// one per lane, and CG waves; wave g walks kz-columns g, g + CG, ... (columns
-// are sorted by length, so the waves get similar trip counts).  All lanes of a
-// wave are on the same k at the same time, so the k data (k-vector, 4 pi A_k/V,
-// structure factor) is wave-uniform and read with scalar loads; each lane's
-// phase e^{i k.r} comes from its site's tables, staged in LDS, and is advanced
-// along the column by e^{i 2 pi z/L}.  Along a column kx and ky are fixed, so
-// the x and y field components are kx and ky times one column sum.  The CG
-// partial fields of a site are combined in a fixed order through LDS.
-//   FD_Q : Efq and phi from the charge structure factor (ewald.f90:45-49)
-//   FD_D : Efd from the dipole structure factor (ewald.f90:114-117), then the
-//          SOR update of the induced dipole (pot_ttm.f90:371-385)
-//   FD_QD: phi and dR from the stale dipole and the total structure factors
-//          (ewald.f90:184-193)
-constexpr int FD_SB = 64;  // sites per block, one per lane
-// iter: the SOR iteration (FD_D), or -1 for the mixed form's FP64
-// refinement, the step after the replica's last (maxiter + 1).
-template <int MODE, int MODEL, int CG, bool KL, class R = double>
-__global__ __launch_bounds__(64 * CG) void k_field(const Rep *__restrict__ reps, BlockMap bm,
-                                                   int iter) {
-  using R2 = typename Vec<R>::v2;
-  using R4 = typename Vec<R>::v4;
-  constexpr int SET = MODE == FD_D    ? SET_DIP
-                      : MODE == FD_QD ? (MODEL == 2 ? SET_ALL_T : SET_CHG_T)
-                                      : (MODEL == 2 ? SET_ALL : SET_CHG);
-  // [T][64] phase tables of the block's sites (later reused for the
-  // reduction), then with KL the bead's k data: [nk] (w Re S, w Im S, kz, w)
-  // with w = 4 pi A_k / V, and for FD_QD [nk] (w Re(Sq+Sm), w Im(Sq+Sm))
-  extern __shared__ double2 lds_raw[];
-  R2 *lds_tab = reinterpret_cast<R2 *>(lds_raw);
-  const Blk bk = block_of(bm);
-  const Rep &Rp = reps[bk.r];
-  const SysConst &c = Rp.c;
-  const Site *__restrict__ site = Rp.b.site;
-  const double4 *__restrict__ kv = Rp.b.kv;
-  const int4 *__restrict__ cols = Rp.b.cols;
-  const int *__restrict__ colk = Rp.b.colk;
-  const double *__restrict__ Sq = Rp.b.Sq, *__restrict__ Sm = Rp.b.Sm;
-  // FD_Q and FD_QD write their reciprocal-space parts to kE / kphi, added by
-  // their consumers (the real-space pair pass may be forming the rest meanwhile)
-  double *__restrict__ phi = MODE == FD_D ? Rp.b.phi : Rp.b.kphi;
-  double *__restrict__ Efq = MODE == FD_Q ? Rp.b.kE : Rp.b.Efq;
-  double *__restrict__ dR = MODE == FD_QD ? Rp.b.kE : Rp.b.dR;
-  double *__restrict__ dip = Rp.b.dip, *__restrict__ dip_prev = Rp.b.dip_prev;
-  const double *__restrict__ Efd = Rp.b.Efd;
-  double *__restrict__ diff2 = Rp.b.diff2;
-  const int *__restrict__ active = Rp.b.active;
-  if (iter < 0) iter = c.maxiter + 1;
-  const int b = bk.y;
-  if (MODE == FD_D && !active[b]) return;
-  const int lane = threadIdx.x & 63;
-  const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int M = set_size(c, SET);
-  const int S = 4 * c.N;
-  const int mbase = bk.x * FD_SB;
-  int RS;
-  const R2 *__restrict__ tb = set_rows<R, SET>(Rp, b, RS);
-  for (int e = threadIdx.x; e < c.T * FD_SB; e += 64 * CG) {
-    const int row = e >> 6, l = e & 63;
-    lds_tab[e] = tb[(size_t)row * RS + row_index<SET>(c, min(mbase + l, M - 1))];
-  }
-  R4 *kd = reinterpret_cast<R4 *>(lds_raw + c.fd_tab_d2);
-  double2 *kq = reinterpret_cast<double2 *>(kd + c.nk);
-  if (KL) {
-    const double *sx = (MODE == FD_Q ? Sq : Sm) + (size_t)b * c.nk * 2;
-    const double *sq2 = Sq + (size_t)b * c.nk * 2;
-    for (int k = threadIdx.x; k < c.nk; k += 64 * CG) {
-      const double4 kk = kv[k];
-      kd[k] = Vec<R>::four(kk.w * sx[2 * k], kk.w * sx[2 * k + 1], kk.z, kk.w);
-      if (MODE == FD_QD) kq[k] = make_double2(kk.w * (sq2[2 * k] + sx[2 * k]),
-                                              kk.w * (sq2[2 * k + 1] + sx[2 * k + 1]));
-    }
-  }
-  __syncthreads();
-  const int m = mbase + lane;
-  const bool valid = m < M;
-  const int s = set_site(c, SET, valid ? m : M - 1);
-  const int type = s & 3;
-  const bool has_q = type != 0;
-  const bool has_d = (type >= c.tdip && type < c.tdip + c.nd);
-  const size_t dslot = ((size_t)b * c.N + (s >> 2)) * c.nd + (type - c.tdip);
-  double mu[3] = {0, 0, 0};
-  if ((MODE == FD_D || MODE == FD_QD) && has_d)
-    for (int k = 0; k < 3; ++k) mu[k] = dip[dslot * 3 + k];
-  const double q = (MODE == FD_QD) ? site[(size_t)b * S + s].q : 0.0;
-  // e^{i 2 pi z/L}; with lmax = 0 every column holds one k and no step is taken
-  const R2 zstep =
-      c.lmax >= 1 ? lds_tab[(c.hmax + c.kmax + 3) * FD_SB + lane] : Vec<R>::two(1.0, 0.0);
-  const double *sq = Sq + (size_t)b * c.nk * 2, *sm = Sm + (size_t)b * c.nk * 2;
-  double e0 = 0, e1 = 0, e2 = 0, ph = 0;
-  for (int col = g; col < c.ncol; col += CG) {
-    const int4 cl = cols[col];
-    const int k0 = colk[col];
-    R2 x = lds_tab[cl.x * FD_SB + lane];
-    R2 y = lds_tab[(c.hmax + 1 + abs(cl.y)) * FD_SB + lane];
-    R2 z = lds_tab[(c.hmax + c.kmax + 2 + abs(cl.z)) * FD_SB + lane];
-    if (cl.y < 0) y.y = -y.y;
-    if (cl.z < 0) z.y = -z.y;
-    R ck, sk;
-    phase_from(x, y, z, ck, sk);
-    const double kx = kv[k0].x, ky = kv[k0].y;
-    // column sums of t and kz t (t carries the sign of each mode's field)
-    R at = 0.0, az = 0.0;
-    // FD_QD dipole sites: k.mu = (kx mux + ky muy) + kz muz
-    const double dxy = (MODE == FD_QD) ? kx * mu[0] + ky * mu[1] : 0.0;
-#pragma unroll 4
-    for (int i = 0; i < cl.w; ++i) {
-      const int k = k0 + i;
-      if (KL) {
-        const R4 q4 = kd[k];  // w Re S, w Im S, kz, w
-        if (MODE == FD_Q) {
-          const R t = ck * q4.y - sk * q4.x;
-          at += t;
-          az += q4.z * t;
-          ph += ck * q4.x + sk * q4.y;
-        } else if (MODE == FD_D) {
-          const R t = ck * q4.y - sk * q4.x;
-          at += t;
-          az += q4.z * t;
-        } else {
-          R t = 0.0;
-          if (has_q) {
-            t = -(q * (ck * q4.y - sk * q4.x));
-            ph += ck * q4.x + sk * q4.y;
-          }
-          if (has_d) {
-            const double2 qq = kq[k];
-            const double dk = dxy + q4.z * mu[2];
-            t += dk * (ck * qq.x + sk * qq.y);
-          }
-          at += t;
-          az += q4.z * t;
-        }
-        const R nc = ck * zstep.x - sk * zstep.y;
-        sk = sk * zstep.x + ck * zstep.y;
-        ck = nc;
-        continue;
-      }
-      const double4 kk = kv[k];  // kx, ky, kz, 4 pi A_k / V
-      const R kw = kk.w, kz = kk.z;
-      if (MODE == FD_Q) {
-        const double re = sq[2 * k], im = sq[2 * k + 1];
-        const double t = kk.w * (ck * im - sk * re);
-        at += t;
-        az += kk.z * t;
-        ph += kk.w * (ck * re + sk * im);
-      } else if (MODE == FD_D) {
-        const R re = sm[2 * k], im = sm[2 * k + 1];
-        const R t = kw * (ck * im - sk * re);
-        at += t;
-        az += kz * t;
-      } else {
-        const double rqm = sm[2 * k], iqm = sm[2 * k + 1];
-        double t = 0.0;
-        if (has_q) {
-          t = -(q * kk.w * (ck * iqm - sk * rqm));
-          ph += kk.w * (ck * rqm + sk * iqm);
-        }
-        if (has_d) {
-          const double rqqm = sq[2 * k] + rqm;
-          const double iqqm = sq[2 * k + 1] + iqm;
-          const double dk = dxy + kk.z * mu[2];
-          t += dk * kk.w * (ck * rqqm + sk * iqqm);
-        }
-        at += t;
-        az += kk.z * t;
-      }
-      // advance the phase to the next kz of the column
-      const R nc = ck * zstep.x - sk * zstep.y;
-      sk = sk * zstep.x + ck * zstep.y;
-      ck = nc;
-    }
-    e0 -= kx * (double)at;
-    e1 -= ky * (double)at;
-    e2 -= (double)az;
-  }
-  // combine the CG column groups of each site in a fixed order
-  __syncthreads();
-  double *red = reinterpret_cast<double *>(lds_tab);  // [CG][4][64]
-  red[(g * 4 + 0) * FD_SB + lane] = e0;
-  red[(g * 4 + 1) * FD_SB + lane] = e1;
-  red[(g * 4 + 2) * FD_SB + lane] = e2;
-  red[(g * 4 + 3) * FD_SB + lane] = ph;
-  __syncthreads();
-  if (g != 0 || !valid) return;
-  for (int w = 1; w < CG; ++w) {
-    e0 += red[(w * 4 + 0) * FD_SB + lane];
-    e1 += red[(w * 4 + 1) * FD_SB + lane];
-    e2 += red[(w * 4 + 2) * FD_SB + lane];
-    ph += red[(w * 4 + 3) * FD_SB + lane];
-  }
-  const size_t ss = (size_t)b * S + s;
-  if (MODE == FD_Q || MODE == FD_QD) {
-    // into their own buffers (kE, kphi): the consumer adds them to the
-    // real-space sums, which the pair kernels may be forming meanwhile
-    double *ko = MODE == FD_Q ? Efq : dR;
-    ko[ss * 3 + 0] = e0;
-    ko[ss * 3 + 1] = e1;
-    ko[ss * 3 + 2] = e2;
-    phi[ss] = has_q ? ph : 0.0;
-  } else {
-    const double e[3] = {e0, e1, e2};
-    const double om = c.sor, pol = c.polar[type];
-    double d2 = 0.0;
-    for (int k = 0; k < 3; ++k) {
-      const double etot = (Efd[dslot * 3 + k] + e[k]) + Efq[ss * 3 + k] + c.fac_dd * mu[k];
-      const double nm = (1.0 - om) * mu[k] + om * pol * etot;
-      const double df = nm - (iter == 1 ? 0.0 : mu[k]);
-      d2 += df * df;
-      dip[dslot * 3 + k] = nm;
-      if (c.mixed && iter <= c.maxiter) dip_prev[dslot * 3 + k] = mu[k];
-    }
-    diff2[(size_t)b * c.N * c.nd + m] = d2;
-  }
-}
-
-// Shared memory of k_field: the phase tables (reused for the CG-way
-// reduction; fd_tab_d2 double2 slots cover both), then the staged k data.
-static size_t field_lds(const SysConst &c, int mode, bool kl, bool f32 = false) {
-  return sizeof(double2) * c.fd_tab_d2 +
-         (kl ? c.nk * ((f32 ? sizeof(float4) : sizeof(double4)) +
-                       (mode == FD_QD ? sizeof(double2) : 0))
-             : 0);
-}
-
-
-
-
 // ---------------------------------------------------------------------------
 // After the charge pass: gradient of the charge energy, Uelec partials and the
 // initial induced dipoles (pot_ttm.f90:273-297).  One thread per (bead, molecule).
@@ -2896,174 +2231,6 @@ void launch_pair_qq(const Group &g, hipStream_t s) {
         if (v == 1) hipLaunchKernelGGL(k_pair_qq_partner<3>, grid, dim3(256), 0, s, g.d, m);
         else hipLaunchKernelGGL(k_pair_qq_partner<2>, grid, dim3(256), 0, s, g.d, m);
       });
-}
-
-void launch_tables(const Group &g, hipStream_t s) {
-  launch_over(
-      g, [](const SysConst &c, const MDConst &) { return Plan{0, idiv(4 * c.N, 256), c.P, 1, 0}; },
-      [&](int, dim3 grid, const BlockMap &m, size_t) {
-        hipLaunchKernelGGL(k_tables, grid, dim3(256), 0, s, g.d, m);
-      });
-}
-
-// Structure factor `mode`.  Variant: bit 0 the column kernel (else one k per
-// lane), bits 1-3 its segment-length bucket, bit 4 two lane sets per block,
-// bits 5.. the lane count of a set in units of 64.
-static const int KZ_BUCKET[6] = {4, 8, 12, 16, 24, 32};
-
-template <int MODE, int KZ, class R>
-static void launch_sfac_col_v(bool split, int threads, dim3 grid, const BlockMap &m, size_t lds,
-                              int stale, const Group &g, hipStream_t s) {
-  if (split) hipLaunchKernelGGL((k_sfac_col<MODE, KZ, 2, R>), grid, dim3(2 * threads), lds, s, g.d, m, stale);
-  else hipLaunchKernelGGL((k_sfac_col<MODE, KZ, 1, R>), grid, dim3(threads), lds, s, g.d, m, stale);
-}
-
-template <int MODE, class R>
-static void launch_sfac_kz(int v, dim3 grid, const BlockMap &m, size_t lds, int stale,
-                           const Group &g, hipStream_t s) {
-  const bool split = (v & 16) != 0;
-  const int threads = ((v >> 5) & 7) * 64;
-  switch ((v >> 1) & 7) {
-    case 0: launch_sfac_col_v<MODE, 4, R>(split, threads, grid, m, lds, stale, g, s); break;
-    case 1: launch_sfac_col_v<MODE, 8, R>(split, threads, grid, m, lds, stale, g, s); break;
-    case 2: launch_sfac_col_v<MODE, 12, R>(split, threads, grid, m, lds, stale, g, s); break;
-    case 3: launch_sfac_col_v<MODE, 16, R>(split, threads, grid, m, lds, stale, g, s); break;
-    case 4: launch_sfac_col_v<MODE, 24, R>(split, threads, grid, m, lds, stale, g, s); break;
-    default: launch_sfac_col_v<MODE, 32, R>(split, threads, grid, m, lds, stale, g, s); break;
-  }
-}
-
-// sel (SF_D): SFAC_ITER, the SOR iterations (not the dense systems; the mixed
-// form's in FP32, variant bit 8), SFAC_REFINE the mixed form's FP64
-// refinement step, SFAC_STALE the dense systems' last input.
-// part: 1 the chunk partial sums, 2 their fixed-order reduction, 3 both.
-template <int MODE>
-static void launch_sfac_mode(const Group &g, int sel, int part, hipStream_t s) {
-  constexpr int NV = MODE == SF_V ? 6 : 2;
-  const int stale = MODE == SF_D && sel == SFAC_STALE ? 1 : 0;
-  auto plan = [&](const SysConst &c) {
-        if (MODE != SF_Q && !is_ttm(c)) return Plan{-1, 0, 0, 0, 0};
-        if (sel == SFAC_REFINE && !c.mixed) return Plan{-1, 0, 0, 0, 0};
-        if (MODE == SF_D && (c.dense != 0) != (sel == SFAC_STALE)) return Plan{-1, 0, 0, 0, 0};
-        const bool f32 = MODE == SF_D && c.mixed && sel == SFAC_ITER;
-        int nch, sc, scp;
-        sfac_chunking(c, MODE, sfac_sites(c, MODE), nch, sc, scp);
-        const size_t lds = sfac_lds(c, MODE, sc, scp, f32);
-        int kzb = -1;
-        for (int i = 0; i < 6; ++i)
-          if (kzb < 0 && c.segmax <= KZ_BUCKET[i]) kzb = i;
-        const bool col = c.sf_kind == 1 && (MODE != SF_V || c.sfv_col) && lds <= 64 * 1024 && kzb >= 0;
-        if (!col) return Plan{0, idiv(c.nk, 256), nch, c.P, sfac_lds(c, MODE, sc, scp)};
-        const int threads = std::min(256, idiv(c.nseg, 64) * 64);
-        // two lane sets per block where the second set's sums fit beside the tables
-        const size_t red = (f32 ? sizeof(float) : sizeof(double)) *
-                           ((size_t)NV * KZ_BUCKET[kzb] * threads + 4);
-        const bool split = MODE != SF_V && c.sf_split && lds + red <= 96 * 1024;
-        return Plan{1 | (kzb << 1) | (split ? 16 : 0) | ((threads / 64) << 5) | (f32 ? 256 : 0),
-                    idiv(c.nseg, threads), nch, c.P, split ? lds + red : lds};
-  };
-  if (part & 1) launch_over(
-      g, [&](const SysConst &c, const MDConst &) { return plan(c); },
-      [&](int v, dim3 grid, const BlockMap &m, size_t lds) {
-        if (!(v & 1)) {
-          hipLaunchKernelGGL((k_sfac_k<MODE>), grid, dim3(256), lds, s, g.d, m, stale);
-          return;
-        }
-        if constexpr (MODE == SF_D) {
-          if (v & 256) {
-            launch_sfac_kz<MODE, float>(v, grid, m, lds, stale, g, s);
-            return;
-          }
-        }
-        launch_sfac_kz<MODE, double>(v, grid, m, lds, stale, g, s);
-      });
-  if (part & 2) launch_over(
-      g,
-      [&](const SysConst &c, const MDConst &) {
-        if (plan(c).variant < 0) return Plan{-1, 0, 0, 0, 0};
-        return Plan{0, idiv((long)NV * c.nk, 256), c.P, 1, 0};
-      },
-      [&](int, dim3 grid, const BlockMap &m, size_t) {
-        hipLaunchKernelGGL(k_sfac_reduce, grid, dim3(256), 0, s, g.d, m, MODE, stale);
-      });
-}
-
-void launch_sfac(const Group &g, int mode, hipStream_t s, int sel, int part) {
-  if (mode == SF_Q) launch_sfac_mode<SF_Q>(g, SFAC_ITER, part, s);
-  else if (mode == SF_D) launch_sfac_mode<SF_D>(g, sel, part, s);
-  else launch_sfac_mode<SF_V>(g, SFAC_ITER, part, s);
-}
-
-// The FP32 dipole field of the mixed form's SOR iterations (variant bits as
-// launch_field_mode's).
-static void launch_field_f32(int v, bool kl, dim3 grid, const BlockMap &m, size_t lds, int iter,
-                             const Group &g, hipStream_t s) {
-#define PIMD_FIELD32(ML, CG)                                                                      \
-  if (kl) hipLaunchKernelGGL((k_field<FD_D, ML, CG, true, float>), grid, dim3(64 * CG), lds, s, g.d, m, iter); \
-  else hipLaunchKernelGGL((k_field<FD_D, ML, CG, false, float>), grid, dim3(64 * CG), lds, s, g.d, m, iter)
-  switch (v & 7) {
-    case 0: PIMD_FIELD32(2, 4); break;
-    case 1: PIMD_FIELD32(3, 4); break;
-    case 2: PIMD_FIELD32(2, 8); break;
-    case 3: PIMD_FIELD32(3, 8); break;
-    case 4: PIMD_FIELD32(2, 16); break;
-    default: PIMD_FIELD32(3, 16); break;
-  }
-#undef PIMD_FIELD32
-}
-
-// Reciprocal-space field `mode`.  Variant: bit 0 TTM3-F site sets (the
-// fixed-charge models share them), bits 1-2 the column groups (4, 8, 16),
-// bit 3 k data staged in LDS.  sel_mixed: only the mixed-form replicas.
-template <int MO>
-static void launch_field_mode(const Group &g, int iter, bool sel_mixed, hipStream_t s) {
-  launch_over(
-      g,
-      [&](const SysConst &c, const MDConst &) {
-        if ((MO != FD_Q && !is_ttm(c)) || (sel_mixed && !c.mixed) || (MO == FD_D && c.dense))
-          return Plan{-1, 0, 0, 0, 0};
-        const int ML = c.model == 2 ? 2 : 3;
-        const int M = MO == FD_D ? c.nd * c.N : (ML == 2 ? 4 * c.N : 3 * c.N);
-        // as many column groups as the columns keep busy: more resident waves hide
-        // the table and structure-factor reads (512 H2O x 32 beads: the charge
-        // fields at 16 groups instead of 8 take 1.68 instead of 1.73 ms per force
-        // call)
-        int cg = c.fd_cg;
-        if (cg == 0) cg = c.ncol < 8 ? 4 : c.ncol < 16 ? 8 : 16;
-        const int cgi = cg == 4 ? 0 : cg == 8 ? 1 : 2;
-        // the mixed form's SOR iterations in FP32 (its refinement, iter < 0, in FP64)
-        const bool f32 = MO == FD_D && c.mixed && iter > 0;
-        const bool kl = c.fd_klds && field_lds(c, MO, true, f32) <= 160 * 1024;
-        return Plan{(ML == 3 ? 1 : 0) | (cgi << 1) | (kl ? 8 : 0) | (f32 ? 16 : 0), idiv(M, FD_SB),
-                    c.P, 1, field_lds(c, MO, kl, f32)};
-      },
-      [&](int v, dim3 grid, const BlockMap &m, size_t lds) {
-        const bool kl = (v & 8) != 0;
-        if constexpr (MO == FD_D) {
-          if (v & 16) {
-            launch_field_f32(v, kl, grid, m, lds, iter, g, s);
-            return;
-          }
-        }
-#define PIMD_FIELD(ML, CG)                                                                     \
-  if (kl) hipLaunchKernelGGL((k_field<MO, ML, CG, true>), grid, dim3(64 * CG), lds, s, g.d, m, iter); \
-  else hipLaunchKernelGGL((k_field<MO, ML, CG, false>), grid, dim3(64 * CG), lds, s, g.d, m, iter)
-        switch (v & 7) {
-          case 0: PIMD_FIELD(2, 4); break;
-          case 1: PIMD_FIELD(3, 4); break;
-          case 2: PIMD_FIELD(2, 8); break;
-          case 3: PIMD_FIELD(3, 8); break;
-          case 4: PIMD_FIELD(2, 16); break;
-          default: PIMD_FIELD(3, 16); break;
-        }
-#undef PIMD_FIELD
-      });
-}
-
-void launch_field(const Group &g, int mode, int iter, hipStream_t s, bool sel_mixed) {
-  if (mode == FD_Q) launch_field_mode<FD_Q>(g, iter, sel_mixed, s);
-  else if (mode == FD_D) launch_field_mode<FD_D>(g, iter, sel_mixed, s);
-  else launch_field_mode<FD_QD>(g, iter, sel_mixed, s);
 }
 
 void launch_post_qq(const Group &g, hipStream_t s) {
