@@ -83,12 +83,12 @@ __global__ __launch_bounds__(256) void k_nm_evolve(const Rep *__restrict__ reps,
 // The same transforms on FP64 matrix cores.  v_mfma_f64_16x16x4_f64 adds
 // A (16 x 4) B (4 x 16) to D (16 x 16) across one wave: lane l holds
 // A[l % 16][l / 16] and B[l / 16][l % 16], and D[l / 16 + 4 i][l % 16] in
-// element i (rows interleaved over the four lane groups).  A block is one wave and 16 (atom, component) columns; P is
-// padded with zeros to PT (a multiple of 16) modes and beads, C sits in LDS
-// with rows padded by one double (no bank conflicts between the 16 rows a
-// wave reads at once), and the mode-space slab goes through LDS between the
-// two transforms (the D layout of one product is not the B layout of the
-// next).  Products are summed in the matrix cores' order, not the
+// element i (rows interleaved over the four lane groups).  A block takes 16
+// (atom, component) columns; P is padded with zeros to PT (a multiple of 16)
+// modes and beads, and the mode-space slab goes through LDS between the two
+// transforms (the D layout of one product is not the B layout of the next).
+// The Langevin form is one wave, with C in LDS, rows padded by one double (no
+// bank conflicts between the 16 rows a wave reads at once).  Products are summed in the matrix cores' order, not the
 // reference's; the difference is rounding.
 typedef double v4d __attribute__((ext_vector_type(4)));
 
@@ -137,76 +137,75 @@ __device__ __forceinline__ void mfma_bwd(const double *Cs, const double *Ys, v4d
   }
 }
 
+// The free ring-polymer step: a block takes 16 columns of RR and PP in two
+// waves per 16 modes, one for positions and one for momenta, whose operands
+// (its rows and columns of C, the 16 columns of its array) all load at once
+// from global memory; the mode amplitudes meet in LDS, where each wave forms
+// the propagated ones as it reads them.  Bound by latency
+// (512 H2O x 32 beads: one wave and C staged in LDS / now, 12.5 / 9.6 us).
 template <int PT>
-__global__ __launch_bounds__(64) void k_nm_evolve_mfma(const Rep *__restrict__ reps, BlockMap bm,
-                                                       int kick, int kick2) {
+__global__ __launch_bounds__(8 * PT) void k_nm_evolve_mfma(const Rep *__restrict__ reps, BlockMap bm,
+                                                           int kick, int kick2) {
   constexpr int KS = PT / 4, RT = PT / 16;
-  __shared__ double Cs[PT * (PT + 1)], Yr[PT * 17], Yp[PT * 17];
+  __shared__ double Y[2][PT * 17];
   const Blk bk = block_of(bm);
   const Rep &R = reps[bk.r];
   const int P = R.c.P, natoms = 3 * R.c.N;
   const double *__restrict__ Cg = R.b.C, *__restrict__ A = R.b.A, *__restrict__ msf = R.b.msf;
   const double *__restrict__ masses = R.b.masses;
-  double *RR = R.b.RR, *PP = R.b.PP;
   const int ncols = natoms * 3;
   const size_t stride = (size_t)ncols;
-  const int j = threadIdx.x & 15, q = threadIdx.x >> 4;
-  const int col = bk.x * NM_TILE + j;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int rt = wave % RT;      // this wave's 16 modes, later its 16 beads
+  const bool mom = wave >= RT;   // momenta or positions
+  const int j = lane & 15, q = lane >> 4;
+  const int col = bk.x * NM_TILE + j, row = rt * 16 + j;
   const bool vc = col < ncols;
-  stage_C<PT>(Cs, Cg, P);
-  double xr[KS], xp[KS];
+  double *X = mom ? R.b.PP : R.b.RR;
+  double x[KS], cf[KS], cb[KS];
 #pragma unroll
   for (int kk = 0; kk < KS; ++kk) {
     const int bead = kk * 4 + q;
-    const bool in = vc && bead < P;
+    const bool in = vc && bead < P, inc = bead < P && row < P;
     const size_t o = (size_t)bead * stride + col;
-    xr[kk] = in ? RR[o] : 0.0;
-    double p = in ? PP[o] : 0.0;
+    x[kk] = in ? X[o] : 0.0;
+    cf[kk] = inc ? Cg[row * P + bead] : 0.0;
+    cb[kk] = inc ? Cg[bead * P + row] : 0.0;
     // the half kicks before the step (MD.f90:49), rounded as k_kick does
-    if (in) p = kicked(R, kick2, o, kicked(R, kick, o, p));
-    xp[kk] = p;
+    if (mom && in) x[kk] = kicked(R, kick2, o, kicked(R, kick, o, x[kk]));
   }
+  v4d y = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int kk = 0; kk < KS; ++kk) y = mfma_f64(cf[kk], x[kk], y);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) Y[mom][(rt * 16 + q + 4 * i) * 17 + j] = y[i];
   __syncthreads();
-  v4d yr[RT], yp[RT];
-  mfma_fwd<PT>(Cs, xr, yr);
-  mfma_fwd<PT>(Cs, xp, yp);
   // exact harmonic propagator of each mode (NormalModes.f90:34-63)
   const double m = vc ? masses[col / 3] : 1.0;
+  v4d out = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int mode = rt * 16 + q + 4 * i;
-      double nr = 0.0, np = 0.0;
-      if (mode < P) {
-        const double vr = yr[rt][i], vp = yp[rt][i];
-        nr = A[mode] * vr + A[P + mode] * vp / (m * msf[mode]);
-        np = A[2 * P + mode] * m * msf[mode] * vr + A[3 * P + mode] * vp;
-      }
-      Yr[mode * 17 + j] = nr;
-      Yp[mode * 17 + j] = np;
+  for (int kk = 0; kk < KS; ++kk) {
+    const int mode = kk * 4 + q;
+    double v = 0.0;
+    if (mode < P) {
+      const double vr = Y[0][mode * 17 + j], vp = Y[1][mode * 17 + j];
+      v = mom ? A[2 * P + mode] * m * msf[mode] * vr + A[3 * P + mode] * vp
+              : A[mode] * vr + A[P + mode] * vp / (m * msf[mode]);
     }
-  __syncthreads();
-  v4d orr[RT], opp[RT];
-  mfma_bwd<PT>(Cs, Yr, orr);
-  mfma_bwd<PT>(Cs, Yp, opp);
+    out = mfma_f64(cb[kk], v, out);
+  }
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int bead = rt * 16 + q + 4 * i;
-      if (vc && bead < P) {
-        RR[(size_t)bead * stride + col] = orr[rt][i];
-        PP[(size_t)bead * stride + col] = opp[rt][i];
-      }
-    }
+  for (int i = 0; i < 4; ++i) {
+    const int bead = rt * 16 + q + 4 * i;
+    if (vc && bead < P) X[(size_t)bead * stride + col] = out[i];
+  }
 }
 
 // PT: P rounded up to a multiple of 16 (P <= 64).
 static int nm_pt(int P) { return ((P + 15) / 16) * 16; }
 
 // The free ring-polymer step runs on the FP64 matrix cores unless
-// PIMD_NM_MFMA=0 (13 us against 21 us at 512 x 32).  The Langevin step keeps
+// PIMD_NM_MFMA=0 (9.6 us against 21 us at 512 x 32).  The Langevin step keeps
 // the FMA slabs unless PIMD_LANGEVIN_MFMA=1: its time goes to the normal
 // deviates, which the slab layout spreads over twice as many lanes (18 us
 // against 20 us).
@@ -231,10 +230,10 @@ void launch_nm_evolve(const Group &g, hipStream_t s, int kick, int kick2, bool w
         },
         [&](int pt, dim3 grid, const BlockMap &m, size_t) {
           switch (pt) {
-            case 16: hipLaunchKernelGGL(k_nm_evolve_mfma<16>, grid, dim3(64), 0, s, g.d, m, kick, kick2); break;
-            case 32: hipLaunchKernelGGL(k_nm_evolve_mfma<32>, grid, dim3(64), 0, s, g.d, m, kick, kick2); break;
-            case 48: hipLaunchKernelGGL(k_nm_evolve_mfma<48>, grid, dim3(64), 0, s, g.d, m, kick, kick2); break;
-            default: hipLaunchKernelGGL(k_nm_evolve_mfma<64>, grid, dim3(64), 0, s, g.d, m, kick, kick2); break;
+            case 16: hipLaunchKernelGGL(k_nm_evolve_mfma<16>, grid, dim3(128), 0, s, g.d, m, kick, kick2); break;
+            case 32: hipLaunchKernelGGL(k_nm_evolve_mfma<32>, grid, dim3(256), 0, s, g.d, m, kick, kick2); break;
+            case 48: hipLaunchKernelGGL(k_nm_evolve_mfma<48>, grid, dim3(384), 0, s, g.d, m, kick, kick2); break;
+            default: hipLaunchKernelGGL(k_nm_evolve_mfma<64>, grid, dim3(512), 0, s, g.d, m, kick, kick2); break;
           }
         });
     return;
