@@ -188,8 +188,11 @@ __host__ __device__ inline void sfac_chunking(const SysConst &c, int mode, int &
   const int M = sfac_sites(c, mode);
   const int cap = sfac_cap(c), pref = mode == SF_Q ? c.sf_sites + c.sf_sites / 2 : c.sf_sites;
   const int sites = pref < cap ? pref : cap;
-  const int want = (M + sites - 1) / sites;
-  nch = want < c.sf_chunks_max ? want : c.sf_chunks_max;
+  const int want = (M + sites - 1) / sites, fit = (M + cap - 1) / cap;
+  // SF_V holds three times the values per chunk: half as many chunks at most
+  int most = mode == SF_V ? c.sf_chunks_max / 2 : c.sf_chunks_max;
+  if (most < fit) most = fit;
+  nch = want < most ? want : most;
   if (nch < 1) nch = 1;
   sc = ((M + nch - 1) / nch + 7) / 8 * 8;
   if (sc < 8) sc = 8;
@@ -406,11 +409,12 @@ static size_t sfac_lds(const SysConst &c, int mode, int sc, int scp, bool f32) {
 // Reciprocal-space fields at each site.  A block holds SG groups of 32 sites
 // (two tiles of 16) of one bead and CG column groups, one wave for each pair;
 // a wave takes every CG-th tile of 16 columns (the waves of other site groups
-// read the same operands at about the same time, from the cache next to the CU): U, V (and, for FD_QD at dipole sites, U, V, W of
-// the total structure factor) of 16 columns x 32 sites are one matrix product
-// each over the (cos, sin) of the tile's |kz|, with the operands from
-// k_sfac_reduce read in lane order and the sites' phases from LDS.  Lane l
-// then holds 4 columns of site l % 16 of each tile and adds their fields.
+// read the same operands at about the same time, from the cache next to the
+// CU): U, V (and, for FD_QD at dipole sites, U, V, W of the total structure
+// factor) of 16 columns x 32 sites are one matrix product each over the (cos,
+// sin) of the tile's |kz|, with the operands from k_sfac_reduce read in lane
+// order and the sites' phases from LDS.  Lane l then holds 4 columns of site
+// l % 16 of each tile and adds their fields.
 // The waves' and lane groups' parts are added in a fixed order.
 //   FD_Q : Efq and phi from the charge structure factor (ewald.f90:45-49)
 //   FD_D : Efd from the dipole structure factor (ewald.f90:114-117), then the
