@@ -423,9 +423,10 @@ struct HostTables {
 // The most site pairs (beads x sites^2) for which the dense dipole matrix is
 // taken by launches.  Its cost grows with the pairs (forming it, then 72 bytes
 // of matrix per pair and iteration), the passes' mostly with the launches.
-// Force call, passes against matrix: TTM3-F 128 x 32 (524k pairs) 789 / 566 us,
-// 512 x 4 (1049k) 682 / 641, 256 x 16 (1049k) 816 / 733, 256 x 32 (2097k)
-// 975 / 1058; TTM2.1-F 128 x 8 (1180k) 835 / 688, 128 x 32 (4719k) 1132 / 1924.
+// Force call, passes against matrix: TTM3-F 128 x 32 (524k pairs) 609 / 472 us,
+// 512 x 4 (1049k) 607 / 588, 256 x 16 (1049k) 656 / 653; TTM2.1-F 64 x 16
+// (590k) 535 / 414, 64 x 32 (1180k) 600 / 577, 128 x 8 (1180k) 654 / 620.
+// Beyond, the matrix no longer stays in the caches: 256 x 32 (2097k) lost.
 constexpr long DENSE_MAX_PAIRS = 1200000;
 
 // The k-vector tables, kz-columns and segments and the default launch shapes

@@ -215,7 +215,8 @@ __host__ __device__ inline void sfac_chunking(const SysConst &c, int mode, int &
 // launch; 512 H2O x 32 beads, one kz-segment of 4 per lane / now: SF_D 16.8 /
 // 13.0 us (4.3 us of it matrix time), SF_Q 43 / 22.7 (6.4), SF_V 30 / 18.7.
 template <int MODE, class R>
-__global__ __launch_bounds__(1024) void k_sfac(const Rep *__restrict__ reps, BlockMap bm, int stale) {
+__global__ __launch_bounds__(1024) void k_sfac(const Rep *__restrict__ reps, BlockMap bm, int stale,
+                                               int groups) {
   using R2 = typename Mf<R>::v2;
   using V4 = typename Mf<R>::v4;
   constexpr int SET = MODE == SF_Q ? SET_CHG : SET_DIP;
@@ -257,7 +258,7 @@ __global__ __launch_bounds__(1024) void k_sfac(const Rep *__restrict__ reps, Blo
   const int lane = threadIdx.x & 63, n = lane & 15, q = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
   const double tpz = TWOPI * c.boxi[2];
-  for (int task = wave; task < c.sf_ntask; task += nw) {
+  for (int task = bk.z * nw + wave; task < c.sf_ntask; task += groups * nw) {
     const int tk = Rp.b.sftask[task], ct = tk & 0xffff, l0 = 8 * (tk >> 16);
     const ColRec cr = Rp.b.colrec[ct * 16 + n];
     const R2 *px = tabs + cr.rx * scp + q;
@@ -406,12 +407,12 @@ static size_t sfac_lds(const SysConst &c, int mode, int sc, int scp, bool f32) {
   return 2 * r * c.T * scp + r * sc * (mode == SF_Q ? 1 : 3);
 }
 
-// Reciprocal-space fields at each site.  A block holds SG groups of 32 sites
-// (two tiles of 16) of one bead and CG column groups, one wave for each pair;
+// Reciprocal-space fields at each site.  A block holds SG groups of NT tiles
+// of 16 sites of one bead and CG column groups, one wave for each pair;
 // a wave takes every CG-th tile of 16 columns (the waves of other site groups
 // read the same operands at about the same time, from the cache next to the
 // CU): U, V (and, for FD_QD at dipole sites, U, V, W of the total structure
-// factor) of 16 columns x 32 sites are one matrix product each over the (cos,
+// factor) of 16 columns x 16 NT sites are one matrix product each over the (cos,
 // sin) of the tile's |kz|, with the operands from k_sfac_reduce read in lane
 // order and the sites' phases from LDS.  Lane l then holds 4 columns of site
 // l % 16 of each tile and adds their fields.
@@ -426,28 +427,34 @@ static size_t sfac_lds(const SysConst &c, int mode, int sc, int scp, bool f32) {
 // Bound by the FP64 matrix rate and, in the SOR iterations, the launch:
 // 512 H2O x 32 beads, one site per lane walking the columns / now: FD_D 12.4 /
 // 10.5 us (3.3 us of it matrix time), FD_Q 39 / 25 (9.8), FD_QD 64 / 47 (15).
-constexpr int FD_SB = 32;     // sites per group
+constexpr int FD_SB = 32;     // sites per group of two tiles
 constexpr int FD_WAVES = 8;   // waves per block at most
-// Site groups per block and column groups of one field launch over M sites.
+// Tiles per site group, site groups per block and column groups of one field
+// launch over M sites.  Small systems take one tile to a group, half the work
+// per wave (with the structure factors' rounds in blocks of their own, one
+// bead of 32 H2O 267 -> 250 us per call, 32 beads 373 -> 359).
 // Column groups until the device has two waves per SIMD; blocks of 4 waves,
 // of which a CU holds three, and of 8 only where every CU gets at most one
 // block.  Of 4, 2 and 1 site groups the most that leave few CUs idle at the
 // end.  (Waves per block 4 / 8: FD_D of TTM2.1-F 128 x 32 10.8 / 12.9 us, a
 // whole call of 32 H2O x 32 beads 376 / 369 us.)
-__host__ inline void field_groups(const SysConst &c, int M, int &sg, int &cg) {
-  const long ng = (long)c.P * ((M + FD_SB - 1) / FD_SB);
+__host__ inline void field_groups(const SysConst &c, int M, int &nt, int &sg, int &cg) {
+  long ng = (long)c.P * ((M + FD_SB - 1) / FD_SB);
+  nt = ng <= 128 ? 1 : 2;
+  const int sb = 16 * nt;
+  ng = (long)c.P * ((M + sb - 1) / sb);
   const int most = ng <= 256 ? FD_WAVES : 4;
   cg = 1;
   while (cg < most && cg < col_tiles(c) && ng * cg < 2048) cg *= 2;
   if (c.fd_cg) cg = c.fd_cg < FD_WAVES ? c.fd_cg : FD_WAVES;
   auto idle = [&](int s) {
-    const long nb = (long)c.P * ((M + s * FD_SB - 1) / (s * FD_SB));
+    const long nb = (long)c.P * ((M + s * sb - 1) / (s * sb));
     return 1.0 - (double)nb / ((nb + 255) / 256 * 256);
   };
   for (sg = cg < 4 ? 4 / cg : 1; sg > 1; sg /= 2)
     if (idle(sg) <= 0.1 || idle(sg) <= idle(1)) break;
 }
-template <int MODE, int MODEL, class R>
+template <int MODE, int MODEL, class R, int NT>
 __global__ __launch_bounds__(64 * FD_WAVES, MODE == FD_QD ? 2 : 3) void k_field(const Rep *__restrict__ reps, BlockMap bm,
                                                          int iter, int SG) {
   using R2 = typename Mf<R>::v2;
@@ -468,8 +475,9 @@ __global__ __launch_bounds__(64 * FD_WAVES, MODE == FD_QD ? 2 : 3) void k_field(
   const int lane = threadIdx.x & 63, n = lane & 15, q = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = wave / SG, CG = (blockDim.x >> 6) / SG;
-  const int SB = SG * FD_SB, TS = phase_row(SB);
-  const int M = set_size(c, SET), S = 4 * c.N, mbase = bk.x * SB, sbase = (wave % SG) * FD_SB;
+  constexpr int FS = 16 * NT;  // sites per group
+  const int SB = SG * FS, TS = phase_row(SB);
+  const int M = set_size(c, SET), S = 4 * c.N, mbase = bk.x * SB, sbase = (wave % SG) * FS;
   int RS;
   const R2 *__restrict__ tb = set_rows<R, SET>(Rp, b, RS);
   // one row more than the tables': the last step may reach kz = lmax + 1,
@@ -479,11 +487,12 @@ __global__ __launch_bounds__(64 * FD_WAVES, MODE == FD_QD ? 2 : 3) void k_field(
     tabs[row * TS + l] = tb[(size_t)min(row, c.T - 1) * RS + row_index<SET>(c, min(mbase + l, M - 1))];
   }
   // charge and dipole of this lane's site of each tile
-  double qs[2] = {0, 0}, mu[2][3] = {{0, 0, 0}, {0, 0, 0}};
+  double qs[NT], mu[NT][3];
+  for (int t = 0; t < NT; ++t) qs[t] = mu[t][0] = mu[t][1] = mu[t][2] = 0.0;
   bool any_q = true, any_d = false;
   if (MODE == FD_QD) {
     bool hq = false, hd = false;
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < NT; ++t) {
       const int s = set_site(c, SET, min(mbase + sbase + 16 * t + n, M - 1)), type = s & 3;
       if (type != 0) {
         qs[t] = site[(size_t)b * S + s].q;
@@ -507,8 +516,8 @@ __global__ __launch_bounds__(64 * FD_WAVES, MODE == FD_QD ? 2 : 3) void k_field(
   // this lane's cos or sin row of the first step: kz = q / 2, then two on
   const R *pb = reinterpret_cast<const R *>(
                     tabs + (c.hmax + c.kmax + 2 + (q >> 1)) * TS + sbase + n) + (q & 1);
-  double e[2][4];  // field and potential at this lane's sites
-  for (int t = 0; t < 2; ++t) e[t][0] = e[t][1] = e[t][2] = e[t][3] = 0.0;
+  double e[NT][4];  // field and potential at this lane's sites
+  for (int t = 0; t < NT; ++t) e[t][0] = e[t][1] = e[t][2] = e[t][3] = 0.0;
   for (int ct = g; ct < nct; ct += CG) {
     // the columns are sorted by their reach along kz
     const int ks = kz_steps(rec[ct * 16].reach);
@@ -530,7 +539,7 @@ __global__ __launch_bounds__(64 * FD_WAVES, MODE == FD_QD ? 2 : 3) void k_field(
     auto gemm = [&](auto nc_tag, const R *w, auto &&done) {
       constexpr int NC = decltype(nc_tag)::value;
       const R *wp = w + wo * NC * 64 + lane;
-      V4 D[NC][2];
+      V4 D[NC][NT];
       R a[NC], an[NC];
       auto load = [&](R *to, int s) {
 #pragma unroll
@@ -539,11 +548,11 @@ __global__ __launch_bounds__(64 * FD_WAVES, MODE == FD_QD ? 2 : 3) void k_field(
       auto step = [&](int s, auto first_tag) {
         constexpr bool FIRST = decltype(first_tag)::value;
         const R *p = pb + (size_t)s * (4 * TS);
-        const R b0 = p[0], b1 = p[32];
+        const R b0 = p[0], b1 = NT == 2 ? p[32] : (R)0.0;
 #pragma unroll
         for (int v = 0; v < NC; ++v) {
           D[v][0] = Mf<R>::mma(a[v], b0, FIRST ? V4{0, 0, 0, 0} : D[v][0]);
-          D[v][1] = Mf<R>::mma(a[v], b1, FIRST ? V4{0, 0, 0, 0} : D[v][1]);
+          if constexpr (NT == 2) D[v][1] = Mf<R>::mma(a[v], b1, FIRST ? V4{0, 0, 0, 0} : D[v][NT - 1]);
         }
       };
       // the next step's operands in flight
@@ -559,7 +568,7 @@ __global__ __launch_bounds__(64 * FD_WAVES, MODE == FD_QD ? 2 : 3) void k_field(
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
+        for (int t = 0; t < NT; ++t) {
           const R2 x = px[i][16 * t];
           R2 y = py[i][16 * t];
           y.y = Mf<R>::flip(y.y, sg[i]);
@@ -596,7 +605,7 @@ __global__ __launch_bounds__(64 * FD_WAVES, MODE == FD_QD ? 2 : 3) void k_field(
   __syncthreads();
   double *red = reinterpret_cast<double *>(lds_raw);  // [CG][4][SB]
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int k = 0; k < (MODE == FD_D ? 3 : 4); ++k) {
       double v = e[t][k];
@@ -644,7 +653,9 @@ static int idiv(long a, long b) { return (int)((a + b - 1) / b); }
 // SFAC_STALE the dense systems' last input.  part: 1 the chunk sums, 2 their
 // reduction, 3 both.  Variant: bit 0 FP32, above it the waves per block: one
 // per task up to 16, beyond as few rounds of tasks as 16 waves need; an even
-// number, so that more replicas of a batch share launches.
+// number, so that more replicas of a batch share launches.  Small systems give
+// each round a block of its own (with one-tile site groups: one bead of 32
+// H2O 267 -> 250 us per call, 32 beads 373 -> 359).
 template <int MODE>
 static void launch_sfac_mode(const Group &g, int sel, int part, hipStream_t s) {
   const int stale = MODE == SF_D && sel == SFAC_STALE ? 1 : 0;
@@ -657,19 +668,22 @@ static void launch_sfac_mode(const Group &g, int sel, int part, hipStream_t s) {
     sfac_chunking(c, MODE, nch, sc, scp);
     const int rounds = std::max(1, idiv(c.sf_ntask, 16));
     const int waves = std::max(2, (idiv(c.sf_ntask, rounds) + 1) / 2 * 2);
-    return Plan{(f32 ? 1 : 0) | (waves << 1), nch, c.P, 1, sfac_lds(c, MODE, sc, scp, f32)};
+    const int groups = (long)nch * c.P <= 128 ? rounds : 1;
+    return Plan{(f32 ? 1 : 0) | (waves << 1) | (groups << 6), nch, c.P, groups,
+                sfac_lds(c, MODE, sc, scp, f32)};
   };
   if (part & 1)
     launch_over(
         g, [&](const SysConst &c, const MDConst &) { return plan(c); },
         [&](int v, dim3 grid, const BlockMap &m, size_t lds) {
-          const dim3 block(64 * (v >> 1));
+          const dim3 block(64 * ((v >> 1) & 31));
+          const int groups = v >> 6;
           if constexpr (MODE == SF_D)
             if (v & 1) {
-              hipLaunchKernelGGL((k_sfac<MODE, float>), grid, block, lds, s, g.d, m, stale);
+              hipLaunchKernelGGL((k_sfac<MODE, float>), grid, block, lds, s, g.d, m, stale, groups);
               return;
             }
-          hipLaunchKernelGGL((k_sfac<MODE, double>), grid, block, lds, s, g.d, m, stale);
+          hipLaunchKernelGGL((k_sfac<MODE, double>), grid, block, lds, s, g.d, m, stale, groups);
         });
   if (part & 2)
     launch_over(
@@ -691,7 +705,8 @@ static void launch_sfac_mode(const Group &g, int sel, int part, hipStream_t s) {
 
 // Variant: bit 0 TTM3-F site sets (the fixed-charge models share them), bit 1
 // FP32 (the mixed form's SOR iterations; its refinement, iter < 0, in FP64),
-// above them the waves per block.  sel_mixed: only the mixed-form replicas.
+// above them the
+// site and column groups and the tiles per group.  sel_mixed: only the mixed-form replicas.
 template <int MO>
 static void launch_field_mode(const Group &g, int iter, bool sel_mixed, hipStream_t s) {
   launch_over(
@@ -701,25 +716,28 @@ static void launch_field_mode(const Group &g, int iter, bool sel_mixed, hipStrea
           return Plan{-1, 0, 0, 0, 0};
         const bool f32 = MO == FD_D && c.mixed && iter > 0;
         const int M = MO == FD_D ? c.nd * c.N : (c.model == 2 ? 4 : 3) * c.N;
-        int sg, cg;
-        field_groups(c, M, sg, cg);
-        auto tab = [&] { return (f32 ? sizeof(float2) : sizeof(double2)) * (c.T + 1) * phase_row(sg * FD_SB); };
+        int nt, sg, cg;
+        field_groups(c, M, nt, sg, cg);
+        auto tab = [&] { return (f32 ? sizeof(float2) : sizeof(double2)) * (c.T + 1) * phase_row(sg * 16 * nt); };
         while (sg > 1 && tab() > 64 * 1024) sg /= 2;
-        return Plan{(c.model == 2 ? 0 : 1) | (f32 ? 2 : 0) | (sg << 2) | (cg << 5),
-                    idiv(M, sg * FD_SB), c.P, 1,
-                    std::max(tab(), sizeof(double) * cg * 4 * sg * FD_SB)};
+        return Plan{(c.model == 2 ? 0 : 1) | (f32 ? 2 : 0) | (sg << 2) | (cg << 5) | (nt << 10),
+                    idiv(M, sg * 16 * nt), c.P, 1,
+                    std::max(tab(), sizeof(double) * cg * 4 * sg * 16 * nt)};
       },
       [&](int v, dim3 grid, const BlockMap &m, size_t lds) {
         const int sg = (v >> 2) & 7;
-        const dim3 block(64 * sg * (v >> 5));
+        const dim3 block(64 * sg * ((v >> 5) & 31));
+        const bool two = (v >> 10) == 2;
+#define PIMD_FIELD(ML, R)                                                                          \
+  if (two) hipLaunchKernelGGL((k_field<MO, ML, R, 2>), grid, block, lds, s, g.d, m, iter, sg);     \
+  else hipLaunchKernelGGL((k_field<MO, ML, R, 1>), grid, block, lds, s, g.d, m, iter, sg)
         if constexpr (MO == FD_D)
           if (v & 2) {
-            if (v & 1) hipLaunchKernelGGL((k_field<MO, 3, float>), grid, block, lds, s, g.d, m, iter, sg);
-            else hipLaunchKernelGGL((k_field<MO, 2, float>), grid, block, lds, s, g.d, m, iter, sg);
+            if (v & 1) { PIMD_FIELD(3, float); } else { PIMD_FIELD(2, float); }
             return;
           }
-        if (v & 1) hipLaunchKernelGGL((k_field<MO, 3, double>), grid, block, lds, s, g.d, m, iter, sg);
-        else hipLaunchKernelGGL((k_field<MO, 2, double>), grid, block, lds, s, g.d, m, iter, sg);
+        if (v & 1) { PIMD_FIELD(3, double); } else { PIMD_FIELD(2, double); }
+#undef PIMD_FIELD
       });
 }
 

@@ -1,6 +1,6 @@
 """The reciprocal-space passes at the edges of their tiles: 16 kz-columns and 8
-|kz| to a structure-factor product, chunks of 8 sites, 16-site tiles in groups
-of 32 to a field block, one round of tasks and several.  Molecule counts that
+|kz| to a structure-factor product, chunks of 8 sites, 16-site tiles, one or
+two to a group of a field block, one round of tasks and several.  Molecule counts that
 leave one site, a full tile and one more; boxes of unequal axes, whose |kz|
 reach from 4 past 16; every model; the dipole passes forced where the dense
 solve would take them.  Against the oracle at the bounds of
@@ -20,6 +20,8 @@ CASES = [
     (3, 33, 2, (1.5, 1, 1), 1e-6), (3, 33, 1, (1, 1, 5), 1e-10), (3, 86, 2, (1, 1, 1), 1e-10),
     (2, 2, 1, (1, 1, 1), 1e-6), (2, 11, 2, (1, 2, 1), 1e-8), (2, 43, 2, (1, 1, 2), 1e-8),
     (4, 11, 2, (1, 1, 4), 1e-8), (5, 43, 3, (1, 1, 1), 1e-6),
+    # beads enough for two tiles to a site group
+    (3, 33, 48, (1, 1, 1.5), 1e-6), (2, 17, 64, (1, 1, 1), 1e-6), (4, 22, 64, (1, 1, 1), 1e-6),
 ]
 
 
