@@ -1430,6 +1430,7 @@ template <int MODEL, int G, typename R, bool LDS = false>
 __global__ __launch_bounds__(256) void k_pair_final(const Rep *__restrict__ reps, BlockMap bm) {
   constexpr int ND = MODEL == 2 ? 3 : 1;
   constexpr int T0 = MODEL == 2 ? 0 : 3;
+  constexpr bool SITE_ARM = sizeof(R) == 8;
   constexpr int FIN_SB_UNROLL = MODEL == 2 && sizeof(R) == 8 ? 1 : 4;
   extern __shared__ Site lds_site[];  // [4N] sites, then [N][ND][3] dipoles
   const Blk bk = block_of(bm);
@@ -1471,7 +1472,7 @@ __global__ __launch_bounds__(256) void k_pair_final(const Rep *__restrict__ reps
     for (int k = 0; k < 3; ++k)
       mua[t][k] = is_dip<MODEL>(t) ? bead_dip[((size_t)a * ND + (t - T0)) * 3 + k] : 0.0;
   }
-  double ph[4] = {0, 0, 0, 0}, fr[4][3] = {{0}}, vt[9] = {0};
+  double ph[4] = {0, 0, 0, 0}, fr[4][3] = {{0}}, vc = 0.0, vt[9] = {0};
   const int nf = valid ? nbrc[grp] : 0, nn = valid ? nbrn[grp] : 0;
   const int *list = nbr + (size_t)grp * c.nbr_cap;
   auto visit = [&](const int j, auto thole_tag) {
@@ -1545,7 +1546,16 @@ __global__ __launch_bounds__(256) void k_pair_final(const Rep *__restrict__ reps
         if (have_ts1 && db) ph[sa] += (double)(ts1 * (r[0] * dj[0] + r[1] * dj[1] + r[2] * dj[2]));
         const double dij[3] = {(double)dijr[0], (double)dijr[1], (double)dijr[2]};
         for (int k = 0; k < 3; ++k) fr[sa][k] += dij[k];
-        // the same from either molecule: halved at the end
+        // the same from either molecule: halved at the end.  Rij0 of the dipole
+        // loop is wrapped to ~0 (pot_ttm.f90:406-407,468), so the centroid
+        // virial is Rc . F summed over the sites, in FP64 from their forces at
+        // the end.  The FP32 form rounds the two sides' forces of a pair
+        // apart, so keeps the difference of the centroids here: the virial
+        // then does not depend on the origin
+        if constexpr (!SITE_ARM) {
+          const double *rca = Rcs + (a * 4 + sa) * 3, *rcb = Rcs + (j * 4 + sb) * 3;
+          for (int k = 0; k < 3; ++k) vc += (rca[k] - rcb[k]) * dij[k];
+        }
         for (int col = 0; col < 3; ++col)
           for (int row = 0; row < 3; ++row) vt[col * 3 + row] += dij[row] * v[col];
       }
@@ -1557,6 +1567,7 @@ __global__ __launch_bounds__(256) void k_pair_final(const Rep *__restrict__ reps
     ph[t] = group_sum<G>(ph[t]);
     for (int k = 0; k < 3; ++k) fr[t][k] = group_sum<G>(fr[t][k]);
   }
+  if constexpr (!SITE_ARM) vc = group_sum<G>(vc);
   for (int i = 0; i < 9; ++i) vt[i] = group_sum<G>(vt[i]);
   if (valid && lane == 0) {
     const size_t base = ((size_t)b * N + a) * 4;
@@ -1564,11 +1575,12 @@ __global__ __launch_bounds__(256) void k_pair_final(const Rep *__restrict__ reps
       phi[base + t] += ph[t];
       for (int k = 0; k < 3; ++k) dR[(base + t) * 3 + k] += fr[t][k];
     }
-    // Rij0 of the dipole loop is wrapped to ~0 (pot_ttm.f90:406-407,468): the
-    // centroid virial is Rc . F summed over the sites
-    double vc = 0.0;
-    for (int t = 0; t < 4; ++t)
-      for (int k = 0; k < 3; ++k) vc += Rcs[(a * 4 + t) * 3 + k] * fr[t][k];
+    if constexpr (SITE_ARM) {
+      for (int t = 0; t < 4; ++t)
+        for (int k = 0; k < 3; ++k) vc += Rcs[(a * 4 + t) * 3 + k] * fr[t][k];
+    } else {
+      vc *= 0.5;
+    }
     for (int i = 0; i < 9; ++i) vt[i] *= 0.5;
     double *tl = tally + ((size_t)b * N + a) * T_COUNT;
     tl[T_VIRC] += vc;

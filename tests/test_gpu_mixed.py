@@ -120,3 +120,31 @@ def test_mixed_two_sided_pair_passes(model, N, P, half, monkeypatch):
     r64 = _ff(TTMParams(**kw).resolved()).full_bead_forces(RRt, RRc)
     rmx = _ff(TTMParams(**kw, precision=1).resolved()).full_bead_forces(RRt, RRc)
     _compare(rmx, _as_ref(r64), f"two-sided mixed vs fp64 ttm{model} N{N} P{P}")
+
+
+@pytest.mark.parametrize("model,N,P", [(3, 64, 2), (2, 24, 2)])
+def test_mixed_two_sided_final_virial_keeps_no_origin(model, N, P, monkeypatch):
+    """The centroid virial of the two-sided final pair pass in FP32 does not
+    depend on where the origin lies.  The once-per-pair pass gives a pair's
+    two molecules the same force with opposite signs, so what the two passes
+    differ by (PIMD_FIN_HALF = 0 and 1, the same charge pass) must not change
+    when every atom moves by whole boxes, some 1000 A.  Forces of each side
+    taken apart would leave a net force of some 1e-7 of the pair forces, times
+    1000 A: 1e-4 and more.  With their difference of centroids only the coordinates'
+    rounding there (2e-13 A), the 2^-40 steps of the partner sums and a
+    flipped FP32 digit of a distance remain: 1e-5."""
+    from pimd_amd.params import TTMParams
+    from pimd_amd.systems import make_system
+    print("case origin", model, N, P, flush=True)
+    RRt, _, RRc, L = make_system(N, P, seed=900 + N)
+    p = TTMParams(pot_model=model, nwaters=N, nbeads=P, box=(L, L, L), rc=-1.0, eps_ewald=1e-6,
+                  precision=1).resolved()
+    diff = []
+    for shift in (0.0, L * round(1000.0 / L)):
+        vc = []
+        for half in ("0", "1"):
+            monkeypatch.setenv("PIMD_FIN_HALF", half)
+            vc.append(_ff(p).full_bead_forces(RRt + shift, RRc + shift)["virialct"])
+        diff.append(vc[0] - vc[1])
+    print("passes apart by", diff[0], "shifted", diff[1], flush=True)
+    assert np.max(np.abs(diff[1] - diff[0])) < 1e-5
