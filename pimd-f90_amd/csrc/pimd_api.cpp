@@ -2267,9 +2267,12 @@ static int tangent_start(pimd_ctx *x, const double *RRt, const double *ew, const
   const int nsweep = adj ? 1 : ndir;  // workgroups per configuration
   const size_t P = (size_t)c.P, n = P * x->natoms * 3, nout = P * nsweep * 4;
   const size_t nadj = adj ? P * TTM_ADJ_NPARAM * 2 : 0;
-  const size_t ext = adj ? (adjoint_extra_doubles(c) + 1) & ~(size_t)1 : 0;
+  const AdjPlan plan = adj ? adjoint_plan(c) : AdjPlan{};
+  const size_t ext = plan.extra;
   const size_t ws = tangent_ws_duals(c) * P * nsweep * 2, cfg = tangent_cfg_doubles(c) * P;
   const size_t bytes = sizeof(double) * (ext + ws + cfg + 2 * n + P + nout + nadj);
+  // the adjoint's own part is not counted: about 1 GB of matrices at most and
+  // a few hundred bytes per molecule
   if (bytes - sizeof(double) * ext > ((size_t)32 << 30))
     return fail(PIMD_EINVAL, "parameter derivatives of %zu configurations need %.1f GB of workspace; "
                 "split them into smaller contexts", P, bytes / 1e9);
@@ -2284,6 +2287,7 @@ static int tangent_start(pimd_ctx *x, const double *RRt, const double *ew, const
     d.tan_bytes = bytes;
   }
   TanLaunch L;
+  L.plan = plan;
   L.extra = d.tan;      // the dual workspaces first: 16-byte aligned
   L.ws = d.tan + ext;
   L.cfg = d.tan + ext + ws;

@@ -429,6 +429,14 @@ constexpr int TTM_ADJ_NPARAM = TTM_NPARAM + DMS_NCOEF + 1;
 enum TtmParam { TP_VDWA = 0, TP_VDWB, TP_VDWC, TP_VDWD, TP_VDWE, TP_POLARO, TP_POLARH, TP_POLARM,
                 TP_POLFACO, TP_POLFACH, TP_POLFACM, TP_ADD, TP_ACC, TP_DMS1, TP_DMS2, TP_DMS3 };
 
+// How the adjoint solves for the induced dipoles, chosen once per call: the
+// environment is read here, for the workspace's size and the launches alike.
+struct AdjPlan {
+  bool dense = false;  // from a dense matrix, `slice` configurations at a time
+  int slice = 0;
+  size_t solve = 0;    // doubles of the solve, the first of ...
+  size_t extra = 0;    // ... all doubles beyond the dual workspaces
+};
 // Buffers and parameters of one tangent launch (ttm_tangent.hip).
 struct TanLaunch {
   const double *RR, *pes;
@@ -444,12 +452,13 @@ struct TanLaunch {
   int gamma_m;   // 1: the one direction is the M-site fraction gammaM (moves the M sites)
   int adjoint;   // 1: the adjoint of all TTM_ADJ_NPARAM parameters (one sweep along gw)
   double *adj;   // adjoint output [P][TTM_ADJ_NPARAM][2]
-  double *extra; // adjoint: adjoint_extra_doubles(c)
+  double *extra; // adjoint: plan.extra doubles
+  AdjPlan plan;  // adjoint
   const int4 *cols;
   const int *colk;
   int ndir;
 };
-size_t adjoint_extra_doubles(const SysConst &c);
+AdjPlan adjoint_plan(const SysConst &c);
 size_t tangent_cfg_doubles(const SysConst &c);
 size_t tangent_ws_duals(const SysConst &c);
 void launch_ttm_tangent(const SysConst &c, const TanLaunch &L, hipStream_t s);

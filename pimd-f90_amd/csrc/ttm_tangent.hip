@@ -927,7 +927,9 @@ __global__ __launch_bounds__(TAN_BLOCK) void k_ttm_tangent(SysConst c, TanArgs a
 // the dense one of the force path, on dual numbers: the matrix and its
 // derivative along the positions' direction are formed once (k_adj_build) and
 // an iteration is a product with them (k_adj_solve).  64 five-water clusters
-// and 64 boxes of 32 H2O side by side: 8.8 -> 0.5 ms.
+// and 64 boxes of 32 H2O side by side: 8.8 -> 0.5 ms.  Larger systems, whose
+// matrix grows with the square of the sites, take an iteration pass by pass
+// from the positions (k_adj_sfac, k_adj_step, k_adj_test; adjoint_plan).
 //
 // Values are evaluated in plain FP64 and their position derivatives follow
 // chain_d; the Thole derivatives d ts / d a come from duals along a.
@@ -942,6 +944,7 @@ struct AdjArgs {
   TanArgs t;
   Dual *mat;             // [slice][D][D] dipole matrix, D = 3 nd N
   int b0;                // first configuration of the slice
+  int2 *state;           // [P] of the pass-by-pass solve: active, iterations done
   double *pv, *pa;       // [P][pair workgroups][ADJ_NV], [ADJ_NA]
   const int4 *cols;      // kz-columns and their first k-vectors
   const int *colk;
@@ -1073,14 +1076,18 @@ __global__ __launch_bounds__(TAN_BLOCK) void k_adj_pair_q(SysConst c, AdjArgs x)
   block_sums<ADJ_NV>(v, red, x.pv + ((size_t)b * gridDim.x + blockIdx.x) * ADJ_NV);
 }
 
-// Structure factor of the charges, or of the dipoles of the last SOR step's
-// input (ewald.f90:1-119): four lanes per k-vector share its sites.
+// Structure factor of the charges, or of the dipoles (ewald.f90:1-119): of
+// SOR iteration `it`'s input (odd iterations read dip and write old, even ones
+// the other way round), with it = 0 of the last step's input, left in old.
+// Four lanes per k-vector share its sites.
 template <bool DIP>
-__global__ __launch_bounds__(TAN_BLOCK) void k_adj_sfac(SysConst c, AdjArgs x) {
+__global__ __launch_bounds__(TAN_BLOCK) void k_adj_sfac(SysConst c, AdjArgs x, int it) {
   const TanArgs &a = x.t;
   const int b = blockIdx.y, N = c.N;
+  if (it > 1 && !x.state[b].x) return;
   const AdjCfg g(c, a, b);
   const TanWs W(a.ws + (size_t)b * a.ws_stride, c);
+  const Dual *dip = it & 1 ? W.dip : W.old;
   const int k = blockIdx.x * (TAN_BLOCK / 4) + threadIdx.x / 4, u = threadIdx.x % 4;
   if (k >= c.nk) return;  // alike over the four lanes
   const int4 h = a.khkl[k];
@@ -1091,7 +1098,7 @@ __global__ __launch_bounds__(TAN_BLOCK) void k_adj_sfac(SysConst c, AdjArgs x) {
     Dual ck, sk;
     g.ph.at(s0 + i, h, kv, ck, sk);
     if (DIP) {
-      const Dual *m = W.old + 3 * i;
+      const Dual *m = dip + 3 * i;
       const Dual dk = m[0] * kv.x + m[1] * kv.y + m[2] * kv.z;
       re -= dk * sk;
       im += dk * ck;
@@ -1276,8 +1283,8 @@ __global__ __launch_bounds__(64 * ADJ_BW) void k_adj_build(SysConst c, AdjArgs x
 // The SOR iterations (pot_ttm.f90:306-392) on duals, one workgroup per
 // configuration: 16 lanes per matrix row, the matrix streamed from L2 (147 KB
 // for 32 H2O, about 3 us per iteration: 64 B per clock into one CU), the
-// dipoles in LDS or, beyond 2048 components, in global memory.  Leaves the final dipoles in dip and the last step's input in old.
-template <bool LDS>
+// dipoles in LDS.  Leaves the final dipoles in dip and the last step's input in
+// old.
 __global__ __launch_bounds__(ADJ_SOLVE) void k_adj_solve(SysConst c, AdjArgs x) {
   extern __shared__ Dual lds_mu[];  // [2][D]
   __shared__ double red[2][ADJ_SOLVE / 64];
@@ -1286,18 +1293,13 @@ __global__ __launch_bounds__(ADJ_SOLVE) void k_adj_solve(SysConst c, AdjArgs x) 
   const TanWs W(a.ws + (size_t)b * a.ws_stride, c);
   const Dual *m = x.mat + (size_t)blockIdx.x * D * D;
   const int g = threadIdx.x >> 4, u = threadIdx.x & 15;
-  Dual *buf[2] = {W.dip, W.old};
-  if constexpr (LDS) {
-    buf[0] = lds_mu;
-    buf[1] = lds_mu + D;
-    for (int e = threadIdx.x; e < D; e += ADJ_SOLVE) lds_mu[e] = W.dip[e];
-    __syncthreads();
-  }
+  for (int e = threadIdx.x; e < D; e += ADJ_SOLVE) lds_mu[e] = W.dip[e];
+  __syncthreads();
   const double om = c.sor;
   int cur = 0;
   for (int it = 1;; ++it) {
-    const Dual *mu = LDS ? lds_mu + (size_t)cur * D : buf[cur];
-    Dual *nu = LDS ? lds_mu + (size_t)(cur ^ 1) * D : buf[cur ^ 1];
+    const Dual *mu = lds_mu + (size_t)cur * D;
+    Dual *nu = lds_mu + (size_t)(cur ^ 1) * D;
     double ss = 0.0;
     for (int row = g; row < D; row += ADJ_SOLVE / 16) {
       const Dual *A = m + (size_t)row * D;
@@ -1321,17 +1323,89 @@ __global__ __launch_bounds__(ADJ_SOLVE) void k_adj_solve(SysConst c, AdjArgs x) 
     cur ^= 1;
     if (c.stath * sqrt(sum) < c.peps || it >= c.maxiter) break;
   }
-  if constexpr (LDS) {
-    for (int e = threadIdx.x; e < D; e += ADJ_SOLVE) {
-      W.dip[e] = lds_mu[(size_t)cur * D + e];
-      W.old[e] = lds_mu[(size_t)(cur ^ 1) * D + e];
+  for (int e = threadIdx.x; e < D; e += ADJ_SOLVE) {
+    W.dip[e] = lds_mu[(size_t)cur * D + e];
+    W.old[e] = lds_mu[(size_t)(cur ^ 1) * D + e];
+  }
+}
+
+// One SOR iteration from the positions, a wave per dipole site: the
+// reciprocal-space field of k_adj_sfac's structure factor (lanes over the
+// k-vectors), the real-space one (lanes over the molecules) and the update.
+// The squared change of a site's dipole goes into its Efd.
+__global__ __launch_bounds__(TAN_BLOCK) void k_adj_step(SysConst c, AdjArgs x, int it) {
+  const TanArgs &a = x.t;
+  const int b = blockIdx.y, N = c.N, tend = c.tdip + c.nd;
+  if (it > 1 && !x.state[b].x) return;
+  const int i = blockIdx.x * (TAN_BLOCK / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (i >= c.nd * N) return;
+  const int s = c.tdip * N + i, iw = s % N, ti = s / N;
+  const AdjCfg g(c, a, b);
+  const TanWs W(a.ws + (size_t)b * a.ws_stride, c);
+  const Dual *src = it & 1 ? W.dip : W.old;
+  Dual *dst = it & 1 ? W.old : W.dip;
+  Dual e[3] = {0.0, 0.0, 0.0};
+  for (int k = lane; k < c.nk; k += 64) {
+    const double4 kv = a.kv[k];
+    Dual ck, sk;
+    g.ph.at(s, a.khkl[k], kv, ck, sk);
+    const Dual t = kv.w * (ck * W.Sm[2 * k + 1] - sk * W.Sm[2 * k]);
+    e[0] -= t * kv.x;
+    e[1] -= t * kv.y;
+    e[2] -= t * kv.z;
+  }
+  for (int jw = lane; jw < N; jw += 64) {
+    const bool same = jw == iw;
+    double R[3];
+    if (!same && !g.within(c, iw, jw, R)) continue;
+    for (int tj = c.tdip; tj < tend; ++tj) {
+      if (same && tj == ti) continue;
+      const int sj = tj * N + jw;
+      Dual r[3], o[3];
+      g.vec(c, s, sj, r);
+      const Dual d2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+      double u1, u2, u3;
+      smear3(c, d2.v, c.apolDD[ti][tj], u1, u2, u3);
+      Dual t1 = u1, t2 = u2;
+      chain_d(t1, 1, u2, d2.d);
+      chain_d(t2, 2, u3, d2.d);
+      dd3d(r, t1, t2, src + 3 * (sj - c.tdip * N), o);
+      for (int k = 0; k < 3; ++k) e[k] += o[k];
     }
-  } else if (cur == 1) {  // the final dipoles are in old: exchange the buffers
-    for (int e = threadIdx.x; e < D; e += ADJ_SOLVE) {
-      const Dual t = W.dip[e];
-      W.dip[e] = W.old[e];
-      W.old[e] = t;
-    }
+  }
+  for (int k = 0; k < 3; ++k) e[k] = group_sum(e[k], 64);
+  if (lane != 0) return;
+  const double om = c.sor, pol = c.polar[ti];
+  double d2 = 0.0;
+  for (int k = 0; k < 3; ++k) {
+    const Dual mr = src[3 * i + k], ek = e[k] + W.Efq[3 * s + k] + c.fac_dd * mr;
+    const Dual nr = (1.0 - om) * mr + (om * pol) * ek;
+    const double df = nr.v - (it == 1 ? 0.0 : mr.v);
+    d2 += df * df;
+    dst[3 * i + k] = nr;
+  }
+  W.Efd[i].v = d2;
+}
+
+// The convergence test of iteration `it`, a workgroup per configuration.  One
+// that ends after an odd count exchanges dip and old.
+__global__ __launch_bounds__(TAN_BLOCK) void k_adj_test(SysConst c, AdjArgs x, int it) {
+  __shared__ double red[1][TAN_BLOCK / 64], sum[1];
+  const TanArgs &a = x.t;
+  const int b = blockIdx.x, M = c.nd * c.N;
+  if (it > 1 && !x.state[b].x) return;
+  const TanWs W(a.ws + (size_t)b * a.ws_stride, c);
+  double d2[1] = {0.0};
+  for (int i = threadIdx.x; i < M; i += TAN_BLOCK) d2[0] += W.Efd[i].v;
+  block_sums<1>(d2, red, sum);
+  __syncthreads();
+  const bool last = c.stath * sqrt(sum[0]) < c.peps || it >= c.maxiter;
+  if (threadIdx.x == 0) x.state[b] = make_int2(last ? 0 : 1, it);
+  if (!last || !(it & 1)) return;
+  for (int e = threadIdx.x; e < 3 * M; e += TAN_BLOCK) {
+    const Dual t = W.dip[e];
+    W.dip[e] = W.old[e];
+    W.old[e] = t;
   }
 }
 
@@ -1532,29 +1606,42 @@ __global__ __launch_bounds__(TAN_BLOCK) void k_adj_out(SysConst c, AdjArgs x) {
   }
 }
 
-// Configurations whose dipole matrices are held at a time (PIMD_ADJ_MAT_MB of
-// them, default 1024, at least one), and the adjoint's workspace beyond the
-// duals of tangent_ws_duals: the matrices and the pair kernels' partial sums.
-static size_t adj_mat_duals(const SysConst &c) {
-  const size_t D = 3 * (size_t)c.nd * c.N;
-  return D * D;
-}
-static size_t adj_slice(const SysConst &c) {
-  const char *e = std::getenv("PIMD_ADJ_MAT_MB");
-  const long mb = e ? std::strtol(e, nullptr, 10) : 0;
-  const size_t n = ((size_t)(mb > 0 ? mb : 1024) << 20) / (sizeof(Dual) * adj_mat_duals(c));
-  return std::min((size_t)c.P, std::max<size_t>(n, 1));
-}
-size_t adjoint_extra_doubles(const SysConst &c) {
-  return 2 * adj_slice(c) * adj_mat_duals(c) +
-         (size_t)c.P * adj_pair_blocks(c) * (ADJ_NV + ADJ_NA);
+// The dense solve takes systems of up to ADJ_DENSE_MAX_D dipole components
+// (16 D^2 bytes of matrix each, in slices of as many configurations as
+// PIMD_ADJ_MAT_MB, default 1024, takes, at least one); larger ones, whose
+// matrix one workgroup would stream every iteration, go pass by pass, in
+// memory that grows with the sites.  Whole adjoint, dense / passes, ms
+// (components x configurations): 96 x 64 0.51 / 1.05, 192 x 16 0.47 / 0.69,
+// 384 x 1 0.67 / 0.80, 384 x 64 2.23 / 3.03; 576 x 1 (TTM2.1-F) 0.91 / 0.76,
+// 576 x 16 1.40 / 1.15, 768 x 1 1.85 / 1.22, 768 x 32 5.10 / 3.56, 2040 x 8
+// 21.0 / 4.0.  1000 TTM3-F waters 3.0 (one workgroup per configuration: 215).
+// PIMD_ADJ_DENSE=0: pass by pass at every size.
+constexpr size_t ADJ_DENSE_MAX_D = 480;
+AdjPlan adjoint_plan(const SysConst &c) {
+  AdjPlan p;
+  const size_t D = 3 * (size_t)c.nd * c.N, mat = D * D;
+  auto env = [](const char *name) {
+    const char *e = std::getenv(name);
+    return e && *e ? std::strtol(e, nullptr, 10) : -1;
+  };
+  p.dense = D <= ADJ_DENSE_MAX_D && env("PIMD_ADJ_DENSE") != 0;
+  if (p.dense) {
+    const long mb = env("PIMD_ADJ_MAT_MB");
+    const size_t bytes = (size_t)(mb > 0 ? mb : 1024) << 20;
+    p.slice = (int)std::min((size_t)c.P, std::max<size_t>(bytes / (sizeof(Dual) * mat), 1));
+  }
+  // 16-byte aligned: the dual workspace follows
+  p.solve = p.dense ? 2 * p.slice * mat : ((size_t)c.P + 1) & ~(size_t)1;
+  p.extra = p.solve + (((size_t)c.P * adj_pair_blocks(c) * (ADJ_NV + ADJ_NA) + 1) & ~(size_t)1);
+  return p;
 }
 
 static void launch_adjoint(const SysConst &c, const TanLaunch &L, const TanArgs &a, hipStream_t s) {
   AdjArgs x;
   x.t = a;
   x.mat = (Dual *)L.extra;
-  x.pv = L.extra + 2 * adj_slice(c) * adj_mat_duals(c);
+  x.state = (int2 *)L.extra;
+  x.pv = L.extra + L.plan.solve;
   x.pa = x.pv + (size_t)c.P * adj_pair_blocks(c) * ADJ_NV;
   x.cols = L.cols;
   x.colk = L.colk;
@@ -1565,24 +1652,28 @@ static void launch_adjoint(const SysConst &c, const TanLaunch &L, const TanArgs 
     x.pf[i] = 1.0 / (f6 * f6 * f6);
     x.dpf[i] = -0.5 * x.pf[i] / p;
   }
-  const int P = c.P, ns = 4 * c.N, M = c.nd * c.N, D = 3 * M, nt = (M + 7) / 8;
+  const int P = c.P, ns = 4 * c.N, M = c.nd * c.N, D = 3 * M, nt = (M + 7) / 8, wpb = TAN_BLOCK / 64;
   const dim3 B(TAN_BLOCK), gp(adj_pair_blocks(c), P), gs((c.nk + TAN_BLOCK / 4 - 1) / (TAN_BLOCK / 4), P),
-      gf((ns + TAN_BLOCK / 64 - 1) / (TAN_BLOCK / 64), P);
+      gf((ns + wpb - 1) / wpb, P), gm((M + wpb - 1) / wpb, P);
   hipLaunchKernelGGL(k_tangent_monomer<TAN_ADJOINT>, dim3(P, 1), B, 0, s, c, a);
   hipLaunchKernelGGL(k_adj_pair_q, gp, B, 0, s, c, x);
-  hipLaunchKernelGGL(k_adj_sfac<false>, gs, B, 0, s, c, x);
+  hipLaunchKernelGGL(k_adj_sfac<false>, gs, B, 0, s, c, x, 0);
   hipLaunchKernelGGL(k_adj_field<false>, gf, B, 0, s, c, x);
-  const int slice = (int)adj_slice(c);
-  for (int b0 = 0; b0 < P; b0 += slice) {
-    const int n = std::min(slice, P - b0);
-    x.b0 = b0;
-    hipLaunchKernelGGL(k_adj_build, dim3(nt * (nt + 1) / 2, n), dim3(64 * ADJ_BW), 0, s, c, x);
-    if (D <= 2048)
-      hipLaunchKernelGGL(k_adj_solve<true>, dim3(n), dim3(ADJ_SOLVE), 2 * sizeof(Dual) * D, s, c, x);
-    else
-      hipLaunchKernelGGL(k_adj_solve<false>, dim3(n), dim3(ADJ_SOLVE), 0, s, c, x);
+  if (L.plan.dense) {
+    for (int b0 = 0; b0 < P; b0 += L.plan.slice) {
+      const int n = std::min(L.plan.slice, P - b0);
+      x.b0 = b0;
+      hipLaunchKernelGGL(k_adj_build, dim3(nt * (nt + 1) / 2, n), dim3(64 * ADJ_BW), 0, s, c, x);
+      hipLaunchKernelGGL(k_adj_solve, dim3(n), dim3(ADJ_SOLVE), 2 * sizeof(Dual) * D, s, c, x);
+    }
+  } else {
+    for (int it = 1; it <= c.maxiter; ++it) {
+      hipLaunchKernelGGL(k_adj_sfac<true>, gs, B, 0, s, c, x, it);
+      hipLaunchKernelGGL(k_adj_step, gm, B, 0, s, c, x, it);
+      hipLaunchKernelGGL(k_adj_test, dim3(P), B, 0, s, c, x, it);
+    }
   }
-  hipLaunchKernelGGL(k_adj_sfac<true>, gs, B, 0, s, c, x);
+  hipLaunchKernelGGL(k_adj_sfac<true>, gs, B, 0, s, c, x, 0);
   hipLaunchKernelGGL(k_adj_pair_d, gp, B, 0, s, c, x);
   hipLaunchKernelGGL(k_adj_field<true>, gf, B, 0, s, c, x);
   hipLaunchKernelGGL(k_adj_out, dim3(1 + (3 + DMS_NCOEF + ADJ_PPB - 1) / ADJ_PPB, P), B, 0, s, c, x);
