@@ -758,15 +758,17 @@ __global__ __launch_bounds__(256) void k_pair_qq(const Rep *__restrict__ reps, B
 // matches an FP64 sum and stays smooth in the model parameters.  FP32 form:
 // one word, rint(v 2^40) (range +-2^23): its pair terms already round at
 // 1e-7 relative, far above that quantum, and one LDS atomic per value in
-// place of two.  Integer addition wraps modulo 2^64 and is associative: only
-// totals must fit.  Bound by FP64 issue: about 80 instructions per site pair
+// place of two.  A value beyond the range (molecules that overlap) goes in as
+// the range's end, with its sign.  Integer addition wraps modulo 2^64 and is
+// associative: only totals must fit.  Bound by FP64 issue: about 80 instructions per site pair
 // beyond the 5 A radius and some 300 more inside it (the gamma function's
-// loop), 6 per partner value; 512 H2O x 32 beads 212 -> 117 us FP64 against
+// loop), 8 per partner value; 512 H2O x 32 beads 212 -> 117 us FP64 against
 // library exp, sqrt and division, divisions in the gamma function's loops and
 // f64-to-i64 conversions of the partner values; 110 -> 101 us FP32.
 constexpr double QQ_HI = 1048576.0;               // 2^20
 constexpr double QQ_LO = 18446744073709551616.0;  // 2^64
 constexpr double QQ_ONE = 1099511627776.0;        // 2^40
+constexpr double QQ_END2 = 9.2e18 / 4294967296.0, QQ_END1 = 9.2e18 / QQ_ONE;  // below 2^31, 2^23
 template <typename R>
 struct QqWords {
   static constexpr int n = sizeof(R) == 8 ? 2 : 1;
@@ -788,6 +790,8 @@ constexpr double qq_magic(int q) {
 constexpr double QQ_M20 = qq_magic(20), QQ_M40 = qq_magic(40), QQ_M64 = qq_magic(64);
 template <int NW>
 __device__ __forceinline__ void qq_fix_add(unsigned long long *acc, double v) {
+  constexpr double end = NW == 2 ? QQ_END2 : QQ_END1;
+  v = fmin(fmax(v, -end), end);
   const double t = v + QQ_M20, h = t - QQ_M20, rem = v - h;
   const long long a = __double_as_longlong(t) - __double_as_longlong(QQ_M20);
   if constexpr (NW == 2) {

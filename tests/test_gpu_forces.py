@@ -262,3 +262,35 @@ def test_force_call_in_two_halves():
     assert np.array_equal(ff.full_bead_forces_finish()["dRRt"], ref["dRRt"])
     for c in cases:
         c[0].close()
+
+
+@pytest.mark.parametrize("precision,end", [(0, 9.2e18 / 2 ** 32), (1, 9.2e18 / 2 ** 40)])
+def test_overlapping_molecules_saturate(monkeypatch, precision, end):
+    """Two waters 0.1 A apart, without polarisation: the dispersion force on
+    their oxygens, 4e10, is beyond the range of the once-per-pair pass's partner
+    sums (2^31, 2^23 in FP32).  The owner's side is the two-sided pass's; the
+    partner's is the end of the range with the same sign (the other terms,
+    smeared charges, are below 1e6)."""
+    from pimd_amd.params import TTMParams
+    from pimd_amd.systems import spaced_water_box
+    from pimd_amd.ttm import TTMForceField
+    cen, L = spaced_water_box(8, seed=3, tries=30)
+    R = np.array(cen, dtype=float).reshape(24, 3)
+    R[3:6] = R[0:3] + [0.1, 0.0, 0.0]
+    p = TTMParams(pot_model=3, nwaters=8, nbeads=2, box=(L, L, L), eps_ewald=1e-6,
+                  precision=precision).resolved()
+    gx = []
+    for half in ("0", "2"):
+        monkeypatch.setenv("PIMD_QQ_HALF", half)
+        ff = TTMForceField(p)
+        th = ff.ttm_params()
+        th[5:8] = 0.0
+        ff.set_ttm_params(th)
+        gx.append(ff.full_bead_forces(np.stack([R, R]), R)["dRRt"][0, [0, 3], 0])
+        ff.close()
+    print("case", precision, gx, flush=True)
+    two, one = gx
+    assert np.all(np.abs(two) > 1e10) and np.all(np.sign(one) == np.sign(two))
+    k = int(np.argmin(np.abs(one)))
+    assert abs(one[1 - k] - two[1 - k]) < 1e-5 * abs(two[1 - k])
+    assert abs(abs(one[k]) - end) < 1e6 + 1e-6 * end
