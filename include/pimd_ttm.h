@@ -127,11 +127,16 @@ int pimd_forces_all_beads_dev(pimd_ctx *ctx, const double *d_RRt, const double *
  * parameters are checked and set up as pimd_ctx_create does; every
  * intermediate array of the call lives in one static device workspace of
  * PIMD_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends, and the
- * call makes no device or pinned allocation.  Systems whose arrays exceed the
- * workspace are refused with PIMD_EINVAL (128 waters x 32 beads fit at
- * eps_ewald 1e-6 with Rc = L/2; 512 x 32 does not).  guess_initdip must be 0
- * (the predictor history would have to persist between calls).  Device
- * arrays as in pimd_forces_all_beads_dev; outputs may be NULL.  stream: a
+ * call makes no device or pinned allocation.  The results are the same bits as
+ * a context's.  Where the arrays of all beads exceed the workspace, the beads
+ * are taken in two halves, one after the other; systems that do not fit then
+ * are refused with PIMD_EINVAL (512 waters x 32 beads fit at eps_ewald 1e-6
+ * with Rc = L/2; 512 x 64 does not).  One exception to the same bits: a
+ * system whose context solves for the dipoles with a dense matrix, and where
+ * half the beads fit only without it, agrees to summation order.
+ * guess_initdip must be 0 (the predictor history would have to persist
+ * between calls).  Device arrays as in pimd_forces_all_beads_dev; outputs may
+ * be NULL.  stream: a
  * hipStream_t, NULL for the default stream; the kernels are enqueued there
  * and the call returns without waiting for them.  Every call on one GPU
  * shares that GPU's workspace: calls that overlap on one GPU (on different

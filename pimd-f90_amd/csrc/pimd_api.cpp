@@ -275,7 +275,7 @@ int setup_system(pimd_ctx *x) {
   const pimd_params &p = x->p;
   SysConst &c = x->c;
   c.N = p.nwaters;
-  c.P = p.nbeads;
+  c.P = c.shapeP = p.nbeads;
   c.model = p.pot_model;
   for (int k = 0; k < 3; ++k) {
     c.box[k] = p.box[k];
@@ -618,7 +618,6 @@ void layout_system(pimd_ctx *x, Arena &a, bool full) {
   }
   a.take(&d.Sq, P * nk * 2);
   a.take(&d.Sm, P * nk * 2);
-  a.take(&d.Sv, P * nk * 6);
   a.take(&d.virk, P * ((nk + 255) / 256) * 18);
   a.take(&d.part, full ? P * (size_t)c.sf_chunks_max * nk * 6 : sfac_part_elems(c));
   a.take(&d.wk, field_operand_elems(c));
@@ -2574,13 +2573,22 @@ extern "C" int pimd_forces_all_beads_noalloc(const pimd_params *params, const do
   x.c.poll = 0;
   x.c.overlap = 0;
   x.c.dd_cache = 0;
+  // All beads at once or, where they need up to 7/4 of the workspace, one half
+  // after the other with the launch shapes of all (a bead's results do not
+  // depend on the others); without the dense dipole matrix where it fits
+  // neither way.
   Arena a;
-  layout_system(&x, a, false);
-  if (x.c.dense && a.off > sizeof(scratch)) {
-    // no room for the dense dipole matrix: the pass-by-pass solve
-    x.c.dense = 0;
+  auto fits = [&](int beads) {
+    x.c.P = beads;
     a.off = 0;
     layout_system(&x, a, false);
+    return a.off <= sizeof(scratch);
+  };
+  const int whole = p.nbeads, half = (p.nbeads + 1) / 2;
+  auto lay_out = [&] { return fits(whole) || (a.off / 7 <= sizeof(scratch) / 4 && fits(half)); };
+  if (!lay_out()) {
+    x.c.dense = 0;
+    (void)lay_out();
   }
   if (a.off > sizeof(scratch))
     return fail(PIMD_EINVAL, "%d waters x %d beads need %zu bytes of device workspace, more than "
@@ -2596,26 +2604,32 @@ extern "C" int pimd_forces_all_beads_noalloc(const pimd_params *params, const do
   if ((rc = sync_rep(&x)) != PIMD_OK) return rc;  // the replica record, in the workspace too
   DevBufs &d = x.d;
   hipStream_t s = x.stream;
-  const size_t P = p.nbeads, N = p.nwaters, na = 3 * N;
-  HIPCHK(hipMemcpyAsync(d.RR, RR, sizeof(double) * P * na * 3, hipMemcpyDeviceToDevice, s));
+  const size_t n = x.c.P, N = p.nwaters, na = 3 * N;
   HIPCHK(hipMemcpyAsync(d.RRc, RRc, sizeof(double) * na * 3, hipMemcpyDeviceToDevice, s));
-  launch_set_clock(x.self, t, 0, s);
-  rc = run_forces(&x);
   struct Out {
     void *dst;
     const void *src;
-    size_t bytes;
-  } outs[] = {{Upot, d.Upot, sizeof(double) * P},
-              {dRR, d.dRR, sizeof(double) * P * na * 3},
-              {virt, d.virt, sizeof(double) * P * 9},
-              {virialc, d.virialc, sizeof(double) * P},
-              {dipI, d.dipI, sizeof(double) * P * N * 3},
-              {dipE, d.dipE, sizeof(double) * P * N * 3},
-              {chg, d.chg, sizeof(double) * P * na},
-              {iters, d.iters_out, sizeof(int) * P}};
-  for (const Out &o : outs)
-    if (rc == PIMD_OK && o.dst)
-      HIPCHK(hipMemcpyAsync(o.dst, o.src, o.bytes, hipMemcpyDeviceToDevice, s));
+    size_t bytes;  // of one bead
+  } outs[] = {{Upot, d.Upot, sizeof(double)},
+              {dRR, d.dRR, sizeof(double) * na * 3},
+              {virt, d.virt, sizeof(double) * 9},
+              {virialc, d.virialc, sizeof(double)},
+              {dipI, d.dipI, sizeof(double) * N * 3},
+              {dipE, d.dipE, sizeof(double) * N * 3},
+              {chg, d.chg, sizeof(double) * na},
+              {iters, d.iters_out, sizeof(int)}};
+  // the second half ends at the last bead (an odd count's middle one is in both)
+  for (size_t part = 0; rc == PIMD_OK && part < (n < (size_t)whole ? 2 : 1); ++part) {
+    const size_t b0 = part == 0 ? 0 : (size_t)whole - n;
+    HIPCHK(hipMemcpyAsync(d.RR, RR + b0 * na * 3, sizeof(double) * n * na * 3,
+                          hipMemcpyDeviceToDevice, s));
+    launch_set_clock(x.self, t, 0, s);
+    rc = run_forces(&x);
+    for (const Out &o : outs)
+      if (rc == PIMD_OK && o.dst)
+        HIPCHK(hipMemcpyAsync((char *)o.dst + b0 * o.bytes, o.src, n * o.bytes,
+                              hipMemcpyDeviceToDevice, s));
+  }
   x.d = DevBufs{};  // workspace addresses, not allocations of x
   return rc;
 }

@@ -54,6 +54,8 @@ struct __align__(16) ColRec {
 // Everything the kernels need about the model and the box, passed by value.
 struct SysConst {
   int N, P, model;        // waters, beads, pot_model (2, 3 TTM; 4, 5 fixed-charge SPC)
+  int shapeP;             // beads the launch shapes are chosen for (P, or more where a
+                          // call takes its beads in parts)
   int nd, tdip;           // dipole sites per molecule and the first dipole type
   int nk, ncol, T;        // k-vectors, kz-columns, phase-table rows per site
   int hmax, kmax, lmax;
@@ -147,9 +149,10 @@ struct DevBufs {
   dptr<int4> dcol = nullptr;
   dptr<int> dkx = nullptr;
   dptr<double> Sq = nullptr, Sm = nullptr;  // [P][nk][2]
-  dptr<double> Sv = nullptr;  // [P][nk][6]
   dptr<double> virk = nullptr;  // [P][nkb][9]
-  dptr<double> part = nullptr;  // [P][chunks][nk][2 or 6] structure-factor chunk sums
+  // [P][chunks][nk][2 or 6] structure-factor chunk sums; then, in its first
+  // chunk, the structure factor of the dipole vectors
+  dptr<double> part = nullptr;
   dptr<double> wk = nullptr;  // field operands of the structure factors (recip.hip)
   dptr<int> active = nullptr, iters = nullptr;  // [P]
   dptr<int> nactive = nullptr;  // [1]

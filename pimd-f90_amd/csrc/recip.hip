@@ -150,10 +150,6 @@ __device__ __forceinline__ int row_index(const SysConst &c, int m) {
   return SET == SET_DIP ? m : set_site(c, SET, m);
 }
 
-// LDS row of n staged sites' phases: 4 past a multiple of 8, so that four
-// consecutive sites of neighbouring rows fall on different banks.
-__host__ __device__ inline int phase_row(int n) { return (n + 3) / 8 * 8 + 4; }
-
 // Steps of four (cos, sin) entries along kz = 0..l.
 __host__ __device__ inline int kz_steps(int l) { return (l + 2) / 2; }
 __host__ __device__ inline int col_tiles(const SysConst &c) { return (c.ncol + 15) / 16; }
@@ -166,39 +162,6 @@ __host__ __device__ inline int col_tiles(const SysConst &c) { return (c.ncol + 1
 constexpr int WK_A = 4, WK_B = 6;
 __host__ __device__ inline size_t wk_elems(const SysConst &c, int comps) {
   return (size_t)c.P * col_tiles(c) * kz_steps(c.lmax) * comps * 64;
-}
-
-// Sites of a structure factor's site set.
-__host__ __device__ inline int sfac_sites(const SysConst &c, int mode) {
-  return mode == SF_Q ? 3 * c.N : c.nd * c.N;
-}
-
-// Most sites of a chunk: its phase tables within 150 KB of LDS.
-__host__ __device__ inline int sfac_cap(const SysConst &c) {
-  const int cap = (150 * 1024 / (16 * c.T) - 8) / 8 * 8;
-  return cap < 8 ? 8 : cap;
-}
-
-// Site chunks of a structure factor: nch of sc sites (a multiple of 8, the
-// summed index of two matrix steps), staged in LDS rows of scp.  The charges
-// take half as many sites again as the dipoles: their products are half the
-// work per site.
-__host__ __device__ inline void sfac_chunking(const SysConst &c, int mode, int &nch, int &sc,
-                                              int &scp) {
-  const int M = sfac_sites(c, mode);
-  const int cap = sfac_cap(c), pref = mode == SF_Q ? c.sf_sites + c.sf_sites / 2 : c.sf_sites;
-  const int sites = pref < cap ? pref : cap;
-  const int want = (M + sites - 1) / sites, fit = (M + cap - 1) / cap;
-  // SF_V holds three times the values per chunk: half as many chunks at most
-  int most = mode == SF_V ? c.sf_chunks_max / 2 : c.sf_chunks_max;
-  if (most < fit) most = fit;
-  nch = want < most ? want : most;
-  if (nch < 1) nch = 1;
-  sc = ((M + nch - 1) / nch + 7) / 8 * 8;
-  if (sc < 8) sc = 8;
-  nch = (M + sc - 1) / sc;
-  if (nch < 1) nch = 1;
-  scp = phase_row(sc);
 }
 
 // Chunk partial sums of one structure factor: a wave takes 16 columns and the
@@ -339,8 +302,9 @@ __global__ __launch_bounds__(1024) void k_sfac(const Rep *__restrict__ reps, Blo
 
 // The structure factor from its chunk sums, added in order, and the operands
 // the fields take from it (R: their type, FP32 in the mixed form's SOR
-// iterations).  A thread takes the +-kz pair of one column.  SF_V writes the
-// operands of the total structure factor Sq + Sm.
+// iterations).  A thread takes the +-kz pair of one column.  SF_V stays where
+// its first chunk's sums were, and its operands are those of the total structure
+// factor Sq + Sm.
 template <int MODE, class R>
 __global__ __launch_bounds__(256) void k_sfac_reduce(const Rep *__restrict__ reps, BlockMap bm,
                                                      int stale) {
@@ -370,14 +334,13 @@ __global__ __launch_bounds__(256) void k_sfac_reduce(const Rep *__restrict__ rep
       const int k = k0 + kz - cl.z;
       double v[NV];
       for (int i = 0; i < NV; ++i) v[i] = 0.0;
-      const double *pp = Rp.b.part + ((size_t)b * nch * c.nk + k) * NV;
+      double *pp = Rp.b.part + ((size_t)b * nch * c.nk + k) * NV;
 #pragma unroll 4
       for (int h = 0; h < nch; ++h)
         for (int i = 0; i < NV; ++i) v[i] += pp[(size_t)h * c.nk * NV + i];
-      double *out = (MODE == SF_Q ? Rp.b.Sq : MODE == SF_D ? Rp.b.Sm : Rp.b.Sv) +
-                    ((size_t)b * c.nk + k) * NV;
-      for (int i = 0; i < NV; ++i) out[i] = v[i];
       const size_t o = ((size_t)b * c.nk + k) * 2;
+      double *out = MODE == SF_Q ? Rp.b.Sq + o : MODE == SF_D ? Rp.b.Sm + o : pp;
+      for (int i = 0; i < NV; ++i) out[i] = v[i];
       const double re = MODE == SF_V ? Rp.b.Sq[o] + Rp.b.Sm[o] : v[0];
       const double im = MODE == SF_V ? Rp.b.Sq[o + 1] + Rp.b.Sm[o + 1] : v[1];
       w[s][0] = kv[k].w * re;
@@ -439,16 +402,16 @@ constexpr int FD_WAVES = 8;   // waves per block at most
 // end.  (Waves per block 4 / 8: FD_D of TTM2.1-F 128 x 32 10.8 / 12.9 us, a
 // whole call of 32 H2O x 32 beads 376 / 369 us.)
 __host__ inline void field_groups(const SysConst &c, int M, int &nt, int &sg, int &cg) {
-  long ng = (long)c.P * ((M + FD_SB - 1) / FD_SB);
+  long ng = (long)c.shapeP * ((M + FD_SB - 1) / FD_SB);
   nt = ng <= 128 ? 1 : 2;
   const int sb = 16 * nt;
-  ng = (long)c.P * ((M + sb - 1) / sb);
+  ng = (long)c.shapeP * ((M + sb - 1) / sb);
   const int most = ng <= 256 ? FD_WAVES : 4;
   cg = 1;
   while (cg < most && cg < col_tiles(c) && ng * cg < 2048) cg *= 2;
   if (c.fd_cg) cg = c.fd_cg < FD_WAVES ? c.fd_cg : FD_WAVES;
   auto idle = [&](int s) {
-    const long nb = (long)c.P * ((M + s * sb - 1) / (s * sb));
+    const long nb = (long)c.shapeP * ((M + s * sb - 1) / (s * sb));
     return 1.0 - (double)nb / ((nb + 255) / 256 * 256);
   };
   for (sg = cg < 4 ? 4 / cg : 1; sg > 1; sg /= 2)
@@ -668,7 +631,7 @@ static void launch_sfac_mode(const Group &g, int sel, int part, hipStream_t s) {
     sfac_chunking(c, MODE, nch, sc, scp);
     const int rounds = std::max(1, idiv(c.sf_ntask, 16));
     const int waves = std::max(2, (idiv(c.sf_ntask, rounds) + 1) / 2 * 2);
-    const int groups = (long)nch * c.P <= 128 ? rounds : 1;
+    const int groups = (long)nch * c.shapeP <= 128 ? rounds : 1;
     return Plan{(f32 ? 1 : 0) | (waves << 1) | (groups << 6), nch, c.P, groups,
                 sfac_lds(c, MODE, sc, scp, f32)};
   };

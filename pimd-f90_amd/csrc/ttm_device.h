@@ -780,4 +780,41 @@ __device__ inline void ps_monomer(const SysConst &c, const double r[3][3], doubl
   }
 }
 
+// LDS row of n staged sites' phases: 4 past a multiple of 8, so that four
+// consecutive sites of neighbouring rows fall on different banks.
+__host__ __device__ inline int phase_row(int n) { return (n + 3) / 8 * 8 + 4; }
+
+// Sites of a structure factor's site set.
+__host__ __device__ inline int sfac_sites(const SysConst &c, int mode) {
+  return mode == SF_Q ? 3 * c.N : c.nd * c.N;
+}
+
+// Most sites of a chunk: its phase tables within 150 KB of LDS.
+__host__ __device__ inline int sfac_cap(const SysConst &c) {
+  const int cap = (150 * 1024 / (16 * c.T) - 8) / 8 * 8;
+  return cap < 8 ? 8 : cap;
+}
+
+// Site chunks of a structure factor: nch of sc sites (a multiple of 8, the
+// summed index of two matrix steps), staged in LDS rows of scp.  The charges
+// take half as many sites again as the dipoles: their products are half the
+// work per site.
+__host__ __device__ inline void sfac_chunking(const SysConst &c, int mode, int &nch, int &sc,
+                                              int &scp) {
+  const int M = sfac_sites(c, mode);
+  const int cap = sfac_cap(c), pref = mode == SF_Q ? c.sf_sites + c.sf_sites / 2 : c.sf_sites;
+  const int sites = pref < cap ? pref : cap;
+  const int want = (M + sites - 1) / sites, fit = (M + cap - 1) / cap;
+  // SF_V holds three times the values per chunk: half as many chunks at most
+  int most = mode == SF_V ? c.sf_chunks_max / 2 : c.sf_chunks_max;
+  if (most < fit) most = fit;
+  nch = want < most ? want : most;
+  if (nch < 1) nch = 1;
+  sc = ((M + nch - 1) / nch + 7) / 8 * 8;
+  if (sc < 8) sc = 8;
+  nch = (M + sc - 1) / sc;
+  if (nch < 1) nch = 1;
+  scp = phase_row(sc);
+}
+
 }  // namespace pimd

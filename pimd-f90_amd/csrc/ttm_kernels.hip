@@ -7,7 +7,7 @@
 //                           (M site), 3 for TTM2.1-F (O, H1, H2))
 //   tab   [P][T][4N]      e^{i 2 pi h x/L} per site for h = 0..hmax (x),
 //                         0..kmax (y), 0..lmax (z)
-//   Sq, Sm, Sv [P][nk]    structure factors of charges, dipoles, dipole vectors
+//   Sq, Sm [P][nk]        structure factors of charges, dipoles
 //   tally [P][N][14]      per-molecule partial energies / virials
 //
 // Real-space kernels give each molecule a group of G lanes that walks its full
@@ -1819,7 +1819,7 @@ __global__ __launch_bounds__(256) void k_virk(const Rep *__restrict__ reps, Bloc
   const SysConst &c = Rp.c;
   const double4 *__restrict__ kv = Rp.b.kv;
   const double *__restrict__ Ak = Rp.b.red;
-  const double *__restrict__ Sq = Rp.b.Sq, *__restrict__ Sm = Rp.b.Sm, *__restrict__ Sv = Rp.b.Sv;
+  const double *__restrict__ Sq = Rp.b.Sq, *__restrict__ Sm = Rp.b.Sm;
   double *virk = Rp.b.virk;
   const int b = bk.y;
   const int k = bk.x * 256 + threadIdx.x;
@@ -1841,7 +1841,10 @@ __global__ __launch_bounds__(256) void k_virk(const Rep *__restrict__ reps, Bloc
     for (int col = 0; col < 3; ++col)
       for (int row = 0; row < 3; ++row)
         v[col * 3 + row] = (row == col ? U : 0.0) - U * coeff2 * kx[row] * kx[col];
-    const double *sv = Sv + o * 6;  // sum mu cos (3), sum mu sin (3)
+    int nch, sc, scp;
+    sfac_chunking(c, SF_V, nch, sc, scp);
+    // SF_V, where k_sfac_reduce left it: sum mu cos (3), sum mu sin (3)
+    const double *sv = Rp.b.part + ((size_t)b * nch * c.nk + k) * 6;
     for (int ix = 0; ix < 3 && dip; ++ix) {
       const double t = 2.0 * A * kx[ix];
       for (int iy = 0; iy < 3; ++iy)
@@ -2189,7 +2192,7 @@ constexpr int QQ_HALF_MIN_BLOCKS = 128;
 static bool qq_half_on(const SysConst &c) {
   return c.qq_half && is_ttm(c) && !c.cells && c.g_qq > 0 && qq_half_lds(c) <= PAIR_LDS_MAX &&
          (c.qq_half == 2 ||
-          (long)c.P * qq_half_blocks(c.N, qq_half_lanes(c)) >= QQ_HALF_MIN_BLOCKS);
+          (long)c.shapeP * qq_half_blocks(c.N, qq_half_lanes(c)) >= QQ_HALF_MIN_BLOCKS);
 }
 
 template <int ML, typename R>
@@ -2370,7 +2373,7 @@ static bool fin_half_on(const SysConst &c) {
          c.g_fin > 0 &&
          fin_half_lds(c) <= PAIR_LDS_MAX &&
          (c.qq_half == 2 ||
-          (long)c.P * qq_half_blocks(c.N, half_lanes(c.g_fin)) >= QQ_HALF_MIN_BLOCKS);
+          (long)c.shapeP * qq_half_blocks(c.N, half_lanes(c.g_fin)) >= QQ_HALF_MIN_BLOCKS);
 }
 
 template <int ML, typename R>
