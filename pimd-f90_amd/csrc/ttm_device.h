@@ -303,6 +303,13 @@ __device__ __forceinline__ double rcp_fast(double x) {
   const double e = fma(-x, y, 1.0);
   return fma(y, fma(e, e, e), y);
 }
+// Parameters may be set so that a pair's exponent is far beyond that range: a
+// decay exponent of 1000 stands for any above it (e^-1000 is zero).
+template <typename R>
+__device__ __forceinline__ R decay_exponent(R x) {
+  if constexpr (std::is_same_v<R, double>) return fmin(x, 1000.0);
+  else return x;
+}
 // e^x = 2^n e^r, |r| <= ln 2 / 2; e^r by its interpolation polynomial of
 // degree 11 at the Chebyshev nodes of that interval (relative error 1.7e-17).
 __device__ __forceinline__ double exp_fast(double x) {
@@ -469,7 +476,7 @@ __device__ __forceinline__ void smear01(const SysConst &c, R drsq, R apol, R ra,
   R t0 = s.er * s.dri;
   R t1 = (t0 + (R)c.cts1 * s.expon) * s.drsqi;
   if (THOLE && drsq < (R)25.0) {
-    R rA3 = s.dd * drsq * apol;
+    R rA3 = decay_exponent<R>(s.dd * drsq * apol);
     R exp1 = RM<R>::exp_(-rA3);
     R ch1 = (R)-1.0 * s.dri * s.drsqi;
     R sr1 = ((R)1.0 - exp1) * s.dri * s.drsqi;
@@ -496,7 +503,7 @@ __device__ __forceinline__ void smear2(const SysConst &c, R drsq, R apol, R &ts1
   R t1 = (s.er * s.dri + (R)c.cts1 * s.expon) * s.drsqi;
   R t2 = (t1 + (R)c.cts2 * s.expon) * s.drsqi;
   if (THOLE && drsq < (R)25.0) {
-    R rA3 = (s.dd * drsq) * apol;
+    R rA3 = decay_exponent<R>((s.dd * drsq) * apol);
     R exp1 = RM<R>::exp_(-rA3);
     R ch1 = (R)-1.0 * s.dri * s.drsqi, ch2 = ch1 * s.drsqi;
     R sr1 = ((R)1.0 - exp1) * s.dri * s.drsqi;
@@ -516,7 +523,7 @@ __device__ __forceinline__ void smear3(const SysConst &c, R drsq, R apol, R &ts1
   R t2 = (t1 + (R)c.cts2 * s.expon) * s.drsqi;
   R t3 = (t2 + (R)c.cts3 * s.expon) * s.drsqi;
   if (THOLE && drsq < (R)25.0) {
-    R rA3 = (s.dd * drsq) * apol;
+    R rA3 = decay_exponent<R>((s.dd * drsq) * apol);
     R exp1 = RM<R>::exp_(-rA3);
     R ch1 = (R)-1.0 * s.dri * s.drsqi, ch2 = ch1 * s.drsqi, ch3 = ch2 * s.drsqi;
     R sr1 = ((R)1.0 - exp1) * s.dri * s.drsqi;

@@ -658,7 +658,7 @@ __global__ __launch_bounds__(256) void k_pair_qq(const Rep *__restrict__ reps, B
     const R r2r = (R)r2;
     const R dRij = RM<R>::sqrt_(r2r);
     const R R2i = RM<R>::rcp(r2r), R4i = R2i * R2i, R6i = R2i * R2i * R2i, R8i = R6i * R2i;
-    const R ex = (R)c.vdwD * RM<R>::exp_(-(R)c.vdwE * dRij);
+    const R ex = (R)c.vdwD * RM<R>::exp_(-decay_exponent<R>((R)c.vdwE * dRij));
     const R uij = R6i * (((R)c.vdwA * R6i + (R)c.vdwB * R4i) + (R)c.vdwC) + ex;
     const R xs = dRij - (R)c.rc1;
     const R fsc = -(R8i * (R)6.0 * (R)c.vdwC + RM<R>::div(ex * (R)c.vdwE, dRij) +
@@ -861,7 +861,7 @@ __global__ __launch_bounds__(QQ_HALF_BLOCK) void k_pair_qq_half(const Rep *__res
     const R r2r = (R)r2;
     const R dRij = RM<R>::sqrt_(r2r);
     const R R2i = RM<R>::rcp(r2r), R4i = R2i * R2i, R6i = R2i * R2i * R2i, R8i = R6i * R2i;
-    const R ex = (R)c.vdwD * RM<R>::exp_(-(R)c.vdwE * dRij);
+    const R ex = (R)c.vdwD * RM<R>::exp_(-decay_exponent<R>((R)c.vdwE * dRij));
     const R uij = R6i * (((R)c.vdwA * R6i + (R)c.vdwB * R4i) + (R)c.vdwC) + ex;
     const R xs = dRij - (R)c.rc1;
     const R fsc = -(R8i * (R)6.0 * (R)c.vdwC + RM<R>::div(ex * (R)c.vdwE, dRij) +

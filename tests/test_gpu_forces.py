@@ -294,3 +294,27 @@ def test_overlapping_molecules_saturate(monkeypatch, precision, end):
     k = int(np.argmin(np.abs(one)))
     assert abs(one[1 - k] - two[1 - k]) < 1e-5 * abs(two[1 - k])
     assert abs(abs(one[k]) - end) < 1e6 + 1e-6 * end
+
+
+@pytest.mark.parametrize("index,large,huge", [(4, 1e3, 1e60), (9, 1e-9, 1e-160)])
+def test_pair_terms_of_any_decay(index, large, huge):
+    """Parameters far out: a vdW exponent E and a polfacH (the Thole factors go
+    with 1 / polfac) so large and so small that e^(-E r) and e^(-a r^3) are
+    zero already, and then by 57 and 151 orders more: the same energies and
+    forces, finite."""
+    from pimd_amd.params import TTMParams
+    from pimd_amd.systems import make_system
+    RRt, _, RRc, L = make_system(32, 2, seed=5)
+    p = TTMParams(pot_model=3, nwaters=32, nbeads=2, box=(L, L, L), eps_ewald=1e-6).resolved()
+    print("case", index, large, huge, flush=True)
+    r = []
+    for v in (large, huge):
+        ff = _ff(p)
+        th = ff.ttm_params()
+        th[index] = v
+        ff.set_ttm_params(th)
+        r.append(ff.full_bead_forces(RRt, RRc))
+        ff.close()
+    assert np.all(np.isfinite(r[1]["dRRt"]))
+    assert rel_err(r[1]["Upott"], r[0]["Upott"]) < 1e-14
+    assert max_abs(r[1]["dRRt"], r[0]["dRRt"]) < 1e-10
