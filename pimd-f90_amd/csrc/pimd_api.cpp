@@ -364,8 +364,8 @@ int setup_system(pimd_ctx *x) {
   c.nk = (int)x->Ak.size();
   if (c.nk == 0) return fail(PIMD_EINVAL, "no k-vectors inside the Ewald cut-off");
   c.T = (c.hmax + 1) + (c.kmax + 1) + (c.lmax + 1);
-  // the reciprocal-space kernels stage T table rows of up to 64 sites in LDS
-  // (T KiB of it, within the 160 KiB of a workgroup)
+  // 128 rows let the structure factors stage chunks of 64 sites in LDS (sfac_cap;
+  // sf_chunks_max counts on that many) and the fields two 16-site tiles (73 KB)
   if (c.T > 128)
     return fail(PIMD_EINVAL, "%d Ewald table rows (hmax+kmax+lmax+3) exceed the limit of 128; "
                 "raise eps_ewald or the cut-off", c.T);
@@ -551,7 +551,6 @@ void plan_system(pimd_ctx *x, HostTables &t) {
   c.g_qq = env_int("PIMD_G_QQ", dflt_qq, 0, 32);
   c.g_fin = env_int("PIMD_G_FIN", dflt_qq, 0, 32);
   c.poll = env_int("PIMD_SOR_POLL", 0, 0, 1);
-  c.overlap = 0;
   // the charge pair pass evaluates each molecule pair once (not with the
   // cell-list neighbour search, whose lists are not in partner order):
   // 0 never, 1 where its blocks fill the device, 2 always
@@ -619,7 +618,7 @@ void layout_system(pimd_ctx *x, Arena &a, bool full) {
   a.take(&d.Sq, P * nk * 2);
   a.take(&d.Sm, P * nk * 2);
   a.take(&d.virk, P * ((nk + 255) / 256) * 18);
-  a.take(&d.part, full ? P * (size_t)c.sf_chunks_max * nk * 6 : sfac_part_elems(c));
+  a.take(&d.part, sfac_part_elems(c, full));
   a.take(&d.wk, field_operand_elems(c));
   a.take(&d.active, P);
   a.take(&d.iters, P);
@@ -2571,7 +2570,6 @@ extern "C" int pimd_forces_all_beads_noalloc(const pimd_params *params, const do
   // memory; the dipole pass recomputes its pair screening factors every SOR
   // iteration (the same values as the cache would hold)
   x.c.poll = 0;
-  x.c.overlap = 0;
   x.c.dd_cache = 0;
   // All beads at once or, where they need up to 7/4 of the workspace, one half
   // after the other with the launch shapes of all (a bead's results do not

@@ -73,7 +73,6 @@ struct SysConst {
   int g_qq, g_fin;         // the same for the charge and final pair kernels
   int g_nolds;             // lanes per molecule of the pair kernels that do not stage in LDS
   int poll;                // 1: read the active-bead count back after every SOR iteration
-  int overlap;             // 1: real-space dipole field beside the structure factor (2 streams)
   int dd_cache;            // 1: the SOR dipole pass keeps each pair's screening factors
   int dense;               // SOR by a dense dipole matrix: 0 no, 1 one block per bead, 2 by launches
   int qq_half;             // once-per-pair charge pass: 0 off, 1 where it fills the device, 2 always
@@ -347,7 +346,7 @@ inline size_t dense_elems(const SysConst &c) {
   return (size_t)c.P * 3 * c.nd * c.N * dense_stride(c);
 }
 int sfac_chunks_max(const SysConst &c);
-size_t sfac_part_elems(const SysConst &c);
+size_t sfac_part_elems(const SysConst &c, bool any_sites);
 size_t field_operand_elems(const SysConst &c);
 std::vector<ColRec> column_records(const SysConst &c, const std::vector<int4> &cols);
 std::vector<int> sfac_tasks(const std::vector<int4> &cols);

@@ -393,9 +393,10 @@ static size_t sfac_lds(const SysConst &c, int mode, int sc, int scp, bool f32) {
 constexpr int FD_SB = 32;     // sites per group of two tiles
 constexpr int FD_WAVES = 8;   // waves per block at most
 // Tiles per site group, site groups per block and column groups of one field
-// launch over M sites.  Small systems take one tile to a group, half the work
-// per wave (with the structure factors' rounds in blocks of their own, one
-// bead of 32 H2O 267 -> 250 us per call, 32 beads 373 -> 359).
+// launch over M sites.  Small systems, of up to 128 groups of two tiles, take
+// one tile to a group, half the work per wave: one tile / two, us per call of
+// 32 H2O (Rc 4.9 A), 1 bead 250 / 258, 8 beads (24 groups of charges) 275 / 285,
+// 32 (96) 355 / 364, 48 (144) 374 / 373, 64 (192) 407 / 408.
 // Column groups until the device has two waves per SIMD; blocks of 4 waves,
 // of which a CU holds three, and of 8 only where every CU gets at most one
 // block.  Of 4, 2 and 1 site groups the most that leave few CUs idle at the
@@ -616,9 +617,10 @@ static int idiv(long a, long b) { return (int)((a + b - 1) / b); }
 // SFAC_STALE the dense systems' last input.  part: 1 the chunk sums, 2 their
 // reduction, 3 both.  Variant: bit 0 FP32, above it the waves per block: one
 // per task up to 16, beyond as few rounds of tasks as 16 waves need; an even
-// number, so that more replicas of a batch share launches.  Small systems give
-// each round a block of its own (with one-tile site groups: one bead of 32
-// H2O 267 -> 250 us per call, 32 beads 373 -> 359).
+// number, so that more replicas of a batch share launches.  Passes of up to 128
+// chunks give each round a block of its own: so / one block for all rounds, us
+// per call of 32 H2O (Rc 4.9 A), 1 bead (4 to 8 chunks) 245 / 250, 8 beads (32
+// and 64) 268 / 275, 32 (128 dipole chunks) 350 / 355, 48 (192) 378 / 374.
 template <int MODE>
 static void launch_sfac_mode(const Group &g, int sel, int part, hipStream_t s) {
   const int stale = MODE == SF_D && sel == SFAC_STALE ? 1 : 0;
@@ -704,8 +706,11 @@ static void launch_field_mode(const Group &g, int iter, bool sel_mixed, hipStrea
       });
 }
 
-// Buffer elements: the chunk sums and the field operands.
-size_t sfac_part_elems(const SysConst &c) {
+// Buffer elements: the chunk sums (any_sites: enough for every sf_sites, which
+// the batch tuning changes) and the field operands.
+size_t sfac_part_elems(const SysConst &c0, bool any_sites) {
+  SysConst c = c0;
+  if (any_sites) c.sf_sites = 1;  // as many chunks as there may be
   size_t most = 0;
   for (int mode : {SF_Q, SF_D, SF_V}) {
     int nch, sc, scp;
