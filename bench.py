@@ -68,8 +68,8 @@ def flop_model(kernel, c):
     """Algorithmic FP64/FP32 operations per launch: what the algorithm needs,
     not what the kernel issues.  A fused multiply-add counts two, a
     transcendental, square root or division one.  Pair terms are counted once
-    per unordered molecule pair within the cutoff (the kernels evaluate each
-    pair from both molecules, which is not credited); reciprocal-space terms
+    per unordered molecule pair within the cutoff (passes that evaluate a pair
+    from both molecules get no credit for it); reciprocal-space terms
     once per (site, k) with one complex product to advance the phase along
     the kz column:
       structure factors  q:  phase 6 + accumulate 4                     = 10
@@ -104,9 +104,9 @@ def flop_model(kernel, c):
 
 
 def measured_valu(form, key):
-    """Issued VALU floating-point operations per launch of a kernel from the
-    committed rocprofv3 SQ_INSTS_VALU_* summary (64 lanes per instruction,
-    an FMA two), or None."""
+    """Issued floating-point operations per launch of a kernel from the
+    committed rocprofv3 SQ_INSTS_VALU_* summary (vector, 64 lanes per
+    instruction and an FMA two, and matrix), or None."""
     path = os.path.join(ROOT, "profiles", "valu_counters_h2o512_p32_ttm3f.md")
     if not os.path.exists(path):
         return None
