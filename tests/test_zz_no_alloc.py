@@ -112,11 +112,13 @@ def test_noalloc_mixed_and_fixed_charge():
     _case(4, 32, 2, -1.0, 1e-6, 0, 74, stream=False)
 
 
-@pytest.mark.parametrize("model,N,P,eps", [(3, 128, 64, 1e-6), (2, 16, 48, 1e-10), (2, 16, 47, 1e-10)])
+@pytest.mark.parametrize("model,N,P,eps", [(3, 128, 64, 1e-6), (3, 512, 32, 1e-6), (2, 16, 48, 1e-10),
+                                            (2, 16, 47, 1e-10)])
 def test_noalloc_in_two_halves(model, N, P, eps):
     """Systems whose arrays exceed the workspace together: the dense dipole
-    matrices of 128 waters x 64 beads, the k-vectors of few waters at a tight
-    Ewald tolerance; an odd bead count, whose middle bead both halves take."""
+    matrices of 128 waters x 64 beads, all arrays of 512 x 32, the k-vectors of
+    few waters at a tight Ewald tolerance; an odd bead count, whose middle bead
+    both halves take."""
     _case(model, N, P, -1.0, eps, 0, 75, stream=True)
 
 
